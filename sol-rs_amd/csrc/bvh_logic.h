@@ -239,7 +239,36 @@ SOLHIP_HD uint32_t pow2_ceil_exp(float x)
     return e < 254u ? e : 254u;
 }
 
-// Build wide node w from its binary source node.  `alloc(counter, amount)`
+// quantisation frame of a node box: scale 2^e >= extent / 253 (with a floor of
+// 2^-8 of the largest extent so that flat boxes keep a padding step that is
+// large against fp32 error in the slab distances), origin one step below
+SOLHIP_HD void node_frame(float4 lo, float4 hi, uint32_t eb[3], float sc[3], float org[3])
+{
+    const float ext[3] = {hi.x - lo.x, hi.y - lo.y, hi.z - lo.z};
+    const float los[3] = {lo.x, lo.y, lo.z};
+    const float maxext = fmaxf(fmaxf(ext[0], ext[1]), ext[2]);
+    for (int a = 0; a < 3; ++a) {
+        eb[a] = pow2_ceil_exp(fmaxf(ext[a], maxext * 0x1p-8f) / 253.0f);
+        sc[a] = as_f(eb[a] << 23);
+        org[a] = los[a] - sc[a];
+    }
+}
+
+// a child's range [lo, hi] on one axis in that frame: rounded outward and
+// padded by one step
+SOLHIP_HD void quantise_range(float lo, float hi, float org, float sc, int &ql, int &qh)
+{
+    const double o = (double)org, s = (double)sc;
+    const float fl = floorf((lo - org) / sc) - 1.0f;
+    const float fh = ceilf((hi - org) / sc) + 1.0f;
+    ql = fl <= 0.0f ? 0 : (fl >= 255.0f ? 255 : (int)fl);
+    qh = fh <= 0.0f ? 0 : (fh >= 255.0f ? 255 : (int)fh);
+    while (ql > 0 && o + ql * s > (double)lo) --ql;
+    while (qh < 255 && o + qh * s < (double)hi) ++qh;
+}
+
+// Build wide node w from its binary source node (the library's k_collapse does
+// the same with 8 lanes per node).  `alloc(counter, amount)`
 // returns the previous value of counters[counter] after adding amount.
 // Returns the number of range violations (0 on a consistent tree).
 template <class Alloc>
@@ -335,20 +364,10 @@ SOLHIP_HD uint32_t collapse_node(const CollapseArgs &A, uint32_t w, Alloc alloc)
     const uint32_t child_base = nint ? alloc(0, nint) : 0u;
     const uint32_t prim_base = nprim ? alloc(1, nprim) : 0u;
     if ((uint64_t)child_base + nint > A.node_cap || (uint64_t)prim_base + nprim > (uint64_t)n) return 1;
-    // quantisation frame: scale 2^e >= extent / 253 (with a floor of 2^-8 of
-    // the largest extent so that flat boxes keep a padding step that is
-    // large against fp32 error in the slab distances), origin one step below
     WideNode nd;
-    const float ext[3] = {hi.x - lo.x, hi.y - lo.y, hi.z - lo.z};
-    const float los[3] = {lo.x, lo.y, lo.z};
-    const float maxext = fmaxf(fmaxf(ext[0], ext[1]), ext[2]);
     uint32_t eb[3];
     float sc[3], org[3];
-    for (int a = 0; a < 3; ++a) {
-        eb[a] = pow2_ceil_exp(fmaxf(ext[a], maxext * 0x1p-8f) / 253.0f);
-        sc[a] = as_f(eb[a] << 23);
-        org[a] = los[a] - sc[a];
-    }
+    node_frame(lo, hi, eb, sc, org);
     nd.px = org[0];
     nd.py = org[1];
     nd.pz = org[2];
@@ -375,13 +394,8 @@ SOLHIP_HD uint32_t collapse_node(const CollapseArgs &A, uint32_t w, Alloc alloc)
         const float4 l = A.nbox[2ull * bn], h = A.nbox[2ull * bn + 1];
         const float cl[3] = {l.x, l.y, l.z}, chh[3] = {h.x, h.y, h.z};
         for (int a = 0; a < 3; ++a) {
-            const double o = (double)org[a], s_ = (double)sc[a];
-            float fl = floorf((cl[a] - org[a]) / sc[a]) - 1.0f;
-            float fh = ceilf((chh[a] - org[a]) / sc[a]) + 1.0f;
-            int ql = fl <= 0.0f ? 0 : (fl >= 255.0f ? 255 : (int)fl);
-            int qh = fh <= 0.0f ? 0 : (fh >= 255.0f ? 255 : (int)fh);
-            while (ql > 0 && o + ql * s_ > (double)cl[a]) --ql;
-            while (qh < 255 && o + qh * s_ < (double)chh[a]) ++qh;
+            int ql, qh;
+            quantise_range(cl[a], chh[a], org[a], sc[a], ql, qh);
             qlo[a][s] = (uint8_t)ql;
             qhi[a][s] = (uint8_t)qh;
         }
