@@ -32,13 +32,16 @@ struct BlasRef {
 
 static_assert(sizeof(BlasRef) == 32, "BlasRef layout");
 
+constexpr uint32_t kPinnedWords = 256;
+
 // build scratch, kept by each BLAS / TLAS so that rebuilds allocate nothing
 struct DevScratch {
     DevBuf boxes, bounds, keys[2], vals[2], hist, left, right, parent, rfirst, flags, nbox, ncount, counters,
         wsrc, leaf_ids, frontier;
+    DevBuf sah_work;               // binned SAH builds (bvh_sah.hip)
     std::vector<DevBuf> scan_bufs;
-    uint32_t *pinned = nullptr;
-    int ensure(uint32_t n);
+    uint32_t *pinned = nullptr;    // kPinnedWords words
+    int ensure(uint32_t n, bool sah);
     uint32_t *scan_level(int level, uint32_t count);
     void release();
 };
@@ -58,6 +61,14 @@ struct DeviceBvh {
         root_box.release();
     }
 };
+
+// binary tree of a binned-SAH build (bvh_sah.hip) over the boxes in sc.boxes
+// (2 float4 per primitive, its index in the first one's w) with centroid
+// bounds in sc.bounds, n > 1: fills sc.left / right / rfirst / ncount / nbox
+// and the root's index in sc.wsrc[0]; vals_out: primitive of each leaf
+// position.  Range errors are counted in sc.counters[3].
+int build_binary_sah(hipStream_t s, uint32_t n, DevScratch &sc, const uint32_t *&vals_out);
+uint64_t sah_work_bytes(uint32_t n);
 
 // flags: SOLHIP_BUILD_* (SOLHIP_BUILD_PREFER_FAST_TRACE: binned SAH, else Morton order).
 // geo_dev: the n_geo descriptors (and, after them, the u32 table

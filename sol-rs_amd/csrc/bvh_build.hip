@@ -102,7 +102,7 @@ __global__ void __launch_bounds__(kBlock) k_tri_boxes(const GeomDesc *geo, uint3
                 hi[a] = fmaxf(hi[a], p[a]);
             }
         }
-        boxes[2ull * i] = make_float4(lo[0], lo[1], lo[2], 0.0f);
+        boxes[2ull * i] = make_float4(lo[0], lo[1], lo[2], __uint_as_float(i));   // its index travels with it (SAH)
         boxes[2ull * i + 1] = make_float4(hi[0], hi[1], hi[2], 0.0f);
         for (int a = 0; a < 3; ++a) c[a] = 0.5f * lo[a] + 0.5f * hi[a];
     }
@@ -370,292 +370,6 @@ __global__ void __launch_bounds__(kBlock) k_refit_cross(int n, const uint32_t *l
             node = par;
         }
     }
-}
-
-// ---- binned SAH binary tree (fast-trace BLAS builds) ---------------------
-// Top down, one launch per tree level, one workgroup per node of the level
-// (a task: first position of the node's range in the primitive order, the
-// binary node).  The workgroup finds the node's centroid range and box, bins
-// its primitives (sah_choose), and partitions the range stably into the
-// other order buffer.  A side with one primitive is a leaf, placed at its
-// final position (leaf node n-1+position); a larger side gets the next
-// internal node index and becomes a task of the next level.  Node indices
-// follow the order in which workgroups finish, but the tree's shape does not
-// depend on it: it equals the host replay's.  Nodes of at least big_min
-// primitives go to a second task list, run by 1024-thread workgroups (the
-// top levels, where a few workgroups work through millions of primitives).
-constexpr uint32_t kSahBigMin = 65536;
-
-struct SahArgs {
-    const float4 *boxes;   // 2 per primitive
-    const uint32_t *ids_in;
-    uint32_t *ids_out;
-    uint32_t *vals;        // primitive of each leaf position
-    const uint2 *tasks_in;     // this launch's tasks (small or big list)
-    uint2 *tasks_out;          // next level, nodes of fewer than big_min primitives
-    uint2 *big_out;            // next level, nodes of big_min or more
-    uint32_t *ntasks_out, *nbig_out;
-    uint32_t *node_alloc;
-    uint32_t *left, *right, *rfirst, *ncount;
-    float4 *nbox;
-    uint32_t n, task_cap, big_cap, big_min, level;
-    uint32_t *err;
-};
-
-struct SahLdsBins {
-    const uint32_t (*cnt)[kSahBins];
-    const uint32_t (*lo_)[kSahBins][3];
-    const uint32_t (*hi_)[kSahBins][3];
-    __device__ uint32_t count(int a, int b) const { return cnt[a][b]; }
-    __device__ float lo(int a, int b, int k) const { return ord2f(lo_[a][b][k]); }
-    __device__ float hi(int a, int b, int k) const { return ord2f(hi_[a][b][k]); }
-};
-
-__device__ __forceinline__ void prim_centroid(const float4 *boxes, uint32_t p, float4 &l, float4 &h, float c[3])
-{
-    l = boxes[2ull * p];
-    h = boxes[2ull * p + 1];
-    c[0] = 0.5f * l.x + 0.5f * h.x;
-    c[1] = 0.5f * l.y + 0.5f * h.y;
-    c[2] = 0.5f * l.z + 0.5f * h.z;
-}
-
-template <int BLOCK>
-__global__ void __launch_bounds__(BLOCK) k_sah_level(SahArgs A)
-{
-    __shared__ uint32_t s_cnt[3][kSahBins];
-    __shared__ uint32_t s_lo[3][kSahBins][3], s_hi[3][kSahBins][3];
-    __shared__ uint32_t s_red[BLOCK / 64][12];
-    __shared__ uint32_t s_bounds[12];
-    __shared__ SahSplit s_axis_best[3];
-    __shared__ float s_axis_cost[3];
-    __shared__ int s_split[3];
-    __shared__ uint32_t s_wave[BLOCK / 64];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint2 t = A.tasks_in[blockIdx.x];
-    const uint32_t lo = t.x, node = t.y, n = A.n;
-    // block-uniform checks: every thread of the block takes the same branch
-    if (node >= n - 1u) {
-        if (tid == 0) atomicAdd(A.err, 1u);
-        return;
-    }
-    const uint32_t cnt = A.ncount[node];
-    if (cnt < 2u || cnt > n || lo > n - cnt) {
-        if (tid == 0) atomicAdd(A.err, 1u);
-        return;
-    }
-    const uint32_t hi = lo + cnt;
-    // pass 1: centroid range and node box (ordered-integer min / max)
-    uint32_t r[12];
-    for (int k = 0; k < 3; ++k) {
-        r[k] = 0xFFFFFFFFu;      // centroid min
-        r[3 + k] = 0u;           // centroid max
-        r[6 + k] = 0xFFFFFFFFu;  // box min
-        r[9 + k] = 0u;           // box max
-    }
-    for (uint32_t i = lo + tid; i < hi; i += BLOCK) {
-        const uint32_t p = min(A.ids_in[i], n - 1u);
-        float4 l, h;
-        float c[3];
-        prim_centroid(A.boxes, p, l, h, c);
-        const float lv[3] = {l.x, l.y, l.z}, hv[3] = {h.x, h.y, h.z};
-        for (int k = 0; k < 3; ++k) {
-            r[k] = min(r[k], f2ord(c[k]));
-            r[3 + k] = max(r[3 + k], f2ord(c[k]));
-            r[6 + k] = min(r[6 + k], f2ord(lv[k]));
-            r[9 + k] = max(r[9 + k], f2ord(hv[k]));
-        }
-    }
-    for (int k = 0; k < 12; ++k) {
-        const bool is_min = (k % 6) < 3;
-        for (int off = 32; off > 0; off >>= 1) {
-            const uint32_t o = (uint32_t)__shfl_xor((int)r[k], off);
-            r[k] = is_min ? min(r[k], o) : max(r[k], o);
-        }
-    }
-    if (lane == 0)
-        for (int k = 0; k < 12; ++k) s_red[wave][k] = r[k];
-    // bins start empty
-    for (uint32_t j = tid; j < 3u * kSahBins; j += BLOCK) {
-        (&s_cnt[0][0])[j] = 0u;
-        for (int k = 0; k < 3; ++k) {
-            (&s_lo[0][0][0])[3 * j + k] = f2ord(INFINITY);
-            (&s_hi[0][0][0])[3 * j + k] = f2ord(-INFINITY);
-        }
-    }
-    __syncthreads();
-    if (tid < 12) {
-        const bool is_min = (tid % 6) < 3;
-        uint32_t v = s_red[0][tid];
-        for (int w = 1; w < BLOCK / 64; ++w) v = is_min ? min(v, s_red[w][tid]) : max(v, s_red[w][tid]);
-        s_bounds[tid] = v;
-    }
-    __syncthreads();
-    float cmin[3], scale[3];
-    for (int k = 0; k < 3; ++k) {
-        cmin[k] = ord2f(s_bounds[k]);
-        scale[k] = sah_scale(ord2f(s_bounds[3 + k]) - cmin[k]);
-    }
-    if (tid == 0) {
-        A.nbox[2ull * node] = make_float4(ord2f(s_bounds[6]), ord2f(s_bounds[7]), ord2f(s_bounds[8]), 0.0f);
-        A.nbox[2ull * node + 1] = make_float4(ord2f(s_bounds[9]), ord2f(s_bounds[10]), ord2f(s_bounds[11]), 0.0f);
-    }
-    // pass 2: bins.  Neighbouring primitives mostly share a bin, so a wave
-    // whose valid lanes all fall in one bin reduces them with shuffles and
-    // makes one update; otherwise each lane updates its bin.
-    for (uint32_t base = lo; base < hi; base += BLOCK) {
-        const uint32_t i = base + tid;
-        const bool valid = i < hi;
-        float4 l = make_float4(INFINITY, INFINITY, INFINITY, 0.0f), h = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
-        float c[3] = {0.0f, 0.0f, 0.0f};
-        if (valid) prim_centroid(A.boxes, min(A.ids_in[i], n - 1u), l, h, c);
-        const uint64_t vmask = __ballot(valid);
-        if (vmask == 0) continue;   // wave-uniform
-        const float lv[3] = {l.x, l.y, l.z}, hv[3] = {h.x, h.y, h.z};
-        for (int a = 0; a < 3; ++a) {
-            if (!(scale[a] > 0.0f)) continue;   // block-uniform
-            const int b = sah_bin(c[a], cmin[a], scale[a]);
-            const int b0 = __shfl(b, 0);         // lane 0 is valid when any lane is
-            if (__ballot(valid && b != b0) == 0) {
-                uint32_t v[6];
-                for (int k = 0; k < 3; ++k) {
-                    v[k] = f2ord(lv[k]);
-                    v[3 + k] = f2ord(hv[k]);
-                }
-                for (int off = 32; off > 0; off >>= 1)
-                    for (int k = 0; k < 6; ++k) {
-                        const uint32_t o = (uint32_t)__shfl_xor((int)v[k], off);
-                        v[k] = k < 3 ? min(v[k], o) : max(v[k], o);
-                    }
-                if (lane == 0) {
-                    atomicAdd(&s_cnt[a][b0], (uint32_t)__popcll(vmask));
-                    for (int k = 0; k < 3; ++k) {
-                        atomicMin(&s_lo[a][b0][k], v[k]);
-                        atomicMax(&s_hi[a][b0][k], v[3 + k]);
-                    }
-                }
-            } else if (valid) {
-                atomicAdd(&s_cnt[a][b], 1u);
-                for (int k = 0; k < 3; ++k) {
-                    atomicMin(&s_lo[a][b][k], f2ord(lv[k]));
-                    atomicMax(&s_hi[a][b][k], f2ord(hv[k]));
-                }
-            }
-        }
-    }
-    __syncthreads();
-    // split: one thread per axis, then the first strict minimum in axis order
-    // (sah_choose's result)
-    if (tid < 3) {
-        SahSplit sp{-1, 0, cnt / 2};
-        float cost = INFINITY;
-        if (A.level < kSahMedianLevel && scale[tid] > 0.0f) sah_axis(SahLdsBins{s_cnt, s_lo, s_hi}, (int)tid, cost, sp);
-        s_axis_best[tid] = sp;
-        s_axis_cost[tid] = cost;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        SahSplit sp{-1, 0, cnt / 2};
-        float cost = INFINITY;
-        for (int a = 0; a < 3; ++a)
-            if (s_axis_cost[a] < cost) {
-                cost = s_axis_cost[a];
-                sp = s_axis_best[a];
-            }
-        s_split[0] = sp.axis;
-        s_split[1] = sp.bin;
-        s_split[2] = (int)sp.nleft;
-    }
-    __syncthreads();
-    const int axis = s_split[0], sbin = s_split[1];
-    const uint32_t nleft = (uint32_t)s_split[2], nright = cnt - nleft;
-    // pass 3: stable partition into ids_out, chunk by chunk
-    uint32_t lbase = 0, rbase = 0;
-    for (uint32_t base = lo; base < hi; base += BLOCK) {
-        const uint32_t i = base + tid;
-        const bool valid = i < hi;
-        uint32_t p = 0;
-        bool left_side = false;
-        float4 l, h;
-        if (valid) {
-            p = min(A.ids_in[i], n - 1u);
-            float c[3];
-            prim_centroid(A.boxes, p, l, h, c);
-            left_side = axis >= 0 ? sah_bin(c[axis], cmin[axis], scale[axis]) <= sbin : (i - lo) < nleft;
-        }
-        const uint64_t m = __ballot(left_side);
-        if (lane == 0) s_wave[wave] = (uint32_t)__popcll(m);
-        __syncthreads();
-        uint32_t woff = 0, total = 0;
-        for (uint32_t w = 0; w < BLOCK / 64; ++w) {
-            woff += w < wave ? s_wave[w] : 0u;
-            total += s_wave[w];
-        }
-        const uint32_t lrank = woff + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-        if (valid) {
-            const uint32_t rrank = (i - base) - lrank;
-            const uint32_t pos = left_side ? lo + lbase + lrank : lo + nleft + rbase + rrank;
-            if (pos < hi && (left_side ? lbase + lrank < nleft : rbase + rrank < nright)) {
-                A.ids_out[pos] = p;
-                if ((left_side ? nleft : nright) == 1u) {
-                    // a one-primitive side: leaf n-1+pos at its final position
-                    A.vals[pos] = p;
-                    A.nbox[2ull * (n - 1u + pos)] = l;
-                    A.nbox[2ull * (n - 1u + pos) + 1] = h;
-                    A.ncount[n - 1u + pos] = 1u;
-                }
-            } else {
-                atomicAdd(A.err, 1u);
-            }
-        }
-        lbase += total;
-        rbase += min((uint32_t)BLOCK, hi - base) - total;
-        __syncthreads();   // s_wave is rewritten by the next chunk
-    }
-    if (tid == 0) {
-        if (lbase != nleft || nleft == 0u || nleft >= cnt) atomicAdd(A.err, 1u);
-        for (int side = 0; side < 2; ++side) {
-            const uint32_t start = side ? lo + nleft : lo, m = side ? nright : nleft;
-            uint32_t child;
-            if (m == 1u) {
-                child = n - 1u + start;
-            } else {
-                child = atomicAdd(A.node_alloc, 1u);
-                const bool big = m >= A.big_min;
-                const uint32_t slot = atomicAdd(big ? A.nbig_out : A.ntasks_out, 1u);
-                if (child >= n - 1u || slot >= (big ? A.big_cap : A.task_cap) || m == 0u) {
-                    atomicAdd(A.err, 1u);
-                    child = 0u;
-                } else {
-                    A.rfirst[child] = start;
-                    A.ncount[child] = m;
-                    (big ? A.big_out : A.tasks_out)[slot] = make_uint2(start, child);
-                }
-            }
-            if (side) A.right[node] = child;
-            else A.left[node] = child;
-        }
-    }
-}
-
-// the root task, in the big list (big) or the small one
-__global__ void k_sah_init(uint32_t n, bool big, uint2 *small0, uint2 *big0, uint32_t *ncount, uint32_t *rfirst,
-                           uint32_t *counters)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        (big ? big0 : small0)[0] = make_uint2(0u, 0u);
-        ncount[0] = n;
-        rfirst[0] = 0u;
-        counters[6] = 0u;   // small tasks of the next level
-        counters[7] = 1u;   // internal nodes allocated (the root)
-        counters[8] = 0u;   // big tasks of the next level
-    }
-}
-
-__global__ void __launch_bounds__(kBlock) k_iota(uint32_t *v, uint32_t n)
-{
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < n) v[i] = i;
 }
 
 // ---- collapse to 8-wide quantised nodes ---------------------------------
@@ -959,11 +673,6 @@ __global__ void __launch_bounds__(kBlock) k_validate(const WideNode *wn, uint32_
     }
 }
 
-__global__ void k_fill_u32(uint32_t *p, uint32_t n, uint32_t v)
-{
-    if (threadIdx.x < n) p[threadIdx.x] = v;
-}
-
 // the state a build starts from: counters ([0] wide nodes allocated: the
 // root), level ranges (level 0 is the root), centroid bounds, the root's
 // binary node
@@ -1031,86 +740,6 @@ void DevBuf::release()
 
 static int build_binary_lbvh(hipStream_t s, uint32_t n, DevScratch &sc, const uint32_t *&vals_out);
 
-// Binary tree by binned SAH (k_sah_level), one or two launches (small and big
-// nodes) and one read-back of the next level's task counts per level.  Order
-// buffers: vals[0] / vals[1]; leaf order: keys[0]; small tasks: flags /
-// frontier (at most n / 2 per level); big tasks: the two halves of hist.
-static int build_binary_sah(hipStream_t s, uint32_t n, DevScratch &sc, const uint32_t *&vals_out)
-{
-    uint32_t *counters = (uint32_t *)sc.counters.ptr;
-    uint32_t *pinned = sc.pinned;
-    uint32_t *ids[2] = {(uint32_t *)sc.vals[0].ptr, (uint32_t *)sc.vals[1].ptr};
-    uint32_t *vals = (uint32_t *)sc.keys[0].ptr;
-    uint2 *tasks[2] = {(uint2 *)sc.flags.ptr, (uint2 *)sc.frontier.ptr};
-    const uint32_t big_cap = (uint32_t)std::min<uint64_t>(n / kSahBigMin + 1, sc.hist.bytes / 16);
-    uint2 *bigs[2] = {(uint2 *)sc.hist.ptr, (uint2 *)sc.hist.ptr + big_cap};
-    uint32_t *ncount = (uint32_t *)sc.ncount.ptr, *rfirst = (uint32_t *)sc.rfirst.ptr;
-    const uint32_t cap = n / 2;
-    if (big_cap < 1) {
-        set_error("SAH BVH build: no room for the task lists");
-        return SOLHIP_ERROR_DEVICE;
-    }
-    const bool root_big = n >= kSahBigMin;
-    hipLaunchKernelGGL(k_iota, dim3(cdiv(n, kBlock)), dim3(kBlock), 0, s, ids[0], n);
-    hipLaunchKernelGGL(k_sah_init, dim3(1), dim3(64), 0, s, n, root_big, tasks[0], bigs[0], ncount, rfirst, counters);
-    uint32_t nsmall = root_big ? 0u : 1u, nbig = root_big ? 1u : 0u, level = 0;
-    int cur = 0;
-    while (nsmall || nbig) {
-        SahArgs a;
-        a.boxes = (const float4 *)sc.boxes.ptr;
-        a.ids_in = ids[cur];
-        a.ids_out = ids[cur ^ 1];
-        a.vals = vals;
-        a.tasks_out = tasks[cur ^ 1];
-        a.big_out = bigs[cur ^ 1];
-        a.ntasks_out = counters + 6;
-        a.nbig_out = counters + 8;
-        a.node_alloc = counters + 7;
-        a.left = (uint32_t *)sc.left.ptr;
-        a.right = (uint32_t *)sc.right.ptr;
-        a.rfirst = rfirst;
-        a.ncount = ncount;
-        a.nbox = (float4 *)sc.nbox.ptr;
-        a.n = n;
-        a.task_cap = cap;
-        a.big_cap = big_cap;
-        a.big_min = kSahBigMin;
-        a.level = level;
-        a.err = counters + 3;
-        if (nbig) {
-            a.tasks_in = bigs[cur];
-            hipLaunchKernelGGL(k_sah_level<1024>, dim3(nbig), dim3(1024), 0, s, a);
-        }
-        if (nsmall) {
-            a.tasks_in = tasks[cur];
-            hipLaunchKernelGGL(k_sah_level<kBlock>, dim3(nsmall), dim3(kBlock), 0, s, a);
-        }
-        SOLHIP_HIP_CHECK(hipMemcpyAsync(pinned, counters, 36, hipMemcpyDeviceToHost, s));
-        SOLHIP_HIP_CHECK(hipStreamSynchronize(s));
-        if (pinned[3]) {
-            set_error("SAH BVH build range check failed at level " + std::to_string(level));
-            return SOLHIP_ERROR_DEVICE;
-        }
-        nsmall = pinned[6];
-        nbig = pinned[8];
-        ++level;
-        if (nsmall > cap || nbig > big_cap || level > kSahMedianLevel + 40) {
-            set_error("SAH BVH build did not converge");
-            return SOLHIP_ERROR_DEVICE;
-        }
-        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, counters + 6, 1u, 0u);
-        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, counters + 8, 1u, 0u);
-        cur ^= 1;
-    }
-    if (pinned[7] != n - 1) {
-        set_error("SAH BVH build made " + std::to_string(pinned[7]) + " internal nodes for " + std::to_string(n) +
-                  " primitives");
-        return SOLHIP_ERROR_DEVICE;
-    }
-    vals_out = vals;
-    return 0;
-}
-
 // Generic build over primitive boxes already in scratch.boxes (2 float4 per
 // primitive) with centroid bounds in scratch.bounds: a binary tree (Morton
 // order and radix tree, or binned SAH when `sah`), then the 8-wide collapse,
@@ -1122,13 +751,12 @@ static int build_common(hipStream_t s, uint32_t n, uint32_t leaf_max, bool sah, 
 {
     // counters (set by k_build_init): [0] wide nodes allocated, [1] leaf
     // records allocated, [2] collapse range errors, [3] sort / refit / SAH
-    // range errors, [4] invalid nodes, [5] refit frontier size, [6] SAH tasks
-    // of the next level, [7] SAH internal nodes allocated, [8] SAH big tasks,
-    // [9] vertex references out of range, kCntTicket, kCntLevels
+    // range errors, [4] invalid nodes, [5] refit frontier size, [9] vertex
+    // references out of range, kCntTicket, kCntLevels
     uint32_t *counters = (uint32_t *)sc.counters.ptr;
     uint32_t *pinned = sc.pinned;
     const uint32_t *vals = nullptr;
-    if (sah && n > 1) {
+    if (sah) {
         int rc = build_binary_sah(s, n, sc, vals);
         if (rc) return rc;
     } else {
@@ -1246,31 +874,35 @@ static int build_binary_lbvh(hipStream_t s, uint32_t n, DevScratch &sc, const ui
     return 0;
 }
 
-int DevScratch::ensure(uint32_t n)
+int DevScratch::ensure(uint32_t n, bool sah)
 {
     const uint64_t N = std::max<uint32_t>(n, 1);
-    const uint64_t ntiles = (N + kSortTile - 1) / kSortTile;
     int rc = 0;
     rc |= boxes.reserve(N * 32);
     rc |= bounds.reserve(64);
-    rc |= keys[0].reserve(N * 4);
-    rc |= keys[1].reserve(N * 4);
     rc |= vals[0].reserve(N * 4);
-    rc |= vals[1].reserve(N * 4);
-    rc |= hist.reserve(256 * ntiles * 4);
     rc |= left.reserve(N * 4);
     rc |= right.reserve(N * 4);
-    rc |= parent.reserve(2 * N * 4);
     rc |= rfirst.reserve(N * 4);
-    rc |= flags.reserve(N * 4);
     rc |= nbox.reserve(2 * N * 32);
     rc |= ncount.reserve(2 * N * 4);
     rc |= counters.reserve(kCntWords * 4);
     rc |= wsrc.reserve(N * 4);
     rc |= leaf_ids.reserve(N * 4);
-    rc |= frontier.reserve(N * 4);
+    if (sah) {
+        rc |= sah_work.reserve(sah_work_bytes(n));
+    } else {
+        const uint64_t ntiles = (N + kSortTile - 1) / kSortTile;
+        rc |= keys[0].reserve(N * 4);
+        rc |= keys[1].reserve(N * 4);
+        rc |= vals[1].reserve(N * 4);
+        rc |= hist.reserve(256 * ntiles * 4);
+        rc |= parent.reserve(2 * N * 4);
+        rc |= flags.reserve(N * 4);
+        rc |= frontier.reserve(N * 4);
+    }
     if (!pinned) {
-        if (hipHostMalloc((void **)&pinned, kCntWords * 4, hipHostMallocDefault) != hipSuccess) {
+        if (hipHostMalloc((void **)&pinned, kPinnedWords * 4, hipHostMallocDefault) != hipSuccess) {
             pinned = nullptr;
             set_error("hipHostMalloc failed");
             return SOLHIP_ERROR_OUT_OF_MEMORY;
@@ -1282,7 +914,7 @@ int DevScratch::ensure(uint32_t n)
 void DevScratch::release()
 {
     for (DevBuf *b : {&boxes, &bounds, &keys[0], &keys[1], &vals[0], &vals[1], &hist, &left, &right, &parent, &rfirst,
-                      &flags, &nbox, &ncount, &counters, &wsrc, &leaf_ids, &frontier})
+                      &flags, &nbox, &ncount, &counters, &wsrc, &leaf_ids, &frontier, &sah_work})
         b->release();
     for (auto &b : scan_bufs) b.release();
     scan_bufs.clear();
@@ -1290,7 +922,7 @@ void DevScratch::release()
     pinned = nullptr;
 }
 
-static_assert(kCntWords <= 128, "k_build_init runs one block of 128 threads");
+static_assert(kCntWords <= 128 && kCntWords <= kPinnedWords, "k_build_init runs one block of 128 threads");
 
 static void launch_build_init(hipStream_t s, DevScratch &sc)
 {
@@ -1301,7 +933,8 @@ static void launch_build_init(hipStream_t s, DevScratch &sc)
 int build_blas(hipStream_t s, const GeomDesc *geo_dev, uint32_t n_geo, uint32_t n, uint32_t flags, DevScratch &sc,
                DeviceBvh &out)
 {
-    int rc = sc.ensure(n);
+    const bool sah = (flags & SOLHIP_BUILD_PREFER_FAST_TRACE) != 0 && n > 1;
+    int rc = sc.ensure(n, sah);
     if (rc) return rc;
     const uint64_t nn = std::max<uint32_t>(n, 1);
     rc = out.nodes.reserve(nn * sizeof(WideNode));
@@ -1320,7 +953,7 @@ int build_blas(hipStream_t s, const GeomDesc *geo_dev, uint32_t n_geo, uint32_t 
     launch_build_init(s, sc);
     hipLaunchKernelGGL(k_tri_boxes, dim3(cdiv(n, kBlock)), dim3(kBlock), 0, s, geo_dev, n_geo, n,
                        (float4 *)sc.boxes.ptr, (uint32_t *)sc.bounds.ptr, counters + 9);
-    return build_common(s, n, kLeafMaxTri, (flags & SOLHIP_BUILD_PREFER_FAST_TRACE) != 0, sc, out, [&](uint32_t run) {
+    return build_common(s, n, kLeafMaxTri, sah, sc, out, [&](uint32_t run) {
         hipLaunchKernelGGL(k_write_tris, dim3(cdiv(n, kBlock)), dim3(kBlock), 0, s, (const uint32_t *)sc.leaf_ids.ptr,
                            n, geo_dev, n_geo, (TriRec *)out.leaves.ptr, counters, run);
     });
@@ -1329,7 +962,7 @@ int build_blas(hipStream_t s, const GeomDesc *geo_dev, uint32_t n_geo, uint32_t 
 int build_tlas(hipStream_t s, const solhip_instance *inst_dev, const BlasRef *refs_dev, uint32_t n, DevScratch &sc,
                DeviceBvh &out)
 {
-    int rc = sc.ensure(n);
+    int rc = sc.ensure(n, false);
     if (rc) return rc;
     const uint64_t nn = std::max<uint32_t>(n, 1);
     rc = out.nodes.reserve(nn * sizeof(WideNode));

@@ -57,6 +57,39 @@ __device__ __forceinline__ float group8_fmax(float v)
     }));
 }
 
+// whole wave: rows of 16 by row_shr, then across rows by row_bcast; the result
+// is in lane 63 and returned to every lane
+template <class Op>
+__device__ __forceinline__ uint32_t wave_reduce(uint32_t v, uint32_t identity, Op op)
+{
+    v = op(v, dpp<0x111>(identity, v));
+    v = op(v, dpp<0x112>(identity, v));
+    v = op(v, dpp<0x114>(identity, v));
+    v = op(v, dpp<0x118>(identity, v));
+    v = op(v, dpp<0x142, 0xA>(identity, v));
+    v = op(v, dpp<0x143, 0xC>(identity, v));
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+__device__ __forceinline__ uint32_t wave_min(uint32_t v)
+{
+    return wave_reduce(v, 0xFFFFFFFFu, [](uint32_t a, uint32_t b) { return min(a, b); });
+}
+__device__ __forceinline__ uint32_t wave_max(uint32_t v)
+{
+    return wave_reduce(v, 0u, [](uint32_t a, uint32_t b) { return max(a, b); });
+}
+
+// inclusive scan within each half of 32 lanes
+template <class Op>
+__device__ __forceinline__ uint32_t half_scan(uint32_t v, uint32_t identity, Op op)
+{
+    v = op(v, dpp<0x111>(identity, v));
+    v = op(v, dpp<0x112>(identity, v));
+    v = op(v, dpp<0x114>(identity, v));
+    v = op(v, dpp<0x118>(identity, v));
+    return op(v, dpp<0x142, 0xA>(identity, v));
+}
+
 // orders this wave's LDS accesses (no other wave is involved)
 __device__ __forceinline__ void wave_lds_sync()
 {
