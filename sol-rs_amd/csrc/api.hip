@@ -19,7 +19,7 @@
 #include "objects.h"
 #include "kernels.h"
 #include "accum.h"
-#include "traverse.h"
+#include "traverse_step.h"
 
 namespace solhip {
 
@@ -119,6 +119,7 @@ SceneView view_of(const Tlas *t)
     SceneView v;
     v.stack_depth = std::min<uint32_t>(stack_depth_of(t), (uint32_t)kMaxStack);
     v.single = t->bvh.prim_count == 1 ? 1u : 0u;
+    v.mode = v.single ? kTravSingle : (t->identity ? kTravIdentity : kTravGeneral);
     if (t->bvh.prim_count == 0) {
         v.tnodes = nullptr;
         v.insts = nullptr;
@@ -137,6 +138,8 @@ int tlas_build_into(Context *cx, hipStream_t s, Tlas *t, const solhip_instance *
     std::vector<uint32_t> tris(n ? n : 1, 0u);
     t->built = false;
     t->multi_geo = false;
+    t->identity = n > 0;
+    static const float kIdentity[12] = {1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0};
     t->blas_handles.clear();
     t->blas_gens.clear();
     for (uint32_t i = 0; i < n; ++i) {
@@ -163,6 +166,7 @@ int tlas_build_into(Context *cx, hipStream_t s, Tlas *t, const solhip_instance *
         refs[i].root_box = (const float *)b->bvh.root_box.ptr;
         refs[i].geo = b->geo_table();
         if (refs[i].geo) t->multi_geo = true;
+        if (std::memcmp(inst[i].transform, kIdentity, sizeof(kIdentity)) != 0) t->identity = false;
         tris[i] = b->bvh.prim_count;
     }
     const uint64_t nn = n ? n : 1;
@@ -1069,6 +1073,7 @@ int trace_program(solhip_ctx ctx, solhip_stream st, solhip_program ph, solhip_tl
     a.enable_sky = p->spec.enable_sky;
     a.spp = p->spec.spp_per_frame;
     a.max_depth = p->spec.max_depth;
+    a.ncu = c->ncu;
     a.counters = c->counters;
     a.count = (c->profile & SOLHIP_PROFILE_COUNT) != 0;
     if (images->hits_out) {
@@ -1103,7 +1108,6 @@ int trace_program(solhip_ctx ctx, solhip_stream st, solhip_program ph, solhip_tl
             a.qcount = (uint32_t *)p->qcount.ptr;
             a.occl = (uint8_t *)p->occl.ptr;
         }
-        a.ncu = c->ncu;
         int rc = launch_fill(s, a.qcount, 2, 0u);
         if (rc) return rc;
         rc = launch_ao(s, a, timer);

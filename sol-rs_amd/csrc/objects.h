@@ -120,6 +120,7 @@ struct Tlas : Obj {
     std::vector<uint64_t> blas_handles;   // distinct BLAS referenced by the instances
     std::vector<uint64_t> blas_gens;      // their generations when this TLAS was built
     uint32_t n_inst = 0;
+    bool identity = false;                // every instance is at the identity transform
     bool multi_geo = false;               // some instance's BLAS has several geometries
     bool built = false;                   // the last (re)build succeeded
     uint64_t gen = 0;

@@ -5,7 +5,9 @@
 #include <hip/hip_runtime.h>
 
 #include "kernels.h"
-#include "traverse.h"
+#include <type_traits>
+
+#include "traverse_step.h"
 
 namespace solhip {
 
@@ -14,6 +16,20 @@ namespace solhip {
 #endif
 constexpr int kProgBlock = SOLHIP_PROG_BLOCK;  // a multiple of 64
 constexpr int kTileH = kProgBlock / 8;          // pixel tiles are 8 x kTileH
+
+// launch(mode, count) with a scene's traversal form and the counting switch as
+// compile-time constants (.value)
+template <class Launch>
+inline void trav_dispatch(uint32_t mode, bool count, Launch launch)
+{
+    auto with_mode = [&](auto m) {
+        if (count) launch(m, std::true_type{});
+        else launch(m, std::false_type{});
+    };
+    if (mode == kTravSingle) with_mode(std::integral_constant<int, kTravSingle>{});
+    else if (mode == kTravIdentity) with_mode(std::integral_constant<int, kTravIdentity>{});
+    else with_mode(std::integral_constant<int, kTravGeneral>{});
+}
 
 __device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nb)
 {

@@ -3,7 +3,7 @@
 
 #include "bvh.h"
 #include "kernels.h"
-#include "traverse.h"
+#include "shading.h"
 #include "traverse_step.h"
 
 namespace solhip {
@@ -36,7 +36,7 @@ __device__ __forceinline__ void add_counts(Counters *c, const TravCounts &t, boo
     }
 }
 
-template <bool ANY, bool COUNT>
+template <bool ANY, bool COUNT, int MODE>
 __global__ void __launch_bounds__(kTraceBlock) k_trace_rays(SceneView sv, const solhip_ray *rays, solhip_hit *hits,
                                                             uint32_t n, Counters *counters)
 {
@@ -52,8 +52,8 @@ __global__ void __launch_bounds__(kTraceBlock) k_trace_rays(SceneView sv, const 
         // and counts, in fewer registers); sv.stack_depth includes its two
         // extra entries
         TravState st;
-        trav_init(st, sv, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w);
-        while (!trav_step<ANY, COUNT>(st, sv, 0xFFu, stack + threadIdx.x, kTraceBlock, tc)) {
+        trav_init<MODE, COUNT>(st, sv, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, 0xFFu, tc);
+        while (!trav_step<ANY, COUNT, true, MODE>(st, sv, 0xFFu, stack + threadIdx.x, kTraceBlock, tc)) {
         }
         const Hit h = trav_result(st);
         solhip_hit o;
@@ -84,14 +84,12 @@ int launch_trace_rays(hipStream_t s, const SceneView &sv, const solhip_ray *rays
     v.stack_depth += 2;
     const size_t lds = (size_t)v.stack_depth * sizeof(uint2) * kTraceBlock;
     const bool any = flags & SOLHIP_TRACE_TERMINATE_ON_FIRST_HIT, count = flags & SOLHIP_TRACE_COUNT;
-    if (any && count)
-        hipLaunchKernelGGL((k_trace_rays<true, true>), grid, block, lds, s, v, rays, hits, n, counters);
-    else if (any)
-        hipLaunchKernelGGL((k_trace_rays<true, false>), grid, block, lds, s, v, rays, hits, n, counters);
-    else if (count)
-        hipLaunchKernelGGL((k_trace_rays<false, true>), grid, block, lds, s, v, rays, hits, n, counters);
-    else
-        hipLaunchKernelGGL((k_trace_rays<false, false>), grid, block, lds, s, v, rays, hits, n, counters);
+    trav_dispatch(sv.mode, count, [&](auto mode, auto cnt) {
+        if (any)
+            hipLaunchKernelGGL((k_trace_rays<true, cnt.value, mode.value>), grid, block, lds, s, v, rays, hits, n, counters);
+        else
+            hipLaunchKernelGGL((k_trace_rays<false, cnt.value, mode.value>), grid, block, lds, s, v, rays, hits, n, counters);
+    });
     if (timer) timer->end(s, SOLHIP_KERNEL_TRACE_RAYS);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {

@@ -176,7 +176,6 @@ __global__ void k_pt_fold(WfArgs A, uint32_t pass)
 #define SOLHIP_WF_OCCUPANCY __attribute__((amdgpu_waves_per_eu(SOLHIP_WF_WAVES)))
 
 // lanes of a wave take new queue slots once at least this many are idle
-// (0: one slot per lane per 64-slot fetch, trace_ray to completion)
 #ifndef SOLHIP_WF_REFILL
 #define SOLHIP_WF_REFILL 16
 #endif
@@ -207,7 +206,7 @@ __device__ __forceinline__ void queue_result(const WfArgs &A, uint32_t i, uint32
 // the atomic head.  The resumable traversal lets a lane start its next slot
 // while the rest of the wave is still traversing.  sv.stack_depth includes
 // the two extra entries the step traversal may hold.
-template <bool ANY, bool COUNT>
+template <bool ANY, bool COUNT, int MODE>
 __device__ __forceinline__ void trace_queue(const WfArgs &A, const QRay *q, uint32_t cnt, uint32_t *heads, int kernel)
 {
     extern __shared__ uint2 stack[];
@@ -215,7 +214,6 @@ __device__ __forceinline__ void trace_queue(const WfArgs &A, const QRay *q, uint
     const float tmin = ray_tmin(A);
     TravCounts tc{0, 0, 0, false};
     uint32_t rays = 0;
-#if SOLHIP_WF_REFILL
     TravState st;
     bool has = false;
     uint32_t idx = 0, path = 0;
@@ -240,7 +238,8 @@ __device__ __forceinline__ void trace_queue(const WfArgs &A, const QRay *q, uint
                             queue_result<false>(A, my, r.path, miss);
                         }
                     } else {
-                        trav_init(st, A.sv, v3(r.ox, r.oy, r.oz), v3(r.dx, r.dy, r.dz), tmin, r.tmax);
+                        trav_init<MODE, COUNT>(st, A.sv, v3(r.ox, r.oy, r.oz), v3(r.dx, r.dy, r.dz), tmin, r.tmax, 0xFFu,
+                                               tc);
                         idx = my;
                         path = r.path;
                         has = true;
@@ -249,38 +248,16 @@ __device__ __forceinline__ void trace_queue(const WfArgs &A, const QRay *q, uint
             }
         }
         if (__ballot(has) == 0 && pf.exhausted) break;
-        if (has && trav_step<ANY, COUNT, SOLHIP_WF_WINV>(st, A.sv, 0xFFu, stack + threadIdx.x, A.block, tc)) {
+        if (has && trav_step<ANY, COUNT, SOLHIP_WF_WINV, MODE>(st, A.sv, 0xFFu, stack + threadIdx.x, A.block, tc)) {
             queue_result<ANY>(A, idx, path, trav_result(st));
             ++rays;
             has = false;
         }
     }
-#else
-    for (;;) {
-        uint32_t base = 0;
-        if (lane == 0) base = atomicAdd(heads, 64u);
-        base = __shfl(base, 0);
-        if (base >= cnt) break;
-        const uint32_t i = base + lane;
-        if (i < cnt) {
-            const QRay r = q[i];
-            Hit h;
-            h.t = -1.0f;
-            h.u = h.v = 0.0f;
-            h.inst = h.prim = SOLHIP_MISS;
-            if (r.path != kNoPath) {
-                h = trace_ray<ANY, COUNT>(A.sv, v3(r.ox, r.oy, r.oz), v3(r.dx, r.dy, r.dz), tmin, r.tmax, 0xFFu,
-                                          stack + threadIdx.x, A.block, tc);
-                ++rays;
-            }
-            if (!ANY || r.path != kNoPath) queue_result<ANY>(A, i, r.path, h);
-        }
-    }
-#endif
     count_rays<COUNT>(A.counters + kernel, rays, tc);
 }
 
-template <bool COUNT>
+template <bool COUNT, int MODE>
 __global__ void SOLHIP_WF_OCCUPANCY k_pt_extend(WfArgs A, uint32_t b)
 {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -288,14 +265,14 @@ __global__ void SOLHIP_WF_OCCUPANCY k_pt_extend(WfArgs A, uint32_t b)
         A.counts[(b + 1) & 1] = 0;
         A.counts[2] = 0;
     }
-    trace_queue<false, COUNT>(A, A.q[b & 1], A.counts[b & 1], A.heads + 2 * b * kWfParts * kHeadStride,
+    trace_queue<false, COUNT, MODE>(A, A.q[b & 1], A.counts[b & 1], A.heads + 2 * b * kWfParts * kHeadStride,
                               SOLHIP_KERNEL_PT_EXTEND);
 }
 
-template <bool COUNT>
+template <bool COUNT, int MODE>
 __global__ void SOLHIP_WF_OCCUPANCY k_pt_shadow(WfArgs A, uint32_t b)
 {
-    trace_queue<true, COUNT>(A, A.sq, A.counts[2], A.heads + (2 * b + 1) * kWfParts * kHeadStride,
+    trace_queue<true, COUNT, MODE>(A, A.sq, A.counts[2], A.heads + (2 * b + 1) * kWfParts * kHeadStride,
                              SOLHIP_KERNEL_PT_SHADOW);
 }
 
@@ -758,7 +735,7 @@ int launch_pathtrace_passes(hipStream_t s, const WfArgs &a0, Timer *timer, const
 {
     // the step traversal may hold two more stack entries than trace_ray
     WfArgs a = a0;
-    if (SOLHIP_WF_REFILL) a.sv.stack_depth += 2;
+    a.sv.stack_depth += 2;
     const uint32_t blk = a.block;
     const size_t lds = (size_t)a.sv.stack_depth * sizeof(uint2) * blk;
     const uint32_t nheads = 2 * (a.max_depth + 1);
@@ -788,8 +765,10 @@ int launch_pathtrace_passes(hipStream_t s, const WfArgs &a0, Timer *timer, const
         }
         for (uint32_t b = 0; b <= a.max_depth; ++b) {
             timed(SOLHIP_KERNEL_PT_EXTEND, [&] {
-                if (a.count) hipLaunchKernelGGL(k_pt_extend<true>, dim3(a.persist_blocks), dim3(blk), lds, s, a, b);
-                else hipLaunchKernelGGL(k_pt_extend<false>, dim3(a.persist_blocks), dim3(blk), lds, s, a, b);
+                trav_dispatch(a.sv.mode, a.count, [&](auto mode, auto count) {
+                    hipLaunchKernelGGL((k_pt_extend<count.value, mode.value>), dim3(a.persist_blocks), dim3(blk), lds,
+                                       s, a, b);
+                });
             });
             timed(SOLHIP_KERNEL_PT_SHADE, [&] {
                 if (nrc) hipLaunchKernelGGL(k_pt_shade_nrc, dim3(a.shade_blocks), dim3(blk), 0, s, a, b);
@@ -802,8 +781,10 @@ int launch_pathtrace_passes(hipStream_t s, const WfArgs &a0, Timer *timer, const
             }
             if (shadows && b < a.max_depth) {
                 timed(SOLHIP_KERNEL_PT_SHADOW, [&] {
-                    if (a.count) hipLaunchKernelGGL(k_pt_shadow<true>, dim3(a.persist_blocks), dim3(blk), lds, s, a, b);
-                    else hipLaunchKernelGGL(k_pt_shadow<false>, dim3(a.persist_blocks), dim3(blk), lds, s, a, b);
+                    trav_dispatch(a.sv.mode, a.count, [&](auto mode, auto count) {
+                        hipLaunchKernelGGL((k_pt_shadow<count.value, mode.value>), dim3(a.persist_blocks), dim3(blk),
+                                           lds, s, a, b);
+                    });
                 });
             }
         }
