@@ -256,6 +256,39 @@ int launch_ao(hipStream_t s, const ProgArgs &a, Timer *timer)
 // ---------------------------------------------------------------------------
 // The GLSL programs' pixel loops (ao.*, pathtrace.*)
 // ---------------------------------------------------------------------------
+// A pixel's samples follow one another (one random stream per pixel), and each
+// is a chain of rays.  Two kernels run the same pixel code (AoPixel, PtPixel):
+//
+//   k_pixels_lockstep  one lane per pixel, each ray traced to its end before
+//                      the next.  A wave waits for its slowest ray, then its longest path
+//                      of every sample: cheap while paths are short.
+//   k_pixels           a lane runs its pixel as a state machine on the
+//                      resumable traversal: a ray that is done waits until at
+//                      least SOLHIP_MEGA_SHADE lanes of the wave have something to shade, and
+//                      a lane whose pixel is finished takes the block's next one.  Block b
+//                      owns the 8x8 tiles b, b + grid, b + 2 grid, ... and hands out
+//                      their pixels through a cursor in LDS: no device memory, so
+//                      overlapping launches share nothing.
+//
+// Both are bound by VALU issue (0.58 wave-instructions per ns and SIMD set)
+// with few lanes active: 8.4 of 64 in lockstep on 32-bounce paths, 16.8 as a
+// state machine, which costs a quarter more instructions per ray.  Cornell box, 8
+// samples, 1280x720: depth 32 12.8 -> 6.5 ms, depth 8 4.5 -> 4.0, depth 4 2.6
+// against 3.1; 500x400 (fewer pixels than resident lanes): 5.7 -> 3.9, 2.04
+// against 2.09, 1.15 against 1.42; ao.* (at most 5 rays a sample), 900x600: 0.97 against 1.13.
+// waits of 16 to 64 lanes are within 4 %; 512 threads per block 5 % better than
+// 256, 5 waves per SIMD spill (9.9 ms)
+#ifndef SOLHIP_MEGA_SHADE
+#define SOLHIP_MEGA_SHADE 48
+#endif
+#ifndef SOLHIP_MEGA_WAVES
+#define SOLHIP_MEGA_WAVES 4
+#endif
+#ifndef SOLHIP_MEGA_BLOCK
+#define SOLHIP_MEGA_BLOCK 512
+#endif
+constexpr uint32_t kMegaBlock = SOLHIP_MEGA_BLOCK;
+
 // a lane's ray
 struct Segment {
     V3 o, d;
@@ -433,6 +466,80 @@ struct PtPixel {
 };
 
 template <class Pixel, bool COUNT, int MODE>
+__global__ void __launch_bounds__(kMegaBlock) __attribute__((amdgpu_waves_per_eu(SOLHIP_MEGA_WAVES)))
+k_pixels(ProgArgs A)
+{
+    extern __shared__ uint2 stack[];
+    __shared__ uint32_t s_cursor;
+    if (threadIdx.x == 0) s_cursor = 0;
+    __syncthreads();
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t tiles_x = (A.W + 7) >> 3, tiles = tiles_x * ((A.H + 7) >> 3);
+    // pixels of this block's tiles (in 64 bits: a tile count near 2^32 times 64)
+    const uint64_t items = (uint64_t)((tiles - blockIdx.x + gridDim.x - 1) / gridDim.x) * 64u;
+    TravCounts tc{0, 0, 0, false};
+    uint32_t rays = 0;
+    TravState st;
+    Pixel p;
+    enum : uint32_t { kWant, kTrace, kHit, kEnd };
+    uint32_t state = kWant;
+    while (true) {
+        const uint64_t waiting = __ballot(state == kWant || state == kHit);
+        const bool tracing = __ballot(state == kTrace) != 0;
+        if (!waiting && !tracing) break;
+        if (!tracing || __popcll(waiting) >= SOLHIP_MEGA_SHADE) {
+            Segment r;
+            bool go = false, fresh = false;
+            if (state == kHit) {
+                r.o = st.wo;
+                r.d = st.wd;
+                r.tmin = st.tmin;
+                r.tmax = 10000.0f;   // a pathtrace segment's; ao sets its own
+                const After a = p.shade(A, trav_result(st), r);
+                go = a == After::kRay;
+                fresh = a == After::kSample;
+                if (a == After::kPixel) {
+                    p.finish(A);
+                    state = kWant;
+                }
+            }
+            // lanes without a pixel take the block's next ones
+            for (uint64_t want; (want = __ballot(state == kWant)) != 0;) {
+                uint32_t base = 0;
+                if (lane == (uint32_t)__ffsll((unsigned long long)want) - 1u)
+                    base = atomicAdd(&s_cursor, (uint32_t)__popcll(want));
+                base = __shfl(base, __ffsll((unsigned long long)want) - 1);
+                if (state == kWant) {
+                    const uint32_t k = base + (uint32_t)__popcll(want & ((1ull << lane) - 1ull));
+                    if (k >= items) {
+                        state = kEnd;
+                    } else {
+                        const uint32_t tile = blockIdx.x + (k >> 6) * gridDim.x;
+                        const uint32_t x = (tile % tiles_x) * 8 + (k & 7u), y = (tile / tiles_x) * 8 + ((k >> 3) & 7u);
+                        if (x < A.W && y < A.H) {
+                            p.begin(A, x, y);
+                            fresh = true;
+                            state = kHit;   // leaves the loop; traced below
+                        }
+                    }
+                }
+            }
+            if (fresh) p.camera(A, r);
+            if (go || fresh) {
+                trav_init<MODE, COUNT>(st, A.sv, r.o, r.d, r.tmin, r.tmax, 0xFFu, tc);
+                state = kTrace;
+            }
+        }
+        if (state == kTrace &&
+            trav_step<false, COUNT, true, MODE>(st, A.sv, 0xFFu, stack + threadIdx.x, (int)blockDim.x, tc)) {
+            state = kHit;
+            ++rays;
+        }
+    }
+    count_rays<COUNT>(A.counters + Pixel::kKernel, rays, tc);
+}
+
+template <class Pixel, bool COUNT, int MODE>
 __global__ void __launch_bounds__(kProgBlock) k_pixels_lockstep(ProgArgs A)
 {
     extern __shared__ uint2 stack[];
@@ -458,6 +565,22 @@ __global__ void __launch_bounds__(kProgBlock) k_pixels_lockstep(ProgArgs A)
 }
 
 template <class Pixel>
+static void launch_pixels(hipStream_t s, const ProgArgs &a)
+{
+    ProgArgs p = a;
+    p.sv.stack_depth = a.sv.stack_depth + 2;   // the step traversal's two extra entries
+    // blocks of kMegaBlock lanes, or fewer where their stacks would pass 64 KiB of LDS
+    uint32_t block = kMegaBlock;
+    while (block > 64 && (size_t)p.sv.stack_depth * sizeof(uint2) * block > 65536) block /= 2;
+    const size_t lds = (size_t)p.sv.stack_depth * sizeof(uint2) * block;
+    const uint64_t tiles = (uint64_t)((a.W + 7) / 8) * ((a.H + 7) / 8);
+    const uint32_t grid = (uint32_t)std::min<uint64_t>(tiles, (uint64_t)a.ncu * (4u * SOLHIP_MEGA_WAVES * 64u / block));
+    trav_dispatch(a.sv.mode, a.count, [&](auto mode, auto count) {
+        hipLaunchKernelGGL((k_pixels<Pixel, count.value, mode.value>), dim3(grid), dim3(block), lds, s, p);
+    });
+}
+
+template <class Pixel>
 static void launch_lockstep(hipStream_t s, const ProgArgs &a)
 {
     trav_dispatch(a.sv.mode, a.count, [&](auto mode, auto count) {
@@ -476,8 +599,15 @@ int launch_ao_glsl(hipStream_t s, const ProgArgs &a, Timer *timer)
 
 int launch_pathtrace_glsl(hipStream_t s, const ProgArgs &a, Timer *timer)
 {
+    // long paths differ enough in length for the state machine to pay off, with
+    // 8 bounces only where lanes also get a second pixel (twice the resident
+    // lanes), and from 16 where a lane has a second sample or a second pixel;
+    // see the times above
+    const bool refills = (uint64_t)a.W * a.H >= 2ull * a.ncu * 4u * SOLHIP_MEGA_WAVES * 64u;
+    const bool machine = a.max_depth >= 16 ? refills || a.spp >= 2 : a.max_depth >= 8 && refills;
     if (timer) timer->begin(s, SOLHIP_KERNEL_PATHTRACE_GLSL);
-    launch_lockstep<PtPixel>(s, a);
+    if (machine) launch_pixels<PtPixel>(s, a);
+    else launch_lockstep<PtPixel>(s, a);
     if (timer) timer->end(s, SOLHIP_KERNEL_PATHTRACE_GLSL);
     return launch_status("pathtrace");
 }
