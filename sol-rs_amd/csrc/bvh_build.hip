@@ -511,6 +511,7 @@ __global__ void __launch_bounds__(kCollapseBlock) k_collapse(CollapseDev A)
         const uint32_t inner_slots = group_bits(inner);
         const uint32_t imask = act ? inner_slots : 0u;
         const uint32_t lcnt = act && leaf ? scnt : 0u;
+        const uint32_t leaf_mask = group8(((1u << lcnt) - 1u) << (3u * c), [](uint32_t x, uint32_t y) { return x | y; });
         uint32_t poff = lcnt;
         for (int d = 1; d < 8; d <<= 1) {
             const uint32_t t = __shfl_up(poff, d, 8);
@@ -566,7 +567,6 @@ __global__ void __launch_bounds__(kCollapseBlock) k_collapse(CollapseDev A)
                 nb[32 + 8 * a + c] = (uint8_t)ql;
                 nb[56 + 8 * a + c] = (uint8_t)qh;
             }
-            nb[24 + c] = leaf ? (uint8_t)((scnt << 5) | poff) : (uint8_t)0;
             if (c == 0) {
                 uint32_t *h = reinterpret_cast<uint32_t *>(nb);
                 h[0] = __float_as_uint(org[0]);
@@ -575,6 +575,8 @@ __global__ void __launch_bounds__(kCollapseBlock) k_collapse(CollapseDev A)
                 h[3] = eb[0] | (eb[1] << 8) | (eb[2] << 16) | (imask << 24);
                 h[4] = child_base;
                 h[5] = prim_base;
+                h[6] = leaf_mask;
+                h[7] = 0u;
             }
             if (inner) A.wsrc[child_base + (uint32_t)__builtin_popcount(imask & ((1u << c) - 1u))] = id;
             if (leaf)

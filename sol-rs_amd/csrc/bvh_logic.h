@@ -377,13 +377,14 @@ SOLHIP_HD uint32_t collapse_node(const CollapseArgs &A, uint32_t w, Alloc alloc)
     nd.imask = (uint8_t)imask;
     nd.child_base = child_base;
     nd.prim_base = prim_base;
+    nd.leaf_mask = 0;
+    nd.unused = 0;
     uint32_t rank = 0, poff = 0;
     for (int s = 0; s < 8; ++s) {
         const int c = child_in[s];
         uint8_t *qlo[3] = {nd.qlo_x, nd.qlo_y, nd.qlo_z};
         uint8_t *qhi[3] = {nd.qhi_x, nd.qhi_y, nd.qhi_z};
         if (c < 0) {
-            nd.meta[s] = 0;
             for (int a = 0; a < 3; ++a) {
                 qlo[a][s] = 255;
                 qhi[a][s] = 0;
@@ -401,11 +402,10 @@ SOLHIP_HD uint32_t collapse_node(const CollapseArgs &A, uint32_t w, Alloc alloc)
         }
         const uint32_t cnt = A.ncount[bn];
         if ((imask >> s) & 1u) {
-            nd.meta[s] = 0;
             A.wsrc[child_base + rank] = bn;
             ++rank;
         } else {
-            nd.meta[s] = (uint8_t)((cnt << 5) | poff);
+            nd.leaf_mask |= ((1u << cnt) - 1u) << (3 * s);
             const uint32_t first = bn >= (uint32_t)(n - 1) ? bn - (uint32_t)(n - 1) : A.rfirst[bn];
             if ((uint64_t)first + cnt > (uint64_t)n) return 1;
             for (uint32_t j = 0; j < cnt; ++j) A.leaf_ids[prim_base + poff + j] = A.vals[first + j];
@@ -422,16 +422,16 @@ SOLHIP_HD bool node_valid(const WideNode &nd, uint32_t w, uint32_t nodes, uint32
 {
     uint32_t nint = 0, nprim = 0;
     for (int s = 0; s < 8; ++s) {
+        const uint32_t m = (nd.leaf_mask >> (3 * s)) & 7u;
         if ((nd.imask >> s) & 1u) {
             ++nint;
-            continue;
+            if (m) return false;   // both a child node and a leaf
+        } else if (m & (m + 1u)) {
+            return false;          // a leaf's bits start at its first
         }
-        const uint32_t m = nd.meta[s];
-        if (!m) continue;
-        const uint32_t cnt = m >> 5, off = m & 31u;
-        if (cnt == 0 || (uint64_t)nd.prim_base + off + cnt > prims) return false;
-        nprim += cnt;
+        nprim += (uint32_t)__builtin_popcount(m);
     }
+    if (nd.leaf_mask >> 24) return false;
     if (nint && (nd.child_base <= w || (uint64_t)nd.child_base + nint > nodes)) return false;
     if (nprim && (uint64_t)nd.prim_base + nprim > prims) return false;
     return true;

@@ -12,7 +12,10 @@
 //     uint32   child_base        node index of the first internal child; the
 //                                child in slot s is child_base + popc(imask & (2^s-1))
 //     uint32   prim_base         leaf-record index of the node's first leaf primitive
-//     uint8    meta[8]           leaf slot s: (count << 5) | offset from prim_base
+//     uint32   leaf_mask         leaf slot s with c primitives: bits 3s .. 3s+c-1;
+//                                the record of bit k is
+//                                prim_base + popc(leaf_mask & (2^k-1))
+//     uint32   unused
 //     uint8    qlo_x[8], qlo_y[8], qlo_z[8], qhi_x[8], qhi_y[8], qhi_z[8]
 //                                child boxes, rounded outward and padded by
 //                                one quantisation step
@@ -48,7 +51,7 @@ struct alignas(16) WideNode {
     uint8_t ex, ey, ez, imask;
     uint32_t child_base;
     uint32_t prim_base;
-    uint8_t meta[8];
+    uint32_t leaf_mask, unused;
     uint8_t qlo_x[8], qlo_y[8], qlo_z[8];
     uint8_t qhi_x[8], qhi_y[8], qhi_z[8];
 };

@@ -170,36 +170,41 @@ typedef const __attribute__((address_space(1))) uint32_t *gptr1;
 #define SOLHIP_G1(p) ((const uint32_t *)(p))
 #endif
 
-// reverse the 8-bit slot-order mask into visit order: bit i <-> slot i ^ oct
+// the 8-bit slot-order mask in visit order: bit i <-> slot i ^ oct (three
+// conditional swaps; a shift by 0 leaves the mask as it is)
 SOLHIP_HD uint32_t to_visit_order(uint32_t m, uint32_t oct)
 {
-    if (oct & 1u) m = ((m & 0x55u) << 1) | ((m & 0xAAu) >> 1);
-    if (oct & 2u) m = ((m & 0x33u) << 2) | ((m & 0xCCu) >> 2);
-    if (oct & 4u) m = ((m & 0x0Fu) << 4) | ((m & 0xF0u) >> 4);
-    return m;
+    const uint32_t s1 = oct & 1u, s2 = oct & 2u, s4 = oct & 4u;
+    m = ((m >> s1) & 0x55u) | ((m << s1) & 0xAAu);
+    m = ((m >> s2) & 0x33u) | ((m << s2) & 0xCCu);
+    return ((m >> s4) & 0x0Fu) | ((m << s4) & 0xF0u);
 }
 
-// count bits set from bit offset up: ((1 << count) - 1) << offset (count <=
-// 31).  BFM: on the device one v_bfm_b32 (the compiler turns the shifts into
-// a longer sequence).  The step traversal gains from it; trace_ray, whose
-// loop the compiler schedules around it less well, does not.
-template <bool BFM>
-SOLHIP_HD uint32_t bit_range(uint32_t count, uint32_t offset)
+// (m << 1) | (1 where the slab interval [tn, tf] is empty), from the sign of
+// tf - tn: two instructions, where a compare, a select and an or are three.  A
+// NaN (both infinite) counts as not empty.
+SOLHIP_HD uint32_t push_miss(uint32_t m, float tn, float tf)
 {
+    const float d = tf - tn;
 #if defined(__HIP_DEVICE_COMPILE__)
-    if (BFM) {
-        uint32_t m;
-        asm("v_bfm_b32 %0, %1, %2" : "=v"(m) : "v"(count), "v"(offset));
-        return m;
-    }
+    return __builtin_amdgcn_alignbit(m, as_u(d), 31);
+#else
+    return (m << 1) | (d == d ? as_u(d) >> 31 : 0u);
 #endif
-    return ((1u << count) - 1u) << offset;
 }
 
-// Intersect the 8 child boxes of a node (branch-free).  Returns
-// internal-child hits in visit order (bit i <-> slot i ^ oct) and the mask of
-// leaf primitives (relative to prim_base) of the leaf children hit.
-template <bool BFM = false>
+// the leaf record of primitive bit k of a leaf group (base: the node's first
+// record, valid: its leaf_mask)
+SOLHIP_HD uint32_t leaf_record(uint32_t base, uint32_t valid, uint32_t k)
+{
+    return base + (uint32_t)__builtin_popcount(valid & ((1u << k) - 1u));
+}
+
+// Intersect the 8 child boxes of a node (branch-free).  Returns internal-child
+// hits in visit order (bit i <-> slot i ^ oct) and the hit part of the node's
+// leaf_mask.  Leaves cost nothing per slot: the 8 hit bits are spread to 3 bits a
+// slot once and cut with the node's leaf_mask (a count and an offset
+// per slot, turned into a bit range, were 5 of 24 instructions per slot).
 SOLHIP_HD void intersect_node(const uint4 w0, const uint4 w1, const uint4 w2, const uint4 w3, const uint4 w4, V3 o,
                               V3 inv, uint32_t oct, float tlo, float thi, uint32_t &hits_int, uint32_t &prim_mask)
 {
@@ -219,9 +224,9 @@ SOLHIP_HD void intersect_node(const uint4 w0, const uint4 w1, const uint4 w2, co
     const uint32_t ffy0 = fy ? w2.z : w4.x, ffy1 = fy ? w2.w : w4.y;
     const uint32_t nz0 = fz ? w4.z : w3.x, nz1 = fz ? w4.w : w3.y;
     const uint32_t ffz0 = fz ? w3.x : w4.z, ffz1 = fz ? w3.y : w4.w;
-    uint32_t hm = 0, pm = 0;
+    uint32_t miss = 0;
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
+    for (int s = 7; s >= 0; --s) {
         const int b = s & 3;
         const uint32_t anx = s < 4 ? nx0 : nx1, any_ = s < 4 ? ny0 : ny1, anz = s < 4 ? nz0 : nz1;
         const uint32_t afx = s < 4 ? ffx0 : ffx1, afy = s < 4 ? ffy0 : ffy1, afz = s < 4 ? ffz0 : ffz1;
@@ -233,15 +238,15 @@ SOLHIP_HD void intersect_node(const uint4 w0, const uint4 w1, const uint4 w2, co
         const float tfz = fmaf(byte_f(afz, b), sz, bz);
         const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, tlo));
         const float tf = fminf(fminf(tfx, tfy), fminf(tfz, thi));
-        const bool hit = tn <= tf;
-        // leaf slot: (count << 5) | offset; internal and empty slots: 0
-        const uint32_t meta = ((s < 4 ? w1.z : w1.w) >> (8 * b)) & 0xFFu;
-        const uint32_t lm = bit_range<BFM>(meta >> 5, meta & 31u);
-        hm |= hit ? (1u << s) : 0u;
-        pm |= hit ? lm : 0u;
+        miss = push_miss(miss, tn, tf);
     }
-    hits_int = to_visit_order(hm & imask, oct);
-    prim_mask = pm;
+    const uint32_t hit = ~miss & 0xFFu;
+    hits_int = to_visit_order(hit & imask, oct);
+    // 8 bits to 3 bits a slot
+    uint32_t x = (hit | (hit << 8)) & 0x00F00Fu;
+    x = (x | (x << 4)) & 0x0C30C3u;
+    x = (x | (x << 2)) & 0x249249u;
+    prim_mask = ((x << 3) - x) & w1.z;
 }
 
 // forms of a scene (SceneView::mode): any; one instance; every instance at the
@@ -304,13 +309,13 @@ SOLHIP_HD Hit trace_ray(const SceneView sv, V3 wo, V3 wd, float tmin, float tmax
             const Wt wt = ray.wt;
             const int base = sp;
             uint32_t ng_base = 0, ng_hits = 1u << oct, ng_imask = 1u;
-            uint32_t tg_base = 0, tg_mask = 0;
+            uint32_t tg_base = 0, tg_mask = 0, tg_valid = 0;
             while (true) {
                 if (tg_mask) {
                     // one triangle per iteration
                     const uint32_t k = __builtin_ctz(tg_mask);
                     tg_mask &= tg_mask - 1u;
-                    const uint4 *tp = reinterpret_cast<const uint4 *>(tris + tg_base + k);
+                    const uint4 *tp = reinterpret_cast<const uint4 *>(tris + leaf_record(tg_base, tg_valid, k));
                     const uint4 a = SOLHIP_G4(tp)[0], b = SOLHIP_G4(tp)[1];
                     const uint2 c = SOLHIP_G2(tp + 2)[0];
                     const float vv[9] = {as_f(a.x), as_f(a.y), as_f(a.z), as_f(a.w), as_f(b.x),
@@ -343,6 +348,7 @@ SOLHIP_HD Hit trace_ray(const SceneView sv, V3 wo, V3 wd, float tmin, float tmax
                     ng_base = w1.x;
                     ng_imask = w0.w >> 24;
                     tg_base = w1.y;
+                    tg_valid = w1.z;
                 } else if (sp > base) {
                     const uint2 e = pop();
                     ng_base = e.x;
@@ -375,13 +381,13 @@ SOLHIP_HD Hit trace_ray(const SceneView sv, V3 wo, V3 wd, float tmin, float tmax
         const uint32_t woct = octant(wd);
         // the TLAS root, or, with one instance, its leaf (record 0) at once
         uint32_t ng_base = 0, ng_hits = sv.single ? 0u : 1u << woct, ng_imask = 1u;
-        uint32_t tg_base = 0, tg_mask = sv.single ? 1u : 0u;
+        uint32_t tg_base = 0, tg_mask = sv.single ? 1u : 0u, tg_valid = 1u;
         while (MODE != kTravSingle) {
             if (tg_mask) {
                 // instance leaf: transform the ray and trace its BLAS
                 const uint32_t k = __builtin_ctz(tg_mask);
                 tg_mask &= tg_mask - 1u;
-                const uint32_t li = tg_base + k;
+                const uint32_t li = leaf_record(tg_base, tg_valid, k);
                 const uint32_t meta = SOLHIP_G1(sv.inst_meta + li)[0];
                 if (((meta >> 24) & cull) == 0u) continue;
                 const uint4 *ip = reinterpret_cast<const uint4 *>(sv.insts + li);
@@ -414,6 +420,7 @@ SOLHIP_HD Hit trace_ray(const SceneView sv, V3 wo, V3 wd, float tmin, float tmax
                 ng_base = w1.x;
                 ng_imask = w0.w >> 24;
                 tg_base = w1.y;
+                tg_valid = w1.z;
             } else if (sp > 0) {
                 const uint2 e = pop();
                 ng_base = e.x;

@@ -44,7 +44,8 @@ struct TravState {
     uint32_t inst;             // instance index of the BLAS being traversed
     const WideNode *nodes;     // BLAS nodes
     const TriRec *tris;        // BLAS leaf records
-    uint32_t ng_base, ng_hits, ng_imask, tg_base, tg_mask;
+    uint32_t ng_base, ng_hits, ng_imask;
+    uint32_t tg_base, tg_mask, tg_valid;   // leaf group: first record, primitives left, the node's leaf_mask
     int sp, base;              // stack height; height at BLAS entry
     Hit best;
 };
@@ -75,6 +76,7 @@ SOLHIP_HD void trav_init(TravState &s, const SceneView &sv, V3 wo, V3 wd, float 
     s.tris = nullptr;
     s.tg_base = 0;
     s.tg_mask = 0;
+    s.tg_valid = 1u;
     s.ng_base = 0;
     s.ng_hits = 0;
     s.ng_imask = 1u;
@@ -139,7 +141,7 @@ SOLHIP_HD Hit trav_result(const TravState &s)
 
 // One traversal step; true when the ray is finished.  A step does, in this
 // order and each at most once: one triangle of the current leaf group, the
-// stack pops and BLAS exits that lead to the next piece of work, one instance
+// BLAS exit and stack pop that lead to the next piece of work, one instance
 // entry, one node test.  Running them as phases of one step (rather than one
 // of them per step) lets a wave's lanes share the expensive node test in the
 // same pass whatever bookkeeping each needed first.  lds: this lane's stack
@@ -159,7 +161,7 @@ SOLHIP_HD bool trav_step(TravState &s, const SceneView &sv, uint32_t cull, uint2
     if ((MODE == kTravSingle || s.level) && s.tg_mask) {
         const uint32_t k = __builtin_ctz(s.tg_mask);
         s.tg_mask &= s.tg_mask - 1u;
-        const uint4 *tp = reinterpret_cast<const uint4 *>(s.tris + s.tg_base + k);
+        const uint4 *tp = reinterpret_cast<const uint4 *>(s.tris + leaf_record(s.tg_base, s.tg_valid, k));
         const uint4 a = SOLHIP_G4(tp)[0], b = SOLHIP_G4(tp)[1];
         const uint2 c = SOLHIP_G2(tp + 2)[0];
         const float vv[9] = {as_f(a.x), as_f(a.y), as_f(a.z), as_f(a.w), as_f(b.x),
@@ -175,12 +177,11 @@ SOLHIP_HD bool trav_step(TravState &s, const SceneView &sv, uint32_t cull, uint2
             if (ANY) return true;
         }
     }
-    // 2. pops and BLAS exits up to the next node group or leaf group.  An
-    // empty stack ends the ray at once, also inside a BLAS: nothing of the
-    // TLAS is pending (its work is pushed below the BLAS entry), so the world
-    // ray need not be restored.  Some lane of a wave finishes in almost every
-    // step, so the restore would otherwise be issued in almost every step.
-    while (!s.tg_mask && !s.ng_hits) {
+    // 2. nothing left of the last node: the next stack entry (pushed groups are
+    // never empty, so one pop leads to work).  An empty stack ends the ray at
+    // once, also inside a BLAS: nothing of the TLAS is pending (its work is
+    // pushed below the BLAS entry), so the world ray need not be restored.
+    if (!s.tg_mask && !s.ng_hits) {
         if (s.sp == 0) return true;
         if (MODE != kTravSingle && s.level && s.sp == s.base) {
             // the BLAS is done: back to the world ray and the TLAS stack
@@ -190,24 +191,24 @@ SOLHIP_HD bool trav_step(TravState &s, const SceneView &sv, uint32_t cull, uint2
                 s.inv = WINV ? s.winv : safe_inv(s.wd);
                 s.oct = octant(s.wd);
             }
+        }
+        --s.sp;
+        const uint2 e = lds[s.sp * stride];
+        if (MODE != kTravSingle && (e.y & kLeafGroupTag)) {
+            s.tg_base = e.x;
+            s.tg_mask = e.y & ~kLeafGroupTag;
+            s.tg_valid = 0xFFFFFFu;
         } else {
-            --s.sp;
-            const uint2 e = lds[s.sp * stride];
-            if (MODE != kTravSingle && (e.y & kLeafGroupTag)) {
-                s.tg_base = e.x;
-                s.tg_mask = e.y & ~kLeafGroupTag;
-            } else {
-                s.ng_base = e.x;
-                s.ng_hits = e.y & 0xFFu;
-                s.ng_imask = (e.y >> 8) & 0xFFu;
-            }
+            s.ng_base = e.x;
+            s.ng_hits = e.y & 0xFFu;
+            s.ng_imask = (e.y >> 8) & 0xFFu;
         }
     }
     // 3. an instance leaf: enter its BLAS
     if (MODE != kTravSingle && !s.level && s.tg_mask) {
         const uint32_t k = __builtin_ctz(s.tg_mask);
         s.tg_mask &= s.tg_mask - 1u;
-        const uint32_t li = s.tg_base + k;
+        const uint32_t li = leaf_record(s.tg_base, s.tg_valid, k);
         const uint32_t meta = SOLHIP_G1(sv.inst_meta + li)[0];
         if (((meta >> 24) & cull) != 0u) {
             const uint4 *ip = reinterpret_cast<const uint4 *>(sv.insts + li);
@@ -231,8 +232,12 @@ SOLHIP_HD bool trav_step(TravState &s, const SceneView &sv, uint32_t cull, uint2
                     }
                 }
                 if (s.tg_mask) {
+                    // as record bits relative to the group's base
+                    uint32_t left = 0;
+                    for (uint32_t m = s.tg_mask; m; m &= m - 1u)
+                        left |= 1u << leaf_record(0u, s.tg_valid, (uint32_t)__builtin_ctz(m));
                     if (s.sp < depth) {
-                        lds[s.sp * stride] = make_uint2(s.tg_base, s.tg_mask | kLeafGroupTag);
+                        lds[s.sp * stride] = make_uint2(s.tg_base, left | kLeafGroupTag);
                         ++s.sp;
                     } else {
                         cnt.overflow = true;
@@ -276,10 +281,11 @@ SOLHIP_HD bool trav_step(TravState &s, const SceneView &sv, uint32_t cull, uint2
                     w4 = SOLHIP_G4(np)[4];
         if (COUNT) cnt.nodes++;
         const float thi = s.best.t + fabsf(s.best.t) * 0x1p-20f;
-        intersect_node<true>(w0, w1, w2, w3, w4, s.o, s.inv, s.oct, s.tlo, thi, s.ng_hits, s.tg_mask);
+        intersect_node(w0, w1, w2, w3, w4, s.o, s.inv, s.oct, s.tlo, thi, s.ng_hits, s.tg_mask);
         s.ng_base = w1.x;
         s.ng_imask = w0.w >> 24;
         s.tg_base = w1.y;
+        s.tg_valid = w1.z;
     }
     return false;
 }
