@@ -901,7 +901,7 @@ int32_t solhip_trace_rays(solhip_ctx ctx, solhip_stream st, solhip_tlas th, solh
         return SOLHIP_ERROR_UNSUPPORTED;
     }
     const int rc = launch_trace_rays(s, view_of(t), (const solhip_ray *)rb->ptr, (solhip_hit *)hb->ptr, n, flags,
-                                     c->counters + SOLHIP_KERNEL_TRACE_RAYS, c->timer_or_null());
+                                     c->ncu, c->counters + SOLHIP_KERNEL_TRACE_RAYS, c->timer_or_null());
     if (rc || !t->multi_geo) return rc;
     return launch_split_geometry(s, (solhip_hit *)hb->ptr, n, (const BlasRef *)t->refs_dev.ptr, t->n_inst);
 }

@@ -160,7 +160,7 @@ struct WfArgs {
 };
 
 int launch_trace_rays(hipStream_t s, const SceneView &sv, const solhip_ray *rays, solhip_hit *hits, uint32_t n,
-                      uint32_t flags, Counters *counters, Timer *timer);
+                      uint32_t flags, uint32_t ncu, Counters *counters, Timer *timer);
 // rewrites the BLAS-wide triangle index of every hit (geom = 0) into the
 // triangle index within its geometry and the geometry index, for instances
 // whose BLAS has several geometries (refs: the TLAS's BlasRef per instance)

@@ -9,6 +9,18 @@
 namespace solhip {
 
 constexpr int kTraceBlock = 64;
+// persistent query kernel: waves per SIMD, and idle lanes at which a wave takes
+// new rays (24 instead of 16: within 2 %; 6 waves: 13 % slower at 0.4M rays, level at 2M)
+#ifndef SOLHIP_TRACE_WAVES
+#define SOLHIP_TRACE_WAVES 5
+#endif
+#ifndef SOLHIP_TRACE_REFILL
+#define SOLHIP_TRACE_REFILL 16
+#endif
+// waves per SIMD that a small query is spread over
+#ifndef SOLHIP_TRACE_SPREAD
+#define SOLHIP_TRACE_SPREAD 1
+#endif
 
 // XCD-aware block order: workgroups are dispatched round-robin over the 8
 // XCDs, so physical block b runs on XCD b % 8.  Mapping each XCD to a
@@ -36,14 +48,42 @@ __device__ __forceinline__ void add_counts(Counters *c, const TravCounts &t, boo
     }
 }
 
+// the end of a traversal kernel's wave: the launch's ray count (known without
+// counting) is added once, by the first wave; one atomic per wave on that
+// counter took about 15 ns each
+__device__ __forceinline__ void end_wave(Counters *counters, uint32_t n, bool count, const TravCounts &tc, bool active)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&counters->rays, (unsigned long long)n);
+    const uint64_t ov = __ballot(active && tc.overflow);
+    if (ov && (threadIdx.x & 63) == 0) atomicAdd(&counters->overflow, (unsigned long long)__popcll(ov));
+    if (count) add_counts(counters, tc, active);
+}
+
+__device__ __forceinline__ void write_hit(solhip_hit *dst, const TravState &st)
+{
+    const Hit h = trav_result(st);
+    solhip_hit o;
+    o.t = h.t;
+    o.u = h.u;
+    o.v = h.v;
+    o.inst = h.inst;
+    o.prim = h.prim;
+    o.geom = h.inst == SOLHIP_MISS ? SOLHIP_MISS : 0u;
+    *dst = o;
+}
+
+// One ray per lane in the first `lanes` lanes of every wave.  A query that
+// would leave SIMDs without a wave is bound by the chain of steps of its slowest
+// wave, and a step issues the work of all its lanes: fewer lanes per wave make
+// shorter chains on SIMDs that are idle otherwise (launch_trace_rays).
 template <bool ANY, bool COUNT, int MODE>
 __global__ void __launch_bounds__(kTraceBlock) k_trace_rays(SceneView sv, const solhip_ray *rays, solhip_hit *hits,
-                                                            uint32_t n, Counters *counters)
+                                                            uint32_t n, uint32_t lanes, Counters *counters)
 {
     extern __shared__ uint2 stack[];
     const uint32_t lb = xcd_logical_block(blockIdx.x, gridDim.x);
-    const uint32_t i = lb * kTraceBlock + threadIdx.x;
-    const bool active = i < n;
+    const uint32_t i = lb * lanes + threadIdx.x;
+    const bool active = threadIdx.x < lanes && i < n;
     TravCounts tc{0, 0, 0, false};
     if (active) {
         const float4 *rp = reinterpret_cast<const float4 *>(rays + i);
@@ -55,41 +95,97 @@ __global__ void __launch_bounds__(kTraceBlock) k_trace_rays(SceneView sv, const 
         trav_init<MODE, COUNT>(st, sv, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, 0xFFu, tc);
         while (!trav_step<ANY, COUNT, true, MODE>(st, sv, 0xFFu, stack + threadIdx.x, kTraceBlock, tc)) {
         }
-        const Hit h = trav_result(st);
-        solhip_hit o;
-        o.t = h.t;
-        o.u = h.u;
-        o.v = h.v;
-        o.inst = h.inst;
-        o.prim = h.prim;
-        o.geom = h.inst == SOLHIP_MISS ? SOLHIP_MISS : 0u;
-        hits[i] = o;
+        write_hit(hits + i, st);
     }
-    const uint64_t ov = __ballot(active && tc.overflow);
-    const uint32_t na = __popcll(__ballot(active));
-    if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&counters->rays, (unsigned long long)na);
-        if (ov) atomicAdd(&counters->overflow, (unsigned long long)__popcll(ov));
+    end_wave(counters, n, COUNT, tc, active);
+}
+
+// More rays than lanes: a persistent grid whose waves take new rays for their
+// idle lanes.  Rays are dealt in groups of 16: every 1024 consecutive rays go
+// to the next XCD (its L2 sees whole stretches of a coherent batch), whose waves
+// take groups in turn.  The deal is fixed, so no counter in memory is
+// needed and overlapping launches share nothing.
+template <bool ANY, bool COUNT, int MODE>
+__global__ void __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(SOLHIP_TRACE_WAVES)))
+k_trace_rays_persist(SceneView sv, const solhip_ray *rays, solhip_hit *hits, uint32_t n, Counters *counters)
+{
+    extern __shared__ uint2 stack[];
+    const uint32_t lane = threadIdx.x, xcd = blockIdx.x & 7u, waves = gridDim.x >> 3, wave = blockIdx.x >> 3;
+    TravCounts tc{0, 0, 0, false};
+    TravState st;
+    bool has = false, more = true;
+    uint32_t ray = 0, taken = 0;   // rays this wave has taken so far
+    while (true) {
+        const uint64_t idle = __ballot(!has);
+        if (more && __popcll(idle) >= SOLHIP_TRACE_REFILL) {
+            const uint32_t k = taken + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
+            taken += (uint32_t)__popcll(idle);
+            // the wave's k-th ray: group t of its XCD's
+            const uint64_t t = wave + (uint64_t)(k >> 4) * waves;
+            const uint64_t i = ((t >> 6) * 8u + xcd) * 1024u + (t & 63u) * 16u + (k & 15u);
+            const bool ok = !has && i < n;
+            if (ok) {
+                ray = (uint32_t)i;
+                const float4 *rp = reinterpret_cast<const float4 *>(rays + ray);
+                const float4 a = rp[0], b = rp[1];
+                trav_init<MODE, COUNT>(st, sv, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, 0xFFu, tc);
+                has = true;
+            }
+            // groups follow one another in ray order: past the end once, past it for good
+            more = __ballot(ok) == idle;
+        }
+        if (__ballot(has) == 0 && !more) break;
+        if (has && trav_step<ANY, COUNT, true, MODE>(st, sv, 0xFFu, stack + lane, kTraceBlock, tc)) {
+            write_hit(hits + ray, st);
+            has = false;
+        }
     }
-    if (COUNT) add_counts(counters, tc, active);
+    end_wave(counters, n, COUNT, tc, true);
 }
 
 int launch_trace_rays(hipStream_t s, const SceneView &sv, const solhip_ray *rays, solhip_hit *hits, uint32_t n,
-                      uint32_t flags, Counters *counters, Timer *timer)
+                      uint32_t flags, uint32_t ncu, Counters *counters, Timer *timer)
 {
     if (n == 0) return 0;
     if (timer) timer->begin(s, SOLHIP_KERNEL_TRACE_RAYS);
-    const dim3 grid((n + kTraceBlock - 1) / kTraceBlock), block(kTraceBlock);
     SceneView v = sv;
     v.stack_depth += 2;
+    const dim3 block(kTraceBlock);
     const size_t lds = (size_t)v.stack_depth * sizeof(uint2) * kTraceBlock;
     const bool any = flags & SOLHIP_TRACE_TERMINATE_ON_FIRST_HIT, count = flags & SOLHIP_TRACE_COUNT;
-    trav_dispatch(sv.mode, count, [&](auto mode, auto cnt) {
-        if (any)
-            hipLaunchKernelGGL((k_trace_rays<true, cnt.value, mode.value>), grid, block, lds, s, v, rays, hits, n, counters);
-        else
-            hipLaunchKernelGGL((k_trace_rays<false, cnt.value, mode.value>), grid, block, lds, s, v, rays, hits, n, counters);
-    });
+    const uint32_t simds = ncu * 4u;
+    const uint32_t resident = (simds * SOLHIP_TRACE_WAVES + 7u) & ~7u;
+    // Refill pays once there are more rays than lanes, except in trees of a few
+    // levels, whose rays end together anyway.  Microseconds, one ray per lane
+    // against refill: 2M rays on 131K triangles 321 / 202, on 500 instances 1692 / 1086,
+    // in the Cornell box (6 instances of 2 to 12 triangles, depth 4) 135 / 164;
+    // 0.4M rays on the triangles 98.7 / 97.5.  (2M with a counter atomic per wave,
+    // as before: 463, 2055 and 400.)
+    if (n > resident * 64u && sv.stack_depth > 4) {
+        trav_dispatch(sv.mode, count, [&](auto mode, auto cnt) {
+            if (any)
+                hipLaunchKernelGGL((k_trace_rays_persist<true, cnt.value, mode.value>), dim3(resident), block, lds, s, v,
+                                   rays, hits, n, counters);
+            else
+                hipLaunchKernelGGL((k_trace_rays_persist<false, cnt.value, mode.value>), dim3(resident), block, lds, s,
+                                   v, rays, hits, n, counters);
+        });
+    } else {
+        // lanes per wave: as many as leave a wave for every SIMD (64 rays on
+        // the instances 185 -> 81 us with one ray per wave; 60,001 on the triangles 98 us with
+        // full waves, 58 spread once over the SIMDs, 70 twice, 89 eight times)
+        uint32_t lanes = 64;
+        while (lanes > 1 && n / lanes < simds * SOLHIP_TRACE_SPREAD) lanes >>= 1;
+        const dim3 grid((n + lanes - 1) / lanes);
+        trav_dispatch(sv.mode, count, [&](auto mode, auto cnt) {
+            if (any)
+                hipLaunchKernelGGL((k_trace_rays<true, cnt.value, mode.value>), grid, block, lds, s, v, rays, hits, n,
+                                   lanes, counters);
+            else
+                hipLaunchKernelGGL((k_trace_rays<false, cnt.value, mode.value>), grid, block, lds, s, v, rays, hits, n,
+                                   lanes, counters);
+        });
+    }
     if (timer) timer->end(s, SOLHIP_KERNEL_TRACE_RAYS);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
