@@ -383,6 +383,7 @@ int trace_wavefront(Context *c, hipStream_t s, Program *p, Tlas *t, const ProgAr
     const uint64_t tiles = (uint64_t)((a.W + 7) / 8) * ((a.H + 7) / 8);
     if (tiles * 64 > 0xFFFFFFF0ull) return bad_arg("image too large");
     w.nslots = (uint32_t)(tiles * 64);
+    w.slice_pix = w.npix;
     w.block = p->spec.wf_block ? p->spec.wf_block : 64u;
     if ((uint64_t)(w.sv.stack_depth + 2) * sizeof(uint2) * w.block > 65536) {
         set_error("traversal stack of the wavefront kernels exceeds 64 KiB of LDS; use a smaller wf_block");
@@ -466,6 +467,13 @@ int trace_wavefront(Context *c, hipStream_t s, Program *p, Tlas *t, const ProgAr
             WfArgs ws = w;
             ws.slot_base = t0 * 64u;
             ws.nslots = (t1 - t0) * 64u;
+            // tiles t0 .. t1 in row-major order: their pixels inside the image
+            auto pixels_before = [&](uint32_t t) {   // pixels of tiles 0 .. t
+                const uint64_t tx = (w.W + 7) / 8, row = t / tx, col = t % tx;
+                const uint64_t top = std::min<uint64_t>(row * 8, w.H), high = std::min<uint64_t>(row * 8 + 8, w.H) - top;
+                return top * w.W + high * std::min<uint64_t>(col * 8, w.W);
+            };
+            ws.slice_pix = (uint32_t)(pixels_before(t1) - pixels_before(t0));
             const uint64_t qb = (uint64_t)w.S * ws.slot_base;   // the slice's part of the queues
             ws.q[0] = w.q[0] + qb;
             ws.q[1] = w.q[1] + qb;

@@ -138,6 +138,7 @@ struct WfArgs {
     float rmin, rmax;                 // ray range of every segment (pathtrace.rgen:35)
     uint32_t nslots;                  // slots of the first queue (8x8 pixel tiles * 64)
     uint32_t slot_base;               // first slot of this image slice (0: the whole image)
+    uint32_t slice_pix;               // pixels of this image slice (nslots without the tiles' overhang)
     // path state, S * npix each: (T, rng), (L, depth | count_emission << 16);
     // per-pixel sum of the finished samples: float (one stream per pixel) or
     // order-free fixed point (per-sample streams, accum.h)

@@ -189,7 +189,6 @@ __device__ __forceinline__ void srv_trace(const SrvArgs &A, const QRay *q, uint3
     extern __shared__ uint2 stack[];
     const uint32_t lane = threadIdx.x & 63u;
     TravCounts tc{0, 0, 0, false};
-    uint32_t rays = 0;
     TravState st;
     SceneView sv;
     bool has = false;
@@ -219,7 +218,6 @@ __device__ __forceinline__ void srv_trace(const SrvArgs &A, const QRay *q, uint3
         if (__ballot(has) == 0 && pf.exhausted) break;
         if (has && trav_step<ANY, false, SOLHIP_SRV_WINV>(st, sv, 0xFFu, stack + threadIdx.x, kSrvBlock, tc)) {
             const Hit h = trav_result(st);
-            ++rays;
             if (!ANY) {
                 QHit out;
                 out.t = h.t;
@@ -239,7 +237,7 @@ __device__ __forceinline__ void srv_trace(const SrvArgs &A, const QRay *q, uint3
             has = false;
         }
     }
-    count_rays<false>(A.counters + kernel, rays, tc);
+    count_known<false>(A.counters + kernel, cnt, tc);
 }
 
 __global__ void __launch_bounds__(kSrvBlock) SOLHIP_SRV_OCCUPANCY k_srv_extend(SrvArgs A,

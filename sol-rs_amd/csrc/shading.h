@@ -107,30 +107,47 @@ __device__ __forceinline__ void store_hit(solhip_hit *dst, const Hit &h)
     *dst = o;
 }
 
-// per-wave sums of rays (and fetches when COUNT), one atomic per wave
+// Counters at the end of a traversal kernel.  Atomics on one address are served
+// one after the other, about 15 ns each (70 per us): one per wave on the ray
+// counter bounded the AO primary kernel and added 60 us to the end of
+// every persistent launch.  A kernel whose ray count is known adds it once
+// (count_known); one that must count adds once per block of its waves' sums.
 template <bool COUNT>
-__device__ __forceinline__ void count_rays(Counters *c, uint32_t rays_this_lane, const TravCounts &tc)
+__device__ __forceinline__ void count_fetches(Counters *c, const TravCounts &tc)
 {
-    unsigned long long r = rays_this_lane;
-    unsigned long long nd = COUNT ? tc.nodes : 0, tr = COUNT ? tc.tris : 0, in = COUNT ? tc.insts : 0;
-    for (int off = 32; off > 0; off >>= 1) {
-        r += __shfl_xor(r, off);
-        if (COUNT) {
+    const uint64_t ov = __ballot(tc.overflow);
+    if (ov && (threadIdx.x & 63) == 0) atomicAdd(&c->overflow, (unsigned long long)__popcll(ov));
+    if (COUNT) {
+        unsigned long long nd = tc.nodes, tr = tc.tris, in = tc.insts;
+        for (int off = 32; off > 0; off >>= 1) {
             nd += __shfl_xor(nd, off);
             tr += __shfl_xor(tr, off);
             in += __shfl_xor(in, off);
         }
-    }
-    const uint64_t ov = __ballot(tc.overflow);
-    if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&c->rays, r);
-        if (ov) atomicAdd(&c->overflow, (unsigned long long)__popcll(ov));
-        if (COUNT) {
+        if ((threadIdx.x & 63) == 0) {
             atomicAdd(&c->nodes, nd);
             atomicAdd(&c->tris, tr);
             atomicAdd(&c->insts, in);
         }
     }
+}
+
+// the launch traces `rays` rays in all
+template <bool COUNT>
+__device__ __forceinline__ void count_known(Counters *c, unsigned long long rays, const TravCounts &tc)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&c->rays, rays);
+    count_fetches<COUNT>(c, tc);
+}
+
+// per-lane ray counts, summed over the wave
+template <bool COUNT>
+__device__ __forceinline__ void count_rays(Counters *c, uint32_t rays_this_lane, const TravCounts &tc)
+{
+    unsigned long long r = rays_this_lane;
+    for (int off = 32; off > 0; off >>= 1) r += __shfl_xor(r, off);
+    if ((threadIdx.x & 63) == 0) atomicAdd(&c->rays, r);
+    count_fetches<COUNT>(c, tc);
 }
 
 __device__ __forceinline__ float length3(V3 a) { return sqrtf(dot(a, a)); }

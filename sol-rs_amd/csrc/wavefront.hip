@@ -207,13 +207,13 @@ __device__ __forceinline__ void queue_result(const WfArgs &A, uint32_t i, uint32
 // while the rest of the wave is still traversing.  sv.stack_depth includes
 // the two extra entries the step traversal may hold.
 template <bool ANY, bool COUNT, int MODE>
-__device__ __forceinline__ void trace_queue(const WfArgs &A, const QRay *q, uint32_t cnt, uint32_t *heads, int kernel)
+__device__ __forceinline__ void trace_queue(const WfArgs &A, const QRay *q, uint32_t cnt, unsigned long long rays,
+                                            uint32_t *heads, int kernel)
 {
     extern __shared__ uint2 stack[];
     const uint32_t lane = threadIdx.x & 63u;
     const float tmin = ray_tmin(A);
     TravCounts tc{0, 0, 0, false};
-    uint32_t rays = 0;
     TravState st;
     bool has = false;
     uint32_t idx = 0, path = 0;
@@ -250,11 +250,10 @@ __device__ __forceinline__ void trace_queue(const WfArgs &A, const QRay *q, uint
         if (__ballot(has) == 0 && pf.exhausted) break;
         if (has && trav_step<ANY, COUNT, SOLHIP_WF_WINV, MODE>(st, A.sv, 0xFFu, stack + threadIdx.x, A.block, tc)) {
             queue_result<ANY>(A, idx, path, trav_result(st));
-            ++rays;
             has = false;
         }
     }
-    count_rays<COUNT>(A.counters + kernel, rays, tc);
+    count_known<COUNT>(A.counters + kernel, rays, tc);
 }
 
 template <bool COUNT, int MODE>
@@ -265,15 +264,19 @@ __global__ void SOLHIP_WF_OCCUPANCY k_pt_extend(WfArgs A, uint32_t b)
         A.counts[(b + 1) & 1] = 0;
         A.counts[2] = 0;
     }
-    trace_queue<false, COUNT, MODE>(A, A.q[b & 1], A.counts[b & 1], A.heads + 2 * b * kWfParts * kHeadStride,
-                              SOLHIP_KERNEL_PT_EXTEND);
+    // the first queue holds whole tiles: sample-in-pass * nslots + slot
+    const uint32_t cnt = A.counts[b & 1];
+    const unsigned long long rays = b ? cnt : (unsigned long long)(cnt / A.nslots) * A.slice_pix;
+    trace_queue<false, COUNT, MODE>(A, A.q[b & 1], cnt, rays, A.heads + 2 * b * kWfParts * kHeadStride,
+                                    SOLHIP_KERNEL_PT_EXTEND);
 }
 
 template <bool COUNT, int MODE>
 __global__ void SOLHIP_WF_OCCUPANCY k_pt_shadow(WfArgs A, uint32_t b)
 {
-    trace_queue<true, COUNT, MODE>(A, A.sq, A.counts[2], A.heads + (2 * b + 1) * kWfParts * kHeadStride,
-                             SOLHIP_KERNEL_PT_SHADOW);
+    const uint32_t cnt = A.counts[2];
+    trace_queue<true, COUNT, MODE>(A, A.sq, cnt, cnt, A.heads + (2 * b + 1) * kWfParts * kHeadStride,
+                                   SOLHIP_KERNEL_PT_SHADOW);
 }
 
 // The shade kernel runs blocks of WAVES waves and appends to its queues once
