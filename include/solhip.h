@@ -191,8 +191,8 @@ typedef struct {
     /* SOLHIP_PROG_PATHTRACE: the image's 8x8 tiles split into this many
      * contiguous slices whose passes run on their own streams at the same
      * time, so one slice's slowest rays overlap the others' work; pixels are
-     * independent, so the image does not depend on it.  0 = default (4
-     * with sample_streams, else 1); always 1 with SOLHIP_PROFILE_TIME or nrc. */
+     * independent, so the image does not depend on it.  0 = default (2
+     * with sample_streams and 2 M paths per pass or more, else 1); always 1 with SOLHIP_PROFILE_TIME or nrc. */
     uint32_t wf_slices;
     /* SOLHIP_PROG_PATHTRACE random streams.  0: one stream per pixel runs
      * through all samples of the frame, as in pathtrace.rgen:47 (samples are

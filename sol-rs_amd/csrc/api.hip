@@ -353,15 +353,26 @@ int trace_nrc(Context *c, hipStream_t s, Program *p, Tlas *t, WfArgs &w, Timer *
     return rc;
 }
 
-// SOLHIP_PROG_PATHTRACE: buffers, emitter table, the wavefront passes
 // image slices of a frame when the spec leaves it open: with a stream per
-// sample, passes are large and slices overlap one another's slowest rays;
-// with one stream per pixel, passes are one sample each and slices only add
-// launches
-constexpr uint32_t kDefaultSlicesStreams = 4;
+// sample and enough paths for both to fill the GPU, two slices overlap one
+// another's slowest rays; more only add launches (1, 2, 3, 4, 6 slices: 10,000
+// instances, 33M paths 58.1, 55.8, 59.7, 58.3, 63.2 ms; Cornell box, 4.2M 3.87,
+// 3.76, 4.05, 4.38, 5.5; 51K 0.50, 0.65, 0.73, 0.82, 1.20).  With one stream
+// per pixel, passes are one sample each
+constexpr uint32_t kDefaultSlicesStreams = 2;
+constexpr uint64_t kSlicePaths = 1ull << 20;   // paths per default slice, at least
+// a queue is finished path by path below this many rays per lane of the
+// finishing kernel: many transformed instances make long and uneven rays, whose
+// tails are worth more than the wider kernels' occupancy.  Milliseconds at 0 (never), 2, 4, 8:
+// 10,000 instances, 1080p, 16 streams 62.2, 60.1, 58.8, 58.5; 1 sample 10.5,
+// 7.8, 7.8, 6.4; 2,000 instances, 720p, 4 samples in sequence 19.4, 13.8, 12.6, 11.5; the
+// Cornell box 4.33, 4.35, 4.93, 5.14, 16 samples in sequence 13.3, 9.0, 9.0, 9.0;
+// a terrain 4.06, 4.10, 4.25, 4.29
+constexpr uint32_t kFinishGeneral = 8, kFinishOther = 2;
 // paths in flight per pass that the default samples-per-pass aims for
 constexpr uint64_t kPathsInFlight = 64ull << 20;
 
+// SOLHIP_PROG_PATHTRACE: buffers, emitter table, the wavefront passes
 int trace_wavefront(Context *c, hipStream_t s, Program *p, Tlas *t, const ProgArgs &a)
 {
     WfArgs w;
@@ -404,6 +415,12 @@ int trace_wavefront(Context *c, hipStream_t s, Program *p, Tlas *t, const ProgAr
     w.S = S;
     w.shade_blocks = (uint32_t)std::min<uint64_t>(((uint64_t)S * w.nslots + w.block - 1) / w.block,
                                                   (uint64_t)c->ncu * 2048 / w.block);
+    // small queues are finished path by path; not with the radiance cache
+    // (queries and records hang on the bounces) nor while launches are timed
+    if (!p->spec.nrc && !c->timer_or_null()) {
+        w.finish_blocks = c->ncu * wf_finish_lanes_per_cu() / 64u;
+        w.finish_at = w.finish_blocks * 64u * (w.sv.mode == kTravGeneral ? kFinishGeneral : kFinishOther);
+    }
     w.counters = c->counters;
     w.count = a.count;
     const uint64_t npix = (uint64_t)a.W * a.H, ns = (uint64_t)w.S * w.nslots, np = (uint64_t)w.S * npix;
@@ -411,7 +428,8 @@ int trace_wavefront(Context *c, hipStream_t s, Program *p, Tlas *t, const ProgAr
     // image slices: profiling times every launch on one stream, and the
     // radiance cache works on the whole image between passes
     const uint32_t tiles32 = (uint32_t)tiles;
-    uint32_t nslices = p->spec.wf_slices ? p->spec.wf_slices : (p->spec.sample_streams ? kDefaultSlicesStreams : 1u);
+    uint32_t nslices = p->spec.wf_slices;
+    if (nslices == 0) nslices = p->spec.sample_streams && ns >= kDefaultSlicesStreams * kSlicePaths ? kDefaultSlicesStreams : 1u;
     if (p->spec.nrc || c->timer_or_null()) nslices = 1;
     nslices = std::max(1u, std::min(nslices, tiles32));
     if (p->st0.reserve(np * 16) || p->st1.reserve(np * 16) || p->psum.reserve(npix * 16) ||

@@ -412,7 +412,8 @@ __global__ void __launch_bounds__(kCollapseBlock) k_collapse(CollapseDev A)
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, c = lane & 7u, g0 = lane & 56u;
     const uint32_t n = A.n, nbin = 2u * n - 1u;
     uint32_t *levels = A.counters + kCntLevels;
-    const uint32_t begin = levels[A.level], end = levels[A.level + 1];
+    // (an allocation beyond n nodes is refused below and fails the build)
+    const uint32_t begin = levels[A.level], end = min(levels[A.level + 1], n);
     // bits of a ballot that belong to this lane's group
     auto group_bits = [&](bool p) -> uint32_t { return (uint32_t)(__ballot(p) >> g0) & 0xFFu; };
     for (uint32_t base = begin + blockIdx.x * kCollapseNodes; base < end; base += gridDim.x * kCollapseNodes) {

@@ -155,6 +155,8 @@ struct WfArgs {
     NrcArgs nrc;
     uint32_t block;                   // threads per block
     uint32_t persist_blocks;          // grid of the extend / shadow kernels
+    uint32_t finish_at;               // queues of at most this many rays are finished by k_pt_finish (0: never)
+    uint32_t finish_blocks;           // its grid (blocks of 64)
     uint32_t shade_blocks;            // grid of the shade kernel
     Counters *counters;
     bool count;
@@ -197,6 +199,8 @@ int launch_pathtrace_passes(hipStream_t s, const WfArgs &a, Timer *timer, const 
 int launch_pathtrace_finalize(hipStream_t s, const WfArgs &a, Timer *timer);
 // threads per CU that the traversal kernels' register budget keeps resident
 uint32_t wf_threads_per_cu();
+// resident lanes of the kernel that finishes small queues, per CU
+uint32_t wf_finish_lanes_per_cu();
 // words of WfArgs::heads per logical fetch head (its partitions' heads)
 uint32_t wf_head_words();
 // writes the frame constants through a kernel argument (no host buffer to keep alive)

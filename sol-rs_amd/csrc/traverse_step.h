@@ -48,7 +48,11 @@ struct TravState {
     uint32_t tg_base, tg_mask, tg_valid;   // leaf group: first record, primitives left, the node's leaf_mask
     int sp, base;              // stack height; height at BLAS entry
     Hit best;
+    bool any;                  // first hit ends the ray (with kAnyOfRay only)
 };
+
+// trav_step's ANY: closest hit, first hit, or as the ray says (TravState::any)
+constexpr int kClosest = 0, kAny = 1, kAnyOfRay = 2;
 
 constexpr uint32_t kLeafGroupTag = 0x80000000u;
 
@@ -153,7 +157,7 @@ SOLHIP_HD Hit trav_result(const TravState &s)
 // with it; the path tracer's extension kernel, whose rays leave a BLAS 3.9
 // times on average, 6 % faster once its register budget holds the three
 // registers (at 5 waves per SIMD they spilled and it ran 1 % slower).
-template <bool ANY, bool COUNT, bool WINV = true, int MODE = kTravGeneral>
+template <int ANY, bool COUNT, bool WINV = true, int MODE = kTravGeneral>
 SOLHIP_HD bool trav_step(TravState &s, const SceneView &sv, uint32_t cull, uint2 *lds, int stride, TravCounts &cnt)
 {
     const int depth = (int)sv.stack_depth;
@@ -174,7 +178,7 @@ SOLHIP_HD bool trav_step(TravState &s, const SceneView &sv, uint32_t cull, uint2
             s.best.v = v;
             s.best.inst = s.inst;
             s.best.prim = c.y;
-            if (ANY) return true;
+            if (ANY == kAny || (ANY == kAnyOfRay && s.any)) return true;
         }
     }
     // 2. nothing left of the last node: the next stack entry (pushed groups are

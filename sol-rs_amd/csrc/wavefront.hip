@@ -266,6 +266,7 @@ __global__ void SOLHIP_WF_OCCUPANCY k_pt_extend(WfArgs A, uint32_t b)
     }
     // the first queue holds whole tiles: sample-in-pass * nslots + slot
     const uint32_t cnt = A.counts[b & 1];
+    if (cnt <= A.finish_at) return;   // k_pt_finish has traced it
     const unsigned long long rays = b ? cnt : (unsigned long long)(cnt / A.nslots) * A.slice_pix;
     trace_queue<false, COUNT, MODE>(A, A.q[b & 1], cnt, rays, A.heads + 2 * b * kWfParts * kHeadStride,
                                     SOLHIP_KERNEL_PT_EXTEND);
@@ -275,8 +276,148 @@ template <bool COUNT, int MODE>
 __global__ void SOLHIP_WF_OCCUPANCY k_pt_shadow(WfArgs A, uint32_t b)
 {
     const uint32_t cnt = A.counts[2];
+    if (cnt == 0) return;
     trace_queue<true, COUNT, MODE>(A, A.sq, cnt, cnt, A.heads + (2 * b + 1) * kWfParts * kHeadStride,
                                    SOLHIP_KERNEL_PT_SHADOW);
+}
+
+__device__ __forceinline__ ShadeParams shade_params(const WfArgs &A)
+{
+    ShadeParams P;
+    P.tb = A.tb;
+    P.enable_sky = A.enable_sky;
+    P.max_depth = A.max_depth;
+    P.rr_start = A.rr_start;
+    P.lights = A.lights;
+    P.nlights = A.nlights;
+    P.total = A.nlights ? A.lights[A.nlights - 1].cdf : 0.0f;
+    P.nee = A.nee && A.nlights > 0 && P.total > 0.0f;
+    P.rmax = A.rmax;
+    return P;
+}
+
+// A small queue's paths to their ends, in one launch: a lane keeps its path
+// (traversal, throughput, radiance) from ray to ray, shades with at least
+// SOLHIP_FINISH_SHADE lanes of its wave, and takes the queue's next path when
+// its own ends.  Bounce by bounce, a queue smaller than the GPU costs a launch
+// of each kernel as long as its slowest ray (the 10,000-instance scene: 1 to 1.8
+// ms for each of the last five bounces), here the slowest path's rays once.  Per path the order
+// of all additions and random draws is the passes' (times at kFinishGeneral).
+#ifndef SOLHIP_FINISH_SHADE
+#define SOLHIP_FINISH_SHADE 16
+#endif
+#ifndef SOLHIP_FINISH_WAVES
+#define SOLHIP_FINISH_WAVES 3
+#endif
+template <bool COUNT, int MODE>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(SOLHIP_FINISH_WAVES)))
+k_pt_finish(WfArgs A, uint32_t b)
+{
+    extern __shared__ uint2 stack[];
+    const uint32_t cnt = A.counts[b & 1];
+    if (cnt == 0 || cnt > A.finish_at) return;
+    const uint32_t lane = threadIdx.x;
+    const ShadeParams P = shade_params(A);
+    const float tmin = ray_tmin(A);
+    const QRay *q = A.q[b & 1];
+    enum : uint32_t { kIdle, kTrace, kDone };
+    uint32_t state = kIdle, path = 0, rays = 0, shadows = 0;
+    TravCounts tc{0, 0, 0, false};
+    TravState st;
+    st.any = false;
+    float4 s0, s1;
+    // while a shadow ray is traced: its contribution, and the path's next direction
+    V3 sc, nd;
+    bool cont = false;
+    PartFetch pf;
+    pf.init(A.heads + 2 * b * kWfParts * kHeadStride, kWfParts, cnt);
+    while (true) {
+        const uint64_t waiting = __ballot(state == kDone || (state == kIdle && !pf.exhausted));
+        const bool tracing = __ballot(state == kTrace) != 0;
+        if (!tracing && !waiting) break;
+        if (!tracing || __popcll(waiting) >= SOLHIP_FINISH_SHADE) {
+            bool go = false, ended = false;
+            V3 o, d;
+            float tmax = A.rmax;
+            if (state == kDone) {
+                const Hit h = trav_result(st);
+                if (st.any) {
+                    // the shadow ray's answer, then the next ray from the same point
+                    if (h.inst == SOLHIP_MISS) {
+                        s1.x = s1.x + sc.x;
+                        s1.y = s1.y + sc.y;
+                        s1.z = s1.z + sc.z;
+                    }
+                    o = st.wo;
+                    d = nd;
+                    st.any = false;
+                    go = cont;
+                    ended = !cont;
+                } else {
+                    QRay r;
+                    r.dx = st.wd.x;
+                    r.dy = st.wd.y;
+                    r.dz = st.wd.z;
+                    QHit qh;
+                    qh.t = h.t;
+                    qh.u = h.u;
+                    qh.v = h.v;
+                    qh.inst = h.inst;
+                    qh.prim = h.prim;
+                    ShadeOut so;
+                    shade_vertex(P, path, r, qh, s0, s1, so);
+                    if (so.shadow) {
+                        cont = so.cont;
+                        nd = v3(so.nr.dx, so.nr.dy, so.nr.dz);
+                        sc = v3(so.sc.x, so.sc.y, so.sc.z);
+                        o = v3(so.sr.ox, so.sr.oy, so.sr.oz);
+                        d = v3(so.sr.dx, so.sr.dy, so.sr.dz);
+                        tmax = so.sr.tmax;
+                        st.any = true;
+                        go = true;
+                    } else {
+                        o = v3(so.nr.ox, so.nr.oy, so.nr.oz);
+                        d = v3(so.nr.dx, so.nr.dy, so.nr.dz);
+                        go = so.cont;
+                        ended = !so.cont;
+                    }
+                }
+                if (ended) {
+                    A.st0[path] = s0;
+                    A.st1[path] = s1;
+                    state = kIdle;
+                }
+            }
+            const uint64_t idle = __ballot(state == kIdle);
+            if (!pf.exhausted && idle) {
+                uint32_t end;
+                const uint32_t base = pf.claim((uint32_t)__popcll(idle), end);
+                const uint32_t my = base + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
+                if (state == kIdle && my < end) {
+                    const QRay r = q[my];
+                    if (r.path != kNoPath) {
+                        path = r.path;
+                        s0 = A.st0[path];
+                        s1 = A.st1[path];
+                        o = v3(r.ox, r.oy, r.oz);
+                        d = v3(r.dx, r.dy, r.dz);
+                        go = true;
+                    }
+                }
+            }
+            if (go) {
+                if (st.any) ++shadows;
+                else ++rays;
+                trav_init<MODE, COUNT>(st, A.sv, o, d, tmin, tmax, 0xFFu, tc);
+                state = kTrace;
+            }
+        }
+        if (state == kTrace && trav_step<kAnyOfRay, COUNT, true, MODE>(st, A.sv, 0xFFu, stack + lane, 64, tc))
+            state = kDone;
+    }
+    for (int off = 32; off > 0; off >>= 1) shadows += __shfl_xor(shadows, off);
+    if (lane == 0 && shadows) atomicAdd(&A.counters[SOLHIP_KERNEL_PT_SHADOW].rays, (unsigned long long)shadows);
+    count_rays<COUNT>(A.counters + SOLHIP_KERNEL_PT_EXTEND, rays, tc);
 }
 
 // The shade kernel runs blocks of WAVES waves and appends to its queues once
@@ -302,20 +443,12 @@ __global__ void __launch_bounds__(64 * WAVES) SOLHIP_WF_SHADE_OCCUPANCY k_pt_sha
 {
     __shared__ uint32_t lds[WAVES + 1];
     const uint32_t cnt = A.counts[b & 1];
+    if (cnt <= A.finish_at) return;   // k_pt_finish has shaded it
     const QRay *qin = A.q[b & 1];
     QRay *qout = A.q[(b + 1) & 1];
     uint32_t *cout = A.counts + ((b + 1) & 1);
     const uint32_t nthreads = gridDim.x * blockDim.x;
-    ShadeParams P;
-    P.tb = A.tb;
-    P.enable_sky = A.enable_sky;
-    P.max_depth = A.max_depth;
-    P.rr_start = A.rr_start;
-    P.lights = A.lights;
-    P.nlights = A.nlights;
-    P.total = A.nlights ? A.lights[A.nlights - 1].cdf : 0.0f;
-    P.nee = A.nee && A.nlights > 0 && P.total > 0.0f;
-    P.rmax = A.rmax;
+    const ShadeParams P = shade_params(A);
     for (uint32_t base = blockIdx.x * blockDim.x; base < cnt; base += nthreads) {
         const uint32_t i = base + threadIdx.x;
         ShadeOut o;
@@ -428,16 +561,7 @@ __global__ void k_pt_shade_nrc(WfArgs A, uint32_t b)
     uint32_t *cout = A.counts + ((b + 1) & 1);
     const NrcArgs &N = A.nrc;
     const uint32_t lane = threadIdx.x & 63u, nthreads = gridDim.x * blockDim.x;
-    ShadeParams P;
-    P.tb = A.tb;
-    P.enable_sky = A.enable_sky;
-    P.max_depth = A.max_depth;
-    P.rr_start = A.rr_start;
-    P.lights = A.lights;
-    P.nlights = A.nlights;
-    P.total = A.nlights ? A.lights[A.nlights - 1].cdf : 0.0f;
-    P.nee = A.nee && A.nlights > 0 && P.total > 0.0f;
-    P.rmax = A.rmax;
+    const ShadeParams P = shade_params(A);
     for (uint32_t base = blockIdx.x * blockDim.x + (threadIdx.x & ~63u); base < cnt; base += nthreads) {
         const uint32_t i = base + lane;
         ShadeOut o;
@@ -690,6 +814,8 @@ uint32_t wf_threads_per_cu() { return 4u * SOLHIP_WF_WAVES * 64u; }
 
 uint32_t wf_head_words() { return kWfParts * kHeadStride; }
 
+uint32_t wf_finish_lanes_per_cu() { return 4u * SOLHIP_FINISH_WAVES * 64u; }
+
 int launch_lights_count(hipStream_t s, const DevTables &tb, const uint32_t *inst_tris, uint32_t n_inst,
                         uint32_t *offsets, Timer *timer)
 {
@@ -767,6 +893,11 @@ int launch_pathtrace_passes(hipStream_t s, const WfArgs &a0, Timer *timer, const
             hipLaunchKernelGGL(k_nrc_select, dim3(a.shade_blocks), dim3(blk), 0, s, a, pass);
         }
         for (uint32_t b = 0; b <= a.max_depth; ++b) {
+            if (a.finish_at)
+                trav_dispatch(a.sv.mode, a.count, [&](auto mode, auto count) {
+                    hipLaunchKernelGGL((k_pt_finish<count.value, mode.value>), dim3(a.finish_blocks), dim3(64),
+                                       (size_t)a.sv.stack_depth * sizeof(uint2) * 64, s, a, b);
+                });
             timed(SOLHIP_KERNEL_PT_EXTEND, [&] {
                 trav_dispatch(a.sv.mode, a.count, [&](auto mode, auto count) {
                     hipLaunchKernelGGL((k_pt_extend<count.value, mode.value>), dim3(a.persist_blocks), dim3(blk), lds,
