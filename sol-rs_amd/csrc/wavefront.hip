@@ -421,11 +421,11 @@ k_pt_finish(WfArgs A, uint32_t b)
 }
 
 // The shade kernel runs blocks of WAVES waves and appends to its queues once
-// per block.  With shadow rays (two appends per ray) 8-wave blocks: the
-// per-wave atomics on the two counters limited the Cornell box (3599 ->
-// 4223 Mrays/s); without them 2-wave blocks: larger blocks wait longer at the
-// append barriers on scattered scenes (10k instances: 1259 with 1 wave, 1277
-// with 2, 1225 with 8).
+// per block: atomics on a queue's counter are served one after the other, about 15 ns
+// each.  10,000 instances, 33M paths, one slice: 13.9, 8.0, 5.3, 4.9, 5.1 ms
+// of shading a frame with 1, 2, 4, 8, 16 waves, but larger blocks wait longer
+// at the append barriers where slices share the GPU (frame 61.7, 56.2, 54.3, 55.6,
+// 56.4 ms): 4 waves, and 8 with shadow rays (two appends per ray; Cornell box).
 // waves per SIMD the shade kernel is compiled for (0: the compiler's choice,
 // 115 VGPRs and 4 waves; 5 fits in 90 VGPRs without spills: Cornell box
 // 4176 -> 4287 Mrays/s, 10k instances 1252 -> 1258; 6 spills and is slower)
@@ -907,7 +907,7 @@ int launch_pathtrace_passes(hipStream_t s, const WfArgs &a0, Timer *timer, const
             timed(SOLHIP_KERNEL_PT_SHADE, [&] {
                 if (nrc) hipLaunchKernelGGL(k_pt_shade_nrc, dim3(a.shade_blocks), dim3(blk), 0, s, a, b);
                 else if (shadows) hipLaunchKernelGGL(k_pt_shade<8>, dim3(shade_grid(8)), dim3(512), 0, s, a, b);
-                else hipLaunchKernelGGL(k_pt_shade<2>, dim3(shade_grid(2)), dim3(128), 0, s, a, b);
+                else hipLaunchKernelGGL(k_pt_shade<4>, dim3(shade_grid(4)), dim3(256), 0, s, a, b);
             });
             if (nrc && b == 1 && hook) {
                 int rc = hook->after_query_shade(hook->user, s);
