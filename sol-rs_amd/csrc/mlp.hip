@@ -13,10 +13,15 @@
 //   A (16 x 32): row r, k = 8q .. 8q+7      B (32 x 16): col r, k = 8q .. 8q+7
 //   D (16 x 16): col r, rows 4q .. 4q+3 (registers 0..3)
 //
-// Kernels: forward (optionally saving every layer's input transposed,
-// feature-major, for the weight gradients), backward-data (loss gradient,
-// ReLU masks, dZ_l per layer, transposed), backward-weights (X_l^T dZ_l over
-// sample chunks into per-chunk partials), reduce + Adam.  Loss: relative L2,
+// Layers are computed transposed, H^T = W^T X^T: A is the weights, B a band of
+// 16 samples.  D then holds 4 features of a sample per lane and tile, and two
+// lane swaps per register pair make it the next layer's B (next_operand), so
+// activations pass from layer to layer in registers.  Products and their order
+// in k are those of X W.
+//
+// Kernels: forward (weights in registers); training (k_mlp_train: forward, loss
+// gradient, ReLU masks and weight gradients of a tile of 64 samples in one kernel,
+// per-workgroup partials); reduce + Adam.  Loss: relative L2,
 // sum_c (p_c - t_c)^2 / (sg(p_c)^2 + 0.01) / N (Mueller et al. 2021).
 #include <hip/hip_runtime.h>
 
@@ -37,11 +42,9 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kOutPad = 16;          // output layer columns in the MFMA tile
 constexpr int kOut = 3;
 constexpr int kHidden = 4;           // layers 0..3 are 64x64 + ReLU, layer 4 is 64x16 linear
 constexpr uint32_t kP = 4 * 4096 + 64 * 16;
-constexpr uint32_t kChunk = 1024;    // samples per backward-weights partial
 constexpr int kMlpBlock = 256;       // 4 waves
 
 __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c)
@@ -49,12 +52,8 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c)
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ bf16x8 zero8()
 {
@@ -63,227 +62,306 @@ __device__ __forceinline__ bf16x8 zero8()
     return z;
 }
 
+constexpr uint32_t kWeights = 4 * 4096 + 16 * 64;   // of either BF16 layout
+
 __device__ __forceinline__ uint32_t wt_offset(int l, int n) { return (uint32_t)l * 4096u + (uint32_t)n * 64u; }
+
+// tiles 2h and 2h + 1 of a layer's output (BF16 x 4 each: features 16 nt + 4q ..
+// 4q+3 of sample r) as half h of the next layer's B operand (features 32h + 8q
+// .. 8q+7).  With the tiles' rows of 16 lanes a0 a1 a2 a3 and b0 b1 b2 b3, the
+// operand's first half is a0 a2 b0 b2 and its second a1 a3 b1 b3: swap a's upper 32
+// lanes with b's lower, then a's odd rows with b's even ones.
+__device__ __forceinline__ bf16x8 next_operand(bf16x4 ta, bf16x4 tb)
+{
+    const u32x2 a = __builtin_bit_cast(u32x2, ta), b = __builtin_bit_cast(u32x2, tb);
+    u32x4 o;
+    for (int k = 0; k < 2; ++k) {
+        const auto s = __builtin_amdgcn_permlane32_swap(a[k], b[k], false, false);
+        const auto t = __builtin_amdgcn_permlane16_swap(s[0], s[1], false, false);
+        o[k] = t[0];
+        o[2 + k] = t[1];
+    }
+    return __builtin_bit_cast(bf16x8, o);
+}
+
+// ReLU and rounding of an accumulator tile
+__device__ __forceinline__ bf16x4 relu4(f32x4 acc)
+{
+    bf16x4 v;
+    for (int i = 0; i < 4; ++i) v[i] = (bf16)fmaxf(acc[i], 0.0f);
+    return v;
+}
 
 struct FwdArgs {
     const bf16 *x;          // N x 64
-    uint32_t n, npad;
+    uint32_t n;
     const uint32_t *n_dev;  // if set, N is read from device memory (at most n)
     const bf16 *wt;         // forward layout
-    float4 *y;              // N outputs (x, y, z, 0), or null
-    bf16 *actT;             // 5 x [64][npad] layer inputs, feature-major, or null
+    float4 *y;              // N outputs (x, y, z written), or null
     // cache-query epilogue: st1[rec.path].xyz += rec.T * max(y, 0)
     const CacheQuery *qrec;
     float4 *st1;
 };
 
-// one wave = 16 rows per band; weights staged in LDS (34 KB)
+// Forward: each wave keeps all weights in registers (34 operands, 136 VGPRs) and
+// streams bands of 16 rows, kFwdBands at a time, the next ones' loads issued
+// before the current ones' layers.  Bound by the 140 B per row it moves.
+// 1M rows 139 -> 60 us, 30,000 20 -> 5.7 (weights read from LDS for every tile and
+// activations through it before).
+constexpr int kFwdBands = 2;
+
 __global__ void __launch_bounds__(kMlpBlock) k_mlp_fwd(FwdArgs A)
 {
-    __shared__ bf16 wl[4 * 4096 + 16 * 64];
-    __shared__ bf16 hbuf[kMlpBlock / 64][16 * 64];
-    for (uint32_t i = threadIdx.x; i < (4 * 4096 + 16 * 64) / 8; i += kMlpBlock)
+    __shared__ bf16 wl[kWeights];
+    for (uint32_t i = threadIdx.x; i < kWeights / 8; i += kMlpBlock)
         reinterpret_cast<bf16x8 *>(wl)[i] = reinterpret_cast<const bf16x8 *>(A.wt)[i];
     __syncthreads();
     const uint32_t lane = threadIdx.x & 63u, r = lane & 15u, q = lane >> 4, wv = threadIdx.x >> 6;
-    bf16 *H = hbuf[wv];
+    bf16x8 w[kHidden][4][2], wo[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int l = 0; l < kHidden; ++l)
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt)
+                w[l][nt][h] = *reinterpret_cast<const bf16x8 *>(wl + wt_offset(l, nt * 16 + (int)r) + 32 * h + 8 * q);
+        wo[h] = *reinterpret_cast<const bf16x8 *>(wl + 4 * 4096 + r * 64 + 32 * h + 8 * q);
+    }
     const uint32_t n = A.n_dev ? min(*A.n_dev, A.n) : A.n;
-    const uint32_t nbands = A.n_dev ? (n + 15) / 16 : A.npad / 16, waves = gridDim.x * (kMlpBlock / 64);
-    for (uint32_t band = blockIdx.x * (kMlpBlock / 64) + wv; band < nbands; band += waves) {
-        const uint32_t row0 = band * 16;
-        const bool rv = row0 + r < n;
-        bf16x8 a0 = rv ? *reinterpret_cast<const bf16x8 *>(A.x + (uint64_t)(row0 + r) * 64 + 8 * q) : zero8();
-        bf16x8 a1 = rv ? *reinterpret_cast<const bf16x8 *>(A.x + (uint64_t)(row0 + r) * 64 + 32 + 8 * q) : zero8();
-        if (A.actT) {
-            // the input, feature-major, through LDS
-            *reinterpret_cast<bf16x8 *>(H + r * 64 + 8 * q) = a0;
-            *reinterpret_cast<bf16x8 *>(H + r * 64 + 32 + 8 * q) = a1;
-            wave_sync();
-            for (int nt = 0; nt < 4; ++nt) {
-                const uint32_t c = nt * 16 + r;
-                bf16x4 v;
-                for (int i = 0; i < 4; ++i) v[i] = H[(4 * q + i) * 64 + c];
-                *reinterpret_cast<bf16x4 *>(A.actT + (uint64_t)c * A.npad + row0 + 4 * q) = v;
-            }
-            wave_sync();
-        }
+    const uint32_t bands = (n + 15) / 16, stride = gridDim.x * (kMlpBlock / 64) * kFwdBands;
+    auto load = [&](uint32_t band, bf16x8 x[2]) {
+        const uint32_t row = band * 16 + r;
+        const bool in = row < n;
+        const bf16 *p = A.x + (uint64_t)(in ? row : 0u) * 64 + 8 * q;
+        x[0] = in ? *reinterpret_cast<const bf16x8 *>(p) : zero8();
+        x[1] = in ? *reinterpret_cast<const bf16x8 *>(p + 32) : zero8();
+    };
+    uint32_t band = (blockIdx.x * (kMlpBlock / 64) + wv) * kFwdBands;
+    bf16x8 x[kFwdBands][2];
+    for (int k = 0; k < kFwdBands; ++k) load(min(band + k, bands), x[k]);
+    for (; band < bands; band += stride) {
+        bf16x8 nx[kFwdBands][2];
+        for (int k = 0; k < kFwdBands; ++k) load(min(band + stride + k, bands), nx[k]);
+#pragma unroll
         for (int l = 0; l < kHidden; ++l) {
-            for (int nt = 0; nt < 4; ++nt) {
-                const bf16 *wb = wl + wt_offset(l, nt * 16 + (int)r);
-                f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-                acc = mfma(a0, *reinterpret_cast<const bf16x8 *>(wb + 8 * q), acc);
-                acc = mfma(a1, *reinterpret_cast<const bf16x8 *>(wb + 32 + 8 * q), acc);
-                const uint32_t c = nt * 16 + r;
-                bf16x4 v;
-                for (int i = 0; i < 4; ++i) {
-                    const bf16 h = (bf16)fmaxf(acc[i], 0.0f);
-                    v[i] = h;
-                    H[(4 * q + i) * 64 + c] = h;
+#pragma unroll
+            for (int k = 0; k < kFwdBands; ++k) {
+                bf16x4 t[4];
+#pragma unroll
+                for (int nt = 0; nt < 4; ++nt) {
+                    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+                    acc = mfma(w[l][nt][0], x[k][0], acc);
+                    acc = mfma(w[l][nt][1], x[k][1], acc);
+                    t[nt] = relu4(acc);
                 }
-                if (A.actT)
-                    *reinterpret_cast<bf16x4 *>(A.actT + (uint64_t)(l + 1) * 64 * A.npad + (uint64_t)c * A.npad + row0 +
-                                                4 * q) = v;
-            }
-            wave_sync();
-            a0 = *reinterpret_cast<const bf16x8 *>(H + r * 64 + 8 * q);
-            a1 = *reinterpret_cast<const bf16x8 *>(H + r * 64 + 32 + 8 * q);
-            wave_sync();
-        }
-        const bf16 *wb = wl + 4 * 4096 + r * 64;
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        acc = mfma(a0, *reinterpret_cast<const bf16x8 *>(wb + 8 * q), acc);
-        acc = mfma(a1, *reinterpret_cast<const bf16x8 *>(wb + 32 + 8 * q), acc);
-        if (A.y && r < kOut) {
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t row = row0 + 4 * q + i;
-                if (row < n) reinterpret_cast<float *>(A.y + row)[r] = acc[i];
+                x[k][0] = next_operand(t[0], t[1]);
+                x[k][1] = next_operand(t[2], t[3]);
             }
         }
-        if (A.qrec && r < kOut) {
-            // one lane per (row, component): distinct addresses, no atomics
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t row = row0 + 4 * q + i;
-                if (row < n) {
+#pragma unroll
+        for (int k = 0; k < kFwdBands; ++k) {
+            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+            acc = mfma(wo[0], x[k][0], acc);
+            acc = mfma(wo[1], x[k][1], acc);
+            // lanes q == 0 hold the outputs of sample r
+            const uint32_t row = (band + k) * 16 + r;
+            if (q == 0 && band + k < bands && row < n) {
+                if (A.y) {
+                    float *o = reinterpret_cast<float *>(A.y + row);
+                    o[0] = acc[0];
+                    o[1] = acc[1];
+                    o[2] = acc[2];
+                }
+                if (A.qrec) {
                     const CacheQuery rec = A.qrec[row];
-                    float *L = reinterpret_cast<float *>(A.st1 + rec.path) + r;
-                    *L = *L + rec.T[r] * fmaxf(acc[i], 0.0f);
+                    float *L = reinterpret_cast<float *>(A.st1 + rec.path);
+                    for (int c = 0; c < kOut; ++c) L[c] = L[c] + rec.T[c] * fmaxf(acc[c], 0.0f);
                 }
             }
+            x[k][0] = nx[k][0];
+            x[k][1] = nx[k][1];
         }
     }
 }
 
-struct BwdArgs {
-    const float4 *y, *target;   // prediction, target (x, y, z, -)
-    uint32_t n, npad;
-    const bf16 *wb;             // backward layout (= master layout)
-    const bf16 *actT;           // layer inputs, feature-major
-    bf16 *dzT;                  // 5 x [64][npad]: gradient at each layer's output, feature-major
-    float *loss;                // sum of the loss (atomic)
+struct TrainArgs {
+    const bf16 *x;              // N x 64
+    const float4 *target;       // N targets (x, y, z, -)
+    uint32_t n;
+    const bf16 *wt, *wb;        // forward / backward layout
+    float *partials;            // [gridDim.x][kP]: weight gradients of the workgroup's rows
+    float *loss;                // [gridDim.x]: their loss
 };
 
-__global__ void __launch_bounds__(kMlpBlock) k_mlp_bwd_data(BwdArgs A)
+// One workgroup (4 waves) per tile of 64 samples, a wave per band of 16.  The
+// weights stand in LDS in both layouts; a layer's inputs and output gradients are
+// written to LDS feature-major, where the weight gradient X^T dZ (k = samples) reads
+// its operands; its accumulators stay in registers over all of the workgroup's tiles (wave
+// w owns input features 16w .. 16w+15 of every layer).  Rows are padded to 36
+// dwords, which spreads both the 2-byte writes and the 16-byte reads over all banks.
+// Nothing but the inputs and one set of partial sums per workgroup goes
+// through memory (activations and gradients of five layers, feature-major, before).
+// 65,536 rows: a step 172 -> 51 us (this kernel 37, Adam 6); bound by the
+// latency of a tile's chain of layers with one wave per SIMD (144 KB of LDS); loading the next tile ahead costs registers
+// and 4 us.
+constexpr uint32_t kTile = 64;                 // samples
+constexpr uint32_t kRow = kTile + 8;           // row stride of every LDS matrix, in elements
+
+struct TrainLds {
+    bf16 wt[(4 * 64 + 16) * kRow];             // forward layout: row = output, 64 inputs
+    bf16 wb[4 * 64 * kRow];                    // backward layout: row = input, 64 outputs
+    bf16 wb4[64 * 24];                         // output layer: row = input, 16 outputs (padded to 24)
+    bf16 act[5][64 * kRow];                    // layer inputs: row = feature
+    bf16 dz[2][64 * kRow];                     // output gradients of the layer at hand: row = feature
+    float loss[4];
+};
+
+__global__ void __launch_bounds__(kMlpBlock) k_mlp_train(TrainArgs A)
 {
-    __shared__ bf16 wl[4 * 4096 + 64 * 16];
-    __shared__ bf16 hbuf[kMlpBlock / 64][16 * 64];
-    for (uint32_t i = threadIdx.x; i < (4 * 4096 + 64 * 16) / 8; i += kMlpBlock)
-        reinterpret_cast<bf16x8 *>(wl)[i] = reinterpret_cast<const bf16x8 *>(A.wb)[i];
-    __syncthreads();
-    const uint32_t lane = threadIdx.x & 63u, r = lane & 15u, q = lane >> 4, wv = threadIdx.x >> 6;
-    bf16 *H = hbuf[wv];
-    const uint32_t nbands = A.npad / 16, waves = gridDim.x * (kMlpBlock / 64);
+    extern __shared__ uint4 lds_raw[];
+    TrainLds &S = *reinterpret_cast<TrainLds *>(lds_raw);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, q = lane >> 4, wv = tid >> 6;
+    // weights: rows of 64 (8 x 16 B), padded
+    for (uint32_t i = tid; i < (4 * 64 + 16) * 8; i += kMlpBlock)
+        *reinterpret_cast<bf16x8 *>(S.wt + (i >> 3) * kRow + (i & 7u) * 8) = reinterpret_cast<const bf16x8 *>(A.wt)[i];
+    for (uint32_t i = tid; i < 4 * 64 * 8; i += kMlpBlock)
+        *reinterpret_cast<bf16x8 *>(S.wb + (i >> 3) * kRow + (i & 7u) * 8) = reinterpret_cast<const bf16x8 *>(A.wb)[i];
+    for (uint32_t i = tid; i < 64 * 2; i += kMlpBlock)
+        *reinterpret_cast<bf16x8 *>(S.wb4 + (i >> 1) * 24 + (i & 1u) * 8) =
+            reinterpret_cast<const bf16x8 *>(A.wb + 4 * 4096)[i];
+    // the output layer's gradient has 16 rows, 3 of them ever written
+    for (uint32_t i = tid; i < 16 * kRow / 8; i += kMlpBlock) reinterpret_cast<bf16x8 *>(S.dz[0])[i] = zero8();
+    f32x4 gw[kHidden][4], gw4 = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int l = 0; l < kHidden; ++l)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) gw[l][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     const float invn = 1.0f / (float)A.n;
     float lsum = 0.0f;
-    for (uint32_t band = blockIdx.x * (kMlpBlock / 64) + wv; band < nbands; band += waves) {
-        const uint32_t row0 = band * 16, row = row0 + r;
-        // output gradient: lanes q == 0 hold row r's 3 components in k = 0..2
-        bf16x8 a0 = zero8();
-        if (q == 0 && row < A.n) {
-            const float4 p = A.y[row], t = A.target[row];
-            const float pc[3] = {p.x, p.y, p.z}, tc[3] = {t.x, t.y, t.z};
-            for (int c = 0; c < kOut; ++c) {
-                const float den = pc[c] * pc[c] + 0.01f, d = pc[c] - tc[c];
-                lsum += d * d / den * invn;
-                a0[c] = (bf16)(2.0f * d / den * invn);
+    const uint32_t tiles = (A.n + kTile - 1) / kTile, s = wv * 16 + r;   // this lane's sample within a tile
+    // a tile's D-layout values (features 16 nt + 4q + i of sample s) into a feature-major matrix
+    auto put = [&](bf16 *m, int nt, bf16x4 v) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m[(nt * 16 + 4 * q + i) * kRow + s] = v[i];
+    };
+    // weight gradient tiles of M-tile wv: X^T (rows = inputs) times dZ (rows = outputs), k = the tile's samples
+    auto accumulate = [&](const bf16 *x, const bf16 *d, f32x4 *acc, int ntiles) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const bf16x8 a = *reinterpret_cast<const bf16x8 *>(x + (wv * 16 + r) * kRow + 32 * h + 8 * q);
+#pragma unroll
+            for (int t = 0; t < ntiles; ++t) {
+                const bf16x8 b = *reinterpret_cast<const bf16x8 *>(d + (t * 16 + r) * kRow + 32 * h + 8 * q);
+                acc[t] = mfma(a, b, acc[t]);
             }
         }
-        // dZ_4 feature-major (16 columns)
-        if (q == 0) {
-            for (int c = 0; c < kOutPad; ++c)
-                A.dzT[(uint64_t)4 * 64 * A.npad + (uint64_t)c * A.npad + row] = c < 8 ? a0[c] : (bf16)0.0f;
+    };
+    __syncthreads();
+    for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const uint32_t row = tile * kTile + s;
+        const bool in = row < A.n;
+        const bf16 *xp = A.x + (uint64_t)(in ? row : 0u) * 64 + 8 * q;
+        bf16x8 x0 = in ? *reinterpret_cast<const bf16x8 *>(xp) : zero8();
+        bf16x8 x1 = in ? *reinterpret_cast<const bf16x8 *>(xp + 32) : zero8();
+        const float4 tg = in && q == 0 ? A.target[row] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            S.act[0][(8 * q + j) * kRow + s] = x0[j];
+            S.act[0][(32 + 8 * q + j) * kRow + s] = x1[j];
         }
-        // back through layer 4: dH4 = dY4 W4^T (k = output column, padded to 32)
-        bf16x8 g0 = zero8(), g1 = zero8();
+        // forward; bit 4 nt + i of mask[l]: the lane's value of layer l's output is positive
+        uint32_t mask[kHidden];
+#pragma unroll
+        for (int l = 0; l < kHidden; ++l) {
+            bf16x4 t[4];
+            uint32_t mk = 0;
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt) {
+                const bf16 *w = S.wt + (l * 64 + nt * 16 + (int)r) * kRow + 8 * q;
+                f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+                acc = mfma(*reinterpret_cast<const bf16x8 *>(w), x0, acc);
+                acc = mfma(*reinterpret_cast<const bf16x8 *>(w + 32), x1, acc);
+                t[nt] = relu4(acc);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) mk |= (float)t[nt][i] > 0.0f ? 1u << (4 * nt + i) : 0u;
+                put(S.act[l + 1], nt, t[nt]);
+            }
+            mask[l] = mk;
+            x0 = next_operand(t[0], t[1]);
+            x1 = next_operand(t[2], t[3]);
+        }
+        f32x4 y = {0.0f, 0.0f, 0.0f, 0.0f};
         {
-            for (int nt = 0; nt < 4; ++nt) {
-                const uint32_t i_in = nt * 16 + r;
-                const bf16x8 b = q < 2 ? *reinterpret_cast<const bf16x8 *>(wl + 4 * 4096 + i_in * 16 + 8 * q) : zero8();
-                f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-                acc = mfma(a0, b, acc);
-                // ReLU mask of layer 3's output (= layer 4's input)
-                const bf16x4 h = *reinterpret_cast<const bf16x4 *>(A.actT + (uint64_t)4 * 64 * A.npad +
-                                                                    (uint64_t)i_in * A.npad + row0 + 4 * q);
-                bf16x4 dz;
-                for (int i = 0; i < 4; ++i) {
-                    const bf16 v = (float)h[i] > 0.0f ? (bf16)acc[i] : (bf16)0.0f;
-                    dz[i] = v;
-                    H[(4 * q + i) * 64 + i_in] = v;
-                }
-                *reinterpret_cast<bf16x4 *>(A.dzT + (uint64_t)3 * 64 * A.npad + (uint64_t)i_in * A.npad + row0 +
-                                            4 * q) = dz;
-            }
-            wave_sync();
-            g0 = *reinterpret_cast<const bf16x8 *>(H + r * 64 + 8 * q);
-            g1 = *reinterpret_cast<const bf16x8 *>(H + r * 64 + 32 + 8 * q);
-            wave_sync();
+            const bf16 *w = S.wt + (4 * 64 + r) * kRow + 8 * q;
+            y = mfma(*reinterpret_cast<const bf16x8 *>(w), x0, y);
+            y = mfma(*reinterpret_cast<const bf16x8 *>(w + 32), x1, y);
         }
-        // layers 3..1: dH_l = dZ_l W_l^T, masked by layer l-1's output
-        for (int l = 3; l >= 1; --l) {
-            for (int nt = 0; nt < 4; ++nt) {
-                const uint32_t i_in = nt * 16 + r;
-                const bf16 *wrow = wl + (uint32_t)l * 4096 + i_in * 64;
-                f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-                acc = mfma(g0, *reinterpret_cast<const bf16x8 *>(wrow + 8 * q), acc);
-                acc = mfma(g1, *reinterpret_cast<const bf16x8 *>(wrow + 32 + 8 * q), acc);
-                const bf16x4 h = *reinterpret_cast<const bf16x4 *>(A.actT + (uint64_t)l * 64 * A.npad +
-                                                                    (uint64_t)i_in * A.npad + row0 + 4 * q);
-                bf16x4 dz;
-                for (int i = 0; i < 4; ++i) {
-                    const bf16 v = (float)h[i] > 0.0f ? (bf16)acc[i] : (bf16)0.0f;
-                    dz[i] = v;
-                    H[(4 * q + i) * 64 + i_in] = v;
-                }
-                *reinterpret_cast<bf16x4 *>(A.dzT + (uint64_t)(l - 1) * 64 * A.npad + (uint64_t)i_in * A.npad +
-                                            row0 + 4 * q) = dz;
+        // output gradient: lanes q == 0, k = 0..2 of the next operand
+        bf16x8 g0 = zero8(), g1 = zero8();
+        if (q == 0 && in) {
+            const float tc[3] = {tg.x, tg.y, tg.z};
+#pragma unroll
+            for (int c = 0; c < kOut; ++c) {
+                const float den = y[c] * y[c] + 0.01f, d = y[c] - tc[c];
+                lsum += d * d / den * invn;
+                g0[c] = (bf16)(2.0f * d / den * invn);
             }
-            wave_sync();
-            g0 = *reinterpret_cast<const bf16x8 *>(H + r * 64 + 8 * q);
-            g1 = *reinterpret_cast<const bf16x8 *>(H + r * 64 + 32 + 8 * q);
-            wave_sync();
         }
+        if (q == 0)
+            for (int c = 0; c < kOut; ++c) S.dz[0][c * kRow + s] = g0[c];
+        __syncthreads();   // all bands' layer inputs and output gradients
+        accumulate(S.act[4], S.dz[0], &gw4, 1);
+        // back through layer 4 (k = 16 outputs, padded to 32), then 3..1
+#pragma unroll
+        for (int l = kHidden; l >= 1; --l) {
+            bf16 *dz = S.dz[(kHidden - l + 1) & 1];
+            bf16x4 t[4];
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt) {
+                f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+                if (l == kHidden) {
+                    const bf16x8 w = q < 2 ? *reinterpret_cast<const bf16x8 *>(S.wb4 + (nt * 16 + r) * 24 + 8 * q) : zero8();
+                    acc = mfma(w, g0, acc);
+                } else {
+                    const bf16 *w = S.wb + (l * 64 + nt * 16 + (int)r) * kRow + 8 * q;
+                    acc = mfma(*reinterpret_cast<const bf16x8 *>(w), g0, acc);
+                    acc = mfma(*reinterpret_cast<const bf16x8 *>(w + 32), g1, acc);
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) t[nt][i] = (mask[l - 1] >> (4 * nt + i)) & 1u ? (bf16)acc[i] : (bf16)0.0f;
+                put(dz, nt, t[nt]);
+            }
+            g0 = next_operand(t[0], t[1]);
+            g1 = next_operand(t[2], t[3]);
+            __syncthreads();   // this layer's gradients; the other buffer is free again
+            accumulate(S.act[l - 1], dz, gw[l - 1], 4);
+        }
+        __syncthreads();       // act and dz are rewritten by the next tile
+        // dz[0] held layer 0's gradients: rows 3..15 are zero again for the output's
+        for (uint32_t i = tid; i < 16 * kRow / 8; i += kMlpBlock) reinterpret_cast<bf16x8 *>(S.dz[0])[i] = zero8();
+        __syncthreads();
+    }
+    float *P = A.partials + (uint64_t)blockIdx.x * kP;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t k_in = wv * 16 + 4 * q + i;
+#pragma unroll
+        for (int l = 0; l < kHidden; ++l)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) P[l * 4096 + k_in * 64 + t * 16 + r] = gw[l][t][i];
+        P[16384 + k_in * 16 + r] = gw4[i];
     }
     for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off);
-    if (lane == 0 && A.loss) atomicAdd(A.loss, lsum);
-}
-
-struct BwdWArgs {
-    const bf16 *actT, *dzT;
-    uint32_t npad;
-    float *partials;   // [nchunks][kP]
-};
-
-// grid (chunks, 5 layers); wave w owns input features 16w .. 16w+15
-__global__ void __launch_bounds__(kMlpBlock) k_mlp_bwd_w(BwdWArgs A)
-{
-    const uint32_t lane = threadIdx.x & 63u, r = lane & 15u, q = lane >> 4, wv = threadIdx.x >> 6;
-    const uint32_t layer = blockIdx.y, chunk = blockIdx.x;
-    const uint32_t s0 = chunk * kChunk, s1 = min(A.npad, s0 + kChunk);
-    const int ntiles = layer < 4 ? 4 : 1;
-    const bf16 *X = A.actT + (uint64_t)layer * 64 * A.npad;
-    const bf16 *D = A.dzT + (uint64_t)layer * 64 * A.npad;
-    const uint32_t i_row = wv * 16 + r;
-    f32x4 acc[4];
-    for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint32_t s = s0; s + 32 <= s1; s += 32) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8 *>(X + (uint64_t)i_row * A.npad + s + 8 * q);
-        for (int t = 0; t < ntiles; ++t) {
-            const bf16x8 b = *reinterpret_cast<const bf16x8 *>(D + (uint64_t)(t * 16 + r) * A.npad + s + 8 * q);
-            acc[t] = mfma(a, b, acc[t]);
-        }
-    }
-    float *P = A.partials + (uint64_t)chunk * kP;
-    for (int t = 0; t < ntiles; ++t) {
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t k_in = wv * 16 + 4 * q + i, n_out = t * 16 + r;
-            const uint32_t idx = layer < 4 ? layer * 4096 + k_in * 64 + n_out : 16384 + k_in * 16 + n_out;
-            P[idx] = acc[t][i];
-        }
-    }
+    if (lane == 0) S.loss[wv] = lsum;
+    __syncthreads();
+    if (tid == 0) A.loss[blockIdx.x] = S.loss[0] + S.loss[1] + S.loss[2] + S.loss[3];
 }
 
 struct AdamArgs {
     const float *partials;
-    uint32_t nchunks;
+    uint32_t nparts;
+    const float *loss_parts;
+    float *loss;
     float *w, *m, *v;
     bf16 *wt, *wb;
     float *grad_out;   // optional: the summed gradient
@@ -306,17 +384,36 @@ __device__ __forceinline__ void write_bf16(bf16 *wt, bf16 *wb, uint32_t p, float
     }
 }
 
-__global__ void k_mlp_adam(AdamArgs A)
+// sums the workgroups' partial gradients (64 parameters per block, 4 threads
+// each, in fixed order) and applies Adam; block 0 also sums the loss
+__global__ void __launch_bounds__(256) k_mlp_adam(AdamArgs A)
 {
-    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= kP) return;
-    float g = 0.0f;
-    for (uint32_t c = 0; c < A.nchunks; ++c) g += A.partials[(uint64_t)c * kP + p];
-    if (padded(p)) g = 0.0f;
-    if (A.grad_out) A.grad_out[p] = g;
+    __shared__ float s_sum[4][64], s_loss[256];
+    const uint32_t j = threadIdx.x & 63u, g = threadIdx.x >> 6, p = blockIdx.x * 64 + j;
+    float g0 = 0.0f;
+#pragma unroll 8
+    for (uint32_t c = g; c < A.nparts; c += 4) g0 += A.partials[(uint64_t)c * kP + p];
+    s_sum[g][j] = g0;
+    if (blockIdx.x == 0) {
+        float l = 0.0f;
+        for (uint32_t c = threadIdx.x; c < A.nparts; c += 256) l += A.loss_parts[c];
+        s_loss[threadIdx.x] = l;
+    }
+    __syncthreads();
+    if (blockIdx.x == 0) {   // block-uniform
+        for (uint32_t h = 128; h > 0; h >>= 1) {
+            if (threadIdx.x < h) s_loss[threadIdx.x] += s_loss[threadIdx.x + h];
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) *A.loss = s_loss[0];
+    }
+    if (g != 0) return;
+    float gr = (s_sum[0][j] + s_sum[1][j]) + (s_sum[2][j] + s_sum[3][j]);
+    if (padded(p)) gr = 0.0f;
+    if (A.grad_out) A.grad_out[p] = gr;
     if (!A.update) return;
-    const float m = A.b1 * A.m[p] + (1.0f - A.b1) * g;
-    const float v = A.b2 * A.v[p] + (1.0f - A.b2) * g * g;
+    const float m = A.b1 * A.m[p] + (1.0f - A.b1) * gr;
+    const float v = A.b2 * A.v[p] + (1.0f - A.b2) * gr * gr;
     A.m[p] = m;
     A.v[p] = v;
     float w = A.w[p];
@@ -324,6 +421,7 @@ __global__ void k_mlp_adam(AdamArgs A)
     A.w[p] = w;
     write_bf16(A.wt, A.wb, p, w);
 }
+static_assert(kP % 64 == 0, "k_mlp_adam: 64 parameters per block");
 
 __global__ void k_mlp_sync_bf16(const float *w, bf16 *wt, bf16 *wb)
 {
@@ -344,67 +442,51 @@ int mlp_status(const char *what)
 }  // namespace
 
 struct Mlp : Obj {
-    DevBuf w, m, v, wt, wb, actT, dzT, partials, loss, grad, ybuf;
+    DevBuf w, m, v, wt, wb, partials, loss, loss_parts, grad;
     float lr = 1e-2f, b1 = 0.9f, b2 = 0.99f, eps = 1e-8f;
     uint32_t step = 0, ncu = 256;
-    uint32_t cap = 0;   // npad the activation buffers hold
     void release_all()
     {
-        for (DevBuf *b : {&w, &m, &v, &wt, &wb, &actT, &dzT, &partials, &loss, &grad, &ybuf}) b->release();
+        for (DevBuf *b : {&w, &m, &v, &wt, &wb, &partials, &loss, &loss_parts, &grad}) b->release();
     }
-    int reserve_rows(uint32_t npad)
+    // blocks of 4 waves that cover the bands of n rows, two per CU at most
+    uint32_t forward_blocks(uint32_t n) const
     {
-        if (npad <= cap) return 0;
-        const uint64_t nchunks = (npad + kChunk - 1) / kChunk;
-        if (actT.reserve((uint64_t)5 * 64 * npad * 2) || dzT.reserve((uint64_t)5 * 64 * npad * 2) ||
-            partials.reserve(nchunks * kP * 4))
-            return SOLHIP_ERROR_OUT_OF_MEMORY;
-        cap = npad;
-        return 0;
+        const uint32_t per_block = 16u * kFwdBands * (kMlpBlock / 64);
+        return std::max(1u, std::min((n + per_block - 1) / per_block, ncu * 2));
     }
-    int forward(hipStream_t s, const bf16 *x, uint32_t n, float4 *y, bool save)
+    int forward(hipStream_t s, const bf16 *x, uint32_t n, float4 *y)
     {
-        const uint32_t npad = (n + 31u) & ~31u;
-        if (save && reserve_rows(npad)) return SOLHIP_ERROR_OUT_OF_MEMORY;
         FwdArgs a;
         std::memset(&a, 0, sizeof(a));
         a.x = x;
         a.n = n;
-        a.npad = npad;
         a.wt = (const bf16 *)wt.ptr;
         a.y = y;
-        a.actT = save ? (bf16 *)actT.ptr : nullptr;
-        const uint32_t blocks = std::min<uint32_t>((npad / 16 + 3) / 4, ncu * 4);
-        hipLaunchKernelGGL(k_mlp_fwd, dim3(std::max(1u, blocks)), dim3(kMlpBlock), 0, s, a);
+        hipLaunchKernelGGL(k_mlp_fwd, dim3(forward_blocks(n)), dim3(kMlpBlock), 0, s, a);
         return mlp_status("mlp forward");
     }
-    // loss gradient of (x, target) summed into grad (and applied by Adam when update)
-    int backward(hipStream_t s, uint32_t n, const float4 *y, const float4 *target, bool update, float *grad_host)
+    // loss and its gradient on (x, target), applied by Adam when update
+    int fit(hipStream_t s, const bf16 *x, const float4 *target, uint32_t n, bool update, float *grad_host)
     {
-        // rows n .. npad (a multiple of 32) carry zero inputs and zero
-        // gradients, so they add nothing to the weight gradients
-        const uint32_t npad = (n + 31u) & ~31u;
-        const uint32_t nchunks = (npad + kChunk - 1) / kChunk;
-        BwdArgs b;
-        b.y = y;
+        // one workgroup per CU, each over several tiles
+        const uint32_t tiles = (n + kTile - 1) / kTile, blocks = std::min(tiles, ncu);
+        if (partials.reserve((uint64_t)blocks * kP * 4) || loss_parts.reserve((uint64_t)blocks * 4))
+            return SOLHIP_ERROR_OUT_OF_MEMORY;
+        TrainArgs b;
+        b.x = x;
         b.target = target;
         b.n = n;
-        b.npad = npad;
+        b.wt = (const bf16 *)wt.ptr;
         b.wb = (const bf16 *)wb.ptr;
-        b.actT = (const bf16 *)actT.ptr;
-        b.dzT = (bf16 *)dzT.ptr;
-        b.loss = (float *)loss.ptr;
-        const uint32_t blocks = std::min<uint32_t>((npad / 16 + 3) / 4, ncu * 4);
-        hipLaunchKernelGGL(k_mlp_bwd_data, dim3(std::max(1u, blocks)), dim3(kMlpBlock), 0, s, b);
-        BwdWArgs c;
-        c.actT = (const bf16 *)actT.ptr;
-        c.dzT = (const bf16 *)dzT.ptr;
-        c.npad = npad;
-        c.partials = (float *)partials.ptr;
-        hipLaunchKernelGGL(k_mlp_bwd_w, dim3(nchunks, 5), dim3(kMlpBlock), 0, s, c);
+        b.partials = (float *)partials.ptr;
+        b.loss = (float *)loss_parts.ptr;
+        hipLaunchKernelGGL(k_mlp_train, dim3(blocks), dim3(kMlpBlock), sizeof(TrainLds), s, b);
         AdamArgs d;
         d.partials = (const float *)partials.ptr;
-        d.nchunks = nchunks;
+        d.nparts = blocks;
+        d.loss_parts = (const float *)loss_parts.ptr;
+        d.loss = (float *)loss.ptr;
         d.w = (float *)w.ptr;
         d.m = (float *)m.ptr;
         d.v = (float *)v.ptr;
@@ -419,8 +501,8 @@ struct Mlp : Obj {
         d.eps = eps;
         d.c1 = 1.0f - std::pow(b1, (float)std::max(1u, step));
         d.c2 = 1.0f - std::pow(b2, (float)std::max(1u, step));
-        hipLaunchKernelGGL(k_mlp_adam, dim3((kP + 255) / 256), dim3(256), 0, s, d);
-        int rc = mlp_status("mlp backward");
+        hipLaunchKernelGGL(k_mlp_adam, dim3(kP / 64), dim3(256), 0, s, d);
+        int rc = mlp_status("mlp training");
         if (rc) return rc;
         if (grad_host) {
             SOLHIP_HIP_CHECK(hipMemcpyAsync(grad_host, grad.ptr, kP * 4, hipMemcpyDeviceToHost, s));
@@ -429,7 +511,6 @@ struct Mlp : Obj {
         return 0;
     }
 };
-
 
 Mlp *mlp_new(Context *c, uint32_t seed, float lr);
 
@@ -440,24 +521,19 @@ int mlp_query(hipStream_t s, Mlp *m, const uint16_t *feat, const uint32_t *n_dev
     std::memset(&a, 0, sizeof(a));
     a.x = (const bf16 *)feat;
     a.n = n_max;
-    a.npad = (n_max + 31u) & ~31u;
     a.n_dev = n_dev;
     a.wt = (const bf16 *)m->wt.ptr;
     a.qrec = qrec;
     a.st1 = st1;
-    const uint32_t blocks = std::min<uint32_t>((a.npad / 16 + 3) / 4, m->ncu * 4);
-    hipLaunchKernelGGL(k_mlp_fwd, dim3(std::max(1u, blocks)), dim3(kMlpBlock), 0, s, a);
+    hipLaunchKernelGGL(k_mlp_fwd, dim3(m->forward_blocks(n_max)), dim3(kMlpBlock), 0, s, a);
     return mlp_status("cache query");
 }
 
 int mlp_train_dev(hipStream_t s, Mlp *m, const uint16_t *feat, const float4 *target, uint32_t n, uint32_t steps)
 {
     if (n == 0) return 0;
-    if (m->ybuf.reserve((uint64_t)n * 16)) return SOLHIP_ERROR_OUT_OF_MEMORY;
     for (uint32_t k = 0; k < steps; ++k) {
-        int rc = m->forward(s, (const bf16 *)feat, n, (float4 *)m->ybuf.ptr, true);
-        if (rc) return rc;
-        rc = m->backward(s, n, (const float4 *)m->ybuf.ptr, target, true, nullptr);
+        const int rc = m->fit(s, (const bf16 *)feat, target, n, true, nullptr);
         if (rc) return rc;
     }
     return 0;
@@ -503,6 +579,13 @@ Mlp *mlp_new(Context *c, uint32_t seed, float lr)
         m->wb.reserve(kP * 2) || m->loss.reserve(256) || m->grad.reserve(kP * 4)) {
         mlp_delete(m);
         set_error("mlp allocation failed");
+        return nullptr;
+    }
+    // more LDS than the 64 KiB a launch may ask for by default
+    if (hipFuncSetAttribute(reinterpret_cast<const void *>(k_mlp_train), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)sizeof(TrainLds)) != hipSuccess) {
+        mlp_delete(m);
+        set_error("the device does not give k_mlp_train its LDS");
         return nullptr;
     }
     std::vector<float> w;
@@ -601,7 +684,7 @@ int32_t solhip_mlp_forward(solhip_ctx ctx, solhip_stream st, solhip_mlp h, solhi
     void *pi, *po;
     int rc = mlp_io(c, in, (uint64_t)n * 128, out, (uint64_t)n * 16, &pi, &po);
     if (rc) return rc;
-    return m->forward(s, (const bf16 *)pi, n, (float4 *)po, false);
+    return m->forward(s, (const bf16 *)pi, n, (float4 *)po);
 }
 
 static int32_t mlp_fit(solhip_ctx ctx, solhip_stream st, solhip_mlp h, solhip_buffer in, solhip_buffer target,
@@ -618,14 +701,8 @@ static int32_t mlp_fit(solhip_ctx ctx, solhip_stream st, solhip_mlp h, solhip_bu
     void *pi, *pt;
     int rc = mlp_io(c, in, (uint64_t)n * 128, target, (uint64_t)n * 16, &pi, &pt);
     if (rc) return rc;
-    if (m->ybuf.reserve((uint64_t)n * 16)) return SOLHIP_ERROR_OUT_OF_MEMORY;
     for (uint32_t k = 0; k < steps; ++k) {
-        rc = launch_fill(s, (uint32_t *)m->loss.ptr, 1, 0u);
-        if (rc) return rc;
-        rc = m->forward(s, (const bf16 *)pi, n, (float4 *)m->ybuf.ptr, true);
-        if (rc) return rc;
-        rc = m->backward(s, n, (const float4 *)m->ybuf.ptr, (const float4 *)pt, update,
-                         k + 1 == steps ? grad_host : nullptr);
+        rc = m->fit(s, (const bf16 *)pi, (const float4 *)pt, n, update, k + 1 == steps ? grad_host : nullptr);
         if (rc) return rc;
     }
     if (loss_out) {
