@@ -34,10 +34,6 @@ namespace solhip {
 #ifndef SOLHIP_AO_REFILL
 #define SOLHIP_AO_REFILL 16
 #endif
-// fetch partitions of the persistent AO kernel (fetch.h)
-#ifndef SOLHIP_AO_PARTS
-#define SOLHIP_AO_PARTS 64
-#endif
 
 // ---------------------------------------------------------------------------
 // plain ray-traced AO (wavefront)
@@ -147,7 +143,7 @@ __global__ void __launch_bounds__(kProgBlock) SOLHIP_AO_RAYS_OCCUPANCY k_ao_rays
     bool has = false;
     uint32_t rid = 0, pix = 0;
     PartFetch pf;
-    pf.init(A.aoheads, SOLHIP_AO_PARTS, total);
+    pf.init(A.aoheads, total);
     while (true) {
         const uint64_t idle = __ballot(!has);
         const uint32_t nidle = (uint32_t)__popcll(idle);
@@ -217,7 +213,7 @@ static int launch_status(const char *what)
         if (timer) (timer)->end(s, id);                                                       \
     } while (0)
 
-uint64_t ao_head_bytes() { return (uint64_t)SOLHIP_AO_PARTS * kHeadStride * 4; }
+uint64_t ao_head_bytes() { return (uint64_t)kFetchWords * 4; }
 
 int launch_ao(hipStream_t s, const ProgArgs &a, Timer *timer)
 {
@@ -229,7 +225,7 @@ int launch_ao(hipStream_t s, const ProgArgs &a, Timer *timer)
     // persistent grid: as many waves as fit (SOLHIP_AO_WAVES per SIMD, 4 SIMDs per CU)
     const uint32_t blocks = a.ncu * 4 * SOLHIP_AO_WAVES;
     // the fetch heads start at zero (a fill kernel: no memset node in a captured graph)
-    int rc = launch_fill(s, a.aoheads, (uint64_t)SOLHIP_AO_PARTS * kHeadStride, 0u);
+    int rc = launch_fill(s, a.aoheads, (uint64_t)kFetchWords, 0u);
     if (rc) return rc;
     trav_dispatch(a.sv.mode, a.count, [&](auto mode, auto count) {
         if (timer) timer->begin(s, SOLHIP_KERNEL_AO_PRIMARY);

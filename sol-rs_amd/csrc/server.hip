@@ -51,8 +51,6 @@ constexpr uint32_t kSrvBlock = 64;
 #define SOLHIP_SRV_WAVES 4
 #endif
 #define SOLHIP_SRV_OCCUPANCY __attribute__((amdgpu_waves_per_eu(SOLHIP_SRV_WAVES)))
-// fetch partitions of the extend and shadow kernels (fetch.h)
-constexpr uint32_t kSrvParts = 64;
 constexpr uint32_t kMaxJobs = 256;   // job index lives in 8 bits of the slot meta word
 
 // per-job constants (device array, one entry per running-job index)
@@ -84,7 +82,7 @@ struct SrvArgs {
     float4 *scontrib;
     uint32_t *retire;
     uint32_t *counts;     // [0], [1] extension queues, [2] shadow queue, [3] retire list
-    uint32_t *heads;      // partitioned fetch heads: extend, then shadow (kSrvParts each)
+    uint32_t *heads;      // partitioned fetch heads: extend, then shadow (kFetchWords each)
     uint32_t *done;       // finished pixels per job index
     Counters *counters;
 };
@@ -194,7 +192,7 @@ __device__ __forceinline__ void srv_trace(const SrvArgs &A, const QRay *q, uint3
     bool has = false;
     uint32_t idx = 0, path = 0;
     PartFetch pf;
-    pf.init(heads, kSrvParts, cnt);
+    pf.init(heads, cnt);
     while (true) {
         const uint64_t idle = __ballot(!has);
         const uint32_t nidle = (uint32_t)__popcll(idle);
@@ -254,7 +252,7 @@ __global__ void __launch_bounds__(kSrvBlock) SOLHIP_SRV_OCCUPANCY k_srv_extend(S
 
 __global__ void __launch_bounds__(kSrvBlock) SOLHIP_SRV_OCCUPANCY k_srv_shadow(SrvArgs A)
 {
-    srv_trace<true>(A, A.sq, A.counts[2], A.heads + kSrvParts * kHeadStride, SOLHIP_KERNEL_SRV_SHADOW);
+    srv_trace<true>(A, A.sq, A.counts[2], A.heads + kFetchWords, SOLHIP_KERNEL_SRV_SHADOW);
 }
 
 // waves per SIMD the shade kernel is compiled for (0: the compiler's choice,
@@ -316,7 +314,7 @@ __global__ void __launch_bounds__(kSrvShadeBlock) k_srv_retire(SrvArgs A, uint32
     __shared__ uint32_t lds[kSrvShadeWaves + 1];
     if (blockIdx.x == 0) {
         // this step's extend and shadow are complete
-        for (uint32_t k = threadIdx.x; k < 2 * kSrvParts; k += blockDim.x) A.heads[k * kHeadStride] = 0;
+        for (uint32_t k = threadIdx.x; k < 2 * kFetchParts; k += blockDim.x) fetch_reset(A.heads, k);
     }
     const uint32_t cnt = A.counts[3];
     const uint32_t nthreads = gridDim.x * blockDim.x;
@@ -698,7 +696,7 @@ int32_t solhip_server_create(solhip_ctx ctx, uint64_t hbm_budget, uint32_t max_j
                 sv->q0.reserve(n * sizeof(QRay)) || sv->q1.reserve(n * sizeof(QRay)) ||
                 sv->hits.reserve(n * sizeof(QHit)) || sv->sq.reserve(n * sizeof(QRay)) ||
                 sv->scontrib.reserve(n * 16) || sv->retire.reserve(n * 4) || sv->counts.reserve(256) ||
-                sv->heads.reserve(2ull * kSrvParts * kHeadStride * 4) || sv->done.reserve((uint64_t)max_jobs * 4);
+                sv->heads.reserve(2ull * kFetchWords * 4) || sv->done.reserve((uint64_t)max_jobs * 4);
     if (!fail) fail = hipStreamCreateWithFlags(&sv->stream, hipStreamNonBlocking) != hipSuccess ||
                       hipHostMalloc((void **)&sv->done_host, sizeof(uint32_t) * max_jobs, hipHostMallocDefault) !=
                           hipSuccess;
@@ -709,7 +707,7 @@ int32_t solhip_server_create(solhip_ctx ctx, uint64_t hbm_budget, uint32_t max_j
         return SOLHIP_ERROR_OUT_OF_MEMORY;
     }
     if (launch_fill(sv->stream, (uint32_t *)sv->counts.ptr, 64, 0u) ||
-        launch_fill(sv->stream, (uint32_t *)sv->heads.ptr, 2ull * kSrvParts * kHeadStride, 0u) ||
+        launch_fill(sv->stream, (uint32_t *)sv->heads.ptr, 2ull * kFetchWords, 0u) ||
         launch_fill(sv->stream, (uint32_t *)sv->done.ptr, max_jobs, 0u) || hipStreamSynchronize(sv->stream)) {
         sv->release_all();
         delete sv;

@@ -68,12 +68,6 @@ __device__ __forceinline__ float ray_tmin(const WfArgs &A)
     return fmaxf(1.0f, sqrtf(o[0] * o[0] + o[1] * o[1] + o[2] * o[2])) * 1e-3f;
 }
 
-// fetch partitions of the extend and shadow kernels (fetch.h)
-#ifndef SOLHIP_WF_PARTS
-#define SOLHIP_WF_PARTS 64
-#endif
-constexpr uint32_t kWfParts = SOLHIP_WF_PARTS;
-
 // samples traced in pass `pass` (the last pass may hold fewer than S)
 __device__ __forceinline__ uint32_t pass_samples(const WfArgs &A, uint32_t pass)
 {
@@ -91,7 +85,7 @@ __global__ void k_pt_generate(WfArgs A, uint32_t pass)
         A.counts[1] = 0;
         A.counts[2] = 0;
     }
-    if (e < 2 * (A.max_depth + 1) * kWfParts) A.heads[e * kHeadStride] = 0;
+    if (e < 2 * (A.max_depth + 1) * kFetchParts) fetch_reset(A.heads, e);
     if (e >= n) return;
     const uint32_t sl = e / A.nslots, slot = e - sl * A.nslots;
     uint32_t x, y;
@@ -218,7 +212,7 @@ __device__ __forceinline__ void trace_queue(const WfArgs &A, const QRay *q, uint
     bool has = false;
     uint32_t idx = 0, path = 0;
     PartFetch pf;
-    pf.init(heads, kWfParts, cnt);
+    pf.init(heads, cnt);
     while (true) {
         const uint64_t idle = __ballot(!has);
         const uint32_t nidle = (uint32_t)__popcll(idle);
@@ -268,7 +262,7 @@ __global__ void SOLHIP_WF_OCCUPANCY k_pt_extend(WfArgs A, uint32_t b)
     const uint32_t cnt = A.counts[b & 1];
     if (cnt <= A.finish_at) return;   // k_pt_finish has traced it
     const unsigned long long rays = b ? cnt : (unsigned long long)(cnt / A.nslots) * A.slice_pix;
-    trace_queue<false, COUNT, MODE>(A, A.q[b & 1], cnt, rays, A.heads + 2 * b * kWfParts * kHeadStride,
+    trace_queue<false, COUNT, MODE>(A, A.q[b & 1], cnt, rays, A.heads + 2 * b * kFetchWords,
                                     SOLHIP_KERNEL_PT_EXTEND);
 }
 
@@ -277,7 +271,7 @@ __global__ void SOLHIP_WF_OCCUPANCY k_pt_shadow(WfArgs A, uint32_t b)
 {
     const uint32_t cnt = A.counts[2];
     if (cnt == 0) return;
-    trace_queue<true, COUNT, MODE>(A, A.sq, cnt, cnt, A.heads + (2 * b + 1) * kWfParts * kHeadStride,
+    trace_queue<true, COUNT, MODE>(A, A.sq, cnt, cnt, A.heads + (2 * b + 1) * kFetchWords,
                                    SOLHIP_KERNEL_PT_SHADOW);
 }
 
@@ -330,7 +324,7 @@ k_pt_finish(WfArgs A, uint32_t b)
     V3 sc, nd;
     bool cont = false;
     PartFetch pf;
-    pf.init(A.heads + 2 * b * kWfParts * kHeadStride, kWfParts, cnt);
+    pf.init(A.heads + 2 * b * kFetchWords, cnt);
     while (true) {
         const uint64_t waiting = __ballot(state == kDone || (state == kIdle && !pf.exhausted));
         const bool tracing = __ballot(state == kTrace) != 0;
@@ -812,7 +806,7 @@ int launch_status(const char *what)
 
 uint32_t wf_threads_per_cu() { return 4u * SOLHIP_WF_WAVES * 64u; }
 
-uint32_t wf_head_words() { return kWfParts * kHeadStride; }
+uint32_t wf_head_words() { return kFetchWords; }
 
 uint32_t wf_finish_lanes_per_cu() { return 4u * SOLHIP_FINISH_WAVES * 64u; }
 
@@ -868,7 +862,7 @@ int launch_pathtrace_passes(hipStream_t s, const WfArgs &a0, Timer *timer, const
     const uint32_t blk = a.block;
     const size_t lds = (size_t)a.sv.stack_depth * sizeof(uint2) * blk;
     const uint32_t nheads = 2 * (a.max_depth + 1);
-    const uint32_t gen_blocks = (std::max(a.S * a.nslots, nheads * kWfParts) + blk - 1) / blk;
+    const uint32_t gen_blocks = (std::max(a.S * a.nslots, nheads * kFetchParts) + blk - 1) / blk;
     const uint32_t fold_blocks = (a.nslots + blk - 1) / blk;
     const uint32_t passes = (a.spp + a.S - 1) / a.S;
     auto shade_grid = [&](uint32_t waves) {
