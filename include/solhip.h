@@ -332,10 +332,10 @@ enum {
     SOLHIP_KERNEL_PT_FINALIZE = 10, /* sample mean, accumulation, RGBA8 */
     SOLHIP_KERNEL_PT_LIGHTS = 11,   /* emitter table (next-event estimation) */
     SOLHIP_KERNEL_SRV_ADMIT = 12,   /* render server: first camera rays of an admitted job */
-    SOLHIP_KERNEL_SRV_EXTEND = 13,  /* render server: closest hits of all live jobs' rays */
-    SOLHIP_KERNEL_SRV_SHADE = 14,
-    SOLHIP_KERNEL_SRV_SHADOW = 15,
-    SOLHIP_KERNEL_SRV_RETIRE = 16,  /* render server: finished samples, next samples, finished pixels */
+    SOLHIP_KERNEL_SRV_EXTEND = 13,  /* render server: all live jobs' rays, shadow rays included */
+    SOLHIP_KERNEL_SRV_SHADE = 14,   /* render server: shading, next samples, finished pixels */
+    SOLHIP_KERNEL_SRV_SHADOW = 15,  /* render server: shadow rays (their count; timed with SRV_EXTEND) */
+    SOLHIP_KERNEL_SRV_RETIRE = 16,  /* none: finished samples are part of SRV_SHADE */
     SOLHIP_KERNEL_COUNT = 17
 };
 #define SOLHIP_PROFILE_TIME   0x1u  /* hipEvents around every launch, on the launch stream */

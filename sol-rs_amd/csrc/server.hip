@@ -2,21 +2,30 @@
 // and sample count traced by one wavefront.
 //
 // Device state is a pool of path slots (one per pixel of every running job),
-// two extension queues, a shadow queue and a retire list.  One step is
+// two extension queues, a shadow queue and a list of finished slots.  One step is
 //
-//   extend  closest hits of every queued ray, each against its job's scene
-//   shade   shade_vertex (the same code as the per-frame wavefront): next
-//           ray, shadow ray, or the path's sample ends (-> retire list)
-//   shadow  any-hit tests; unoccluded contributions join the path radiance
-//   retire  the ended sample joins the pixel sum; the pixel's next sample
-//           starts in the same slot (its RNG runs on, as in pathtrace.rgen's
-//           sample loop) or, after the last sample, the pixel is accumulated
-//           into the job's image and counted done
+//   trace  closest hits of every queued ray and the last step's shadow rays
+//          (unoccluded contributions join the path radiance), each against its
+//          job's scene
+//   shade  shade_vertex (the same code as the per-frame wavefront): next ray,
+//          shadow ray, or the path's sample ends.  The slot then starts its next
+//          sample at once (its RNG runs on, as in pathtrace.rgen's sample loop);
+//          the ended sample's radiance stays in the slot until its first shade of the next
+//          step, when its last shadow ray is answered, and joins the pixel sum
+//          there.  A slot without a next sample goes to the finished list: a step
+//          later its pixel is accumulated into the job's image and counted done.
 //
 // so per pixel the arithmetic and random draws are those of the per-frame
 // wavefront, in the same order: a job's image is bit-identical to a
 // solhip_trace of the same program.  Admission is first-come first-served
-// into free slot ranges; the host polls per-job done counters between steps.
+// into free slot ranges; the trace kernel writes the per-job done counters to pinned memory,
+// where the host reads a step's while the next one runs.
+//
+// A step of four kernels (extend, shade, shadow, retire) and a copy of the counters
+// that the host waited for took 90 steps of a burst of 8 jobs 21.2 ms: 130 us of
+// traversal and 25 of shading each, 55 us in retire, whose lanes counted pixels
+// one atomic each on 8 addresses (15 ns apiece), 35 us between launches.  Now 13.2 ms, a
+// step 110 us of trace and 28 of shade at the mean.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -40,17 +49,15 @@ namespace {
 
 constexpr uint32_t kSrvBlock = 64;
 
-// register budget of the traversal kernels: waves per SIMD they must fit
-// BLAS exits restore the world ray's inverse direction from the ray state
-// (trav_step's WINV), with a budget of 4 waves per SIMD for its registers:
-// C3 capacity 12.04 -> 12.09 jobs/s, p50 at half load 130 -> 122 ms
-#ifndef SOLHIP_SRV_WINV
-#define SOLHIP_SRV_WINV true
-#endif
+// register budget of the trace kernel: waves per SIMD it must fit (88 to 94
+// VGPRs; a burst of 8 jobs takes 13.34, 13.18, 14.7 ms with 4, 5, 6)
 #ifndef SOLHIP_SRV_WAVES
-#define SOLHIP_SRV_WAVES 4
+#define SOLHIP_SRV_WAVES 5
 #endif
 #define SOLHIP_SRV_OCCUPANCY __attribute__((amdgpu_waves_per_eu(SOLHIP_SRV_WAVES)))
+// words between two counters: atomics on one cache line are served one after
+// the other, whichever words they meet (shade 79 us of a full step, 46 with a line each)
+constexpr uint32_t kCount = 32;
 constexpr uint32_t kMaxJobs = 256;   // job index lives in 8 bits of the slot meta word
 
 // per-job constants (device array, one entry per running-job index)
@@ -64,7 +71,7 @@ struct JobDev {
     uint32_t nlights;
     float total;
     uint32_t W, H, frame, spp, max_depth, rr_start, enable_sky, nee;
-    float alpha, rmax;
+    float alpha, tmin, rmax;
     uint32_t base;      // first slot
     uint32_t streams;   // spec.sample_streams: sample s starts tea(p + s * W * H, frame)
     uint32_t lanes;     // slots per pixel (per-sample streams): slot base + j * npix + p runs samples j, j + lanes, ...
@@ -80,10 +87,14 @@ struct SrvArgs {
     QHit *hits;
     QRay *sq;
     float4 *scontrib;
-    uint32_t *retire;
-    uint32_t *counts;     // [0], [1] extension queues, [2] shadow queue, [3] retire list
-    uint32_t *heads;      // partitioned fetch heads: extend, then shadow (kFetchWords each)
+    uint32_t *finished;   // max_slots words: step parity 0 fills it from the front, 1 from the back
+    // counters kCount words apart, by step parity: 0, 1 extension queues, 2, 3 shadow rays, 4, 5 finished slots
+    uint32_t *counts;
+    uint32_t *heads;      // fetch heads of the trace kernel
     uint32_t *done;       // finished pixels per job index
+    uint32_t *done_host;  // pinned: the done counters at the start of a step, by its parity
+    uint32_t max_slots, max_jobs;
+    uint32_t stack;       // stack entries per lane, the step traversal's two extra ones included
     Counters *counters;
 };
 
@@ -100,12 +111,16 @@ __device__ __forceinline__ uint32_t srv_wave_append(uint32_t *counter, bool pred
     return base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
 }
 
-// shade and retire run blocks of kSrvShadeWaves waves and append to the
-// queues once per block: three appends per pass over one counter each for
-// all rays of every job made the per-wave atomics on those few addresses the
-// largest cost of a step
+// The shade kernel runs blocks of kSrvShadeWaves waves and appends to the
+// queues once per block: per-wave atomics on the few counter addresses, for
+// all rays of every job, were the largest cost of a step (a burst takes 13.4, 13.4,
+// 13.9 ms with 4, 8, 16 waves).
 constexpr uint32_t kSrvShadeWaves = 8;
 constexpr uint32_t kSrvShadeBlock = 64 * kSrvShadeWaves;
+
+// bit of a slot's st1.w: its radiance is the ended sample's, not yet in the pixel sum
+constexpr uint32_t kEnded = 0x80000000u;
+constexpr uint32_t kStart = 1u << 16;   // st1.w of a new sample: depth 0, emission counts
 
 // pathtrace.rgen:35 for this job's camera
 __device__ __forceinline__ float job_tmin(const JobDev &J)
@@ -124,7 +139,7 @@ __device__ __forceinline__ QRay start_sample(const JobDev &J, uint32_t slot, uin
     V3 o, d;
     camera_ray(J.cam.view_inverse, J.cam.projection_inverse, x, y, J.W, J.H, jx, jy, o, d);
     s0 = make_float4(1.0f, 1.0f, 1.0f, as_f(rng));
-    s1 = make_float4(0.0f, 0.0f, 0.0f, as_f(1u << 16));
+    s1 = make_float4(0.0f, 0.0f, 0.0f, as_f(kStart));
     QRay r;
     r.ox = o.x;
     r.oy = o.y;
@@ -140,6 +155,7 @@ __device__ __forceinline__ QRay start_sample(const JobDev &J, uint32_t slot, uin
 __global__ void k_srv_set_job(JobDev *jobs, uint32_t *done, uint32_t j, JobDev v)
 {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
+        v.tmin = job_tmin(v);
         jobs[j] = v;
         done[j] = 0;
     }
@@ -174,25 +190,40 @@ __global__ void k_srv_admit(SrvArgs A, uint32_t j, uint32_t cur, uint32_t nslots
         }
         A.pmeta[slot] = j | (ln << 8);
     }
-    const uint32_t at = srv_wave_append(A.counts + cur, valid);
+    const uint32_t at = srv_wave_append(A.counts + cur * kCount, valid);
     if (valid) A.q[cur][at] = r;
 }
 
-// extension / shadow rays of all running jobs, each against its job's scene
-// through the resumable traversal; a lane takes new slots once at least 16
-// lanes of its wave are idle
-template <bool ANY>
-__device__ __forceinline__ void srv_trace(const SrvArgs &A, const QRay *q, uint32_t cnt, uint32_t *heads, int kernel)
+// One step's rays of all running jobs, each against its job's scene, through
+// the resumable traversal: the extension queue, then the shadow rays that the
+// last step's shading queued.  A lane takes a new ray once at least 16 lanes
+// of its wave are idle.  Both kinds in one launch: a launch of either lasts as
+// long as its slowest ray, and the shadow rays fill that time.  MODE: the traversal
+// form that every running job's scene has, or the general one.
+template <int MODE>
+__global__ void __launch_bounds__(kSrvBlock) SOLHIP_SRV_OCCUPANCY k_srv_trace(SrvArgs A, uint32_t cur)
 {
     extern __shared__ uint2 stack[];
-    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t cnt = A.counts[cur * kCount], shadows = A.counts[(2 + (cur ^ 1u)) * kCount], lane = threadIdx.x;
+    if (blockIdx.x == 0) {
+        for (uint32_t j = lane; j < A.max_jobs; j += kSrvBlock) A.done_host[cur * A.max_jobs + j] = A.done[j];
+        if (lane == 0) {
+            // filled by this step's shading; last read a step ago
+            A.counts[(cur ^ 1u) * kCount] = 0;
+            A.counts[(2 + cur) * kCount] = 0;
+            A.counts[(4 + cur) * kCount] = 0;
+            atomicAdd(&A.counters[SOLHIP_KERNEL_SRV_EXTEND].rays, (unsigned long long)cnt);
+            atomicAdd(&A.counters[SOLHIP_KERNEL_SRV_SHADOW].rays, (unsigned long long)shadows);
+        }
+    }
     TravCounts tc{0, 0, 0, false};
     TravState st;
     SceneView sv;
+    sv.stack_depth = A.stack;
     bool has = false;
     uint32_t idx = 0, path = 0;
     PartFetch pf;
-    pf.init(heads, cnt);
+    pf.init(A.heads, cnt + shadows);
     while (true) {
         const uint64_t idle = __ballot(!has);
         const uint32_t nidle = (uint32_t)__popcll(idle);
@@ -202,21 +233,24 @@ __device__ __forceinline__ void srv_trace(const SrvArgs &A, const QRay *q, uint3
             if (!has) {
                 const uint32_t my = base + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
                 if (my < end) {
-                    const QRay r = q[my];
+                    const bool any = my >= cnt;
+                    idx = any ? my - cnt : my;
+                    const QRay r = any ? A.sq[idx] : A.q[cur][idx];
                     const JobDev &J = A.jobs[A.pmeta[r.path] & 0xFFu];
                     sv = J.sv;
-                    sv.stack_depth += 2;   // the step traversal's two extra entries
-                    trav_init(st, sv, v3(r.ox, r.oy, r.oz), v3(r.dx, r.dy, r.dz), job_tmin(J), r.tmax);
-                    idx = my;
+                    sv.stack_depth = A.stack;
+                    trav_init<MODE, false>(st, sv, v3(r.ox, r.oy, r.oz), v3(r.dx, r.dy, r.dz), J.tmin, r.tmax, 0xFFu, tc);
+                    st.any = any;
                     path = r.path;
                     has = true;
                 }
             }
         }
         if (__ballot(has) == 0 && pf.exhausted) break;
-        if (has && trav_step<ANY, false, SOLHIP_SRV_WINV>(st, sv, 0xFFu, stack + threadIdx.x, kSrvBlock, tc)) {
+        if (has &&
+            trav_step<kAnyOfRay, false, true, MODE>(st, sv, 0xFFu, stack + threadIdx.x, kSrvBlock, tc)) {
             const Hit h = trav_result(st);
-            if (!ANY) {
+            if (!st.any) {
                 QHit out;
                 out.t = h.t;
                 out.u = h.u;
@@ -235,52 +269,101 @@ __device__ __forceinline__ void srv_trace(const SrvArgs &A, const QRay *q, uint3
             has = false;
         }
     }
-    count_known<false>(A.counters + kernel, cnt, tc);
+    count_fetches<false>(A.counters + SOLHIP_KERNEL_SRV_EXTEND, tc);
 }
 
-__global__ void __launch_bounds__(kSrvBlock) SOLHIP_SRV_OCCUPANCY k_srv_extend(SrvArgs A,
-                                                                                                  uint32_t cur)
+// the ended sample of radiance s1 joins its slot's sum
+__device__ __forceinline__ void add_sample(const SrvArgs &A, const JobDev &J, uint32_t slot, float4 s1)
 {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        // filled by this step's shade / retire; last read a step ago
-        A.counts[cur ^ 1u] = 0;
-        A.counts[2] = 0;
-        A.counts[3] = 0;
+    if (J.streams) {
+        FixSum fs = A.fsum[slot];
+        fix_add(fs, s1.x, s1.y, s1.z);
+        // field by field: lane 0's count is only ever changed atomically
+        A.fsum[slot].c[0] = fs.c[0];
+        A.fsum[slot].c[1] = fs.c[1];
+        A.fsum[slot].c[2] = fs.c[2];
+        A.fsum[slot].bad = fs.bad;
+    } else {
+        const float4 ps = A.psum[slot];
+        A.psum[slot] = make_float4(ps.x + s1.x, ps.y + s1.y, ps.z + s1.z, 0.0f);
     }
-    srv_trace<false>(A, A.q[cur], A.counts[cur], A.heads, SOLHIP_KERNEL_SRV_EXTEND);
 }
 
-__global__ void __launch_bounds__(kSrvBlock) SOLHIP_SRV_OCCUPANCY k_srv_shadow(SrvArgs A)
+// A slot's last sample has ended: it joins the sum; the pixel, once all its
+// slots are there, is accumulated into the image.  True where it was.
+__device__ __forceinline__ bool finish_slot(const SrvArgs &A, const JobDev &J, uint32_t slot)
 {
-    srv_trace<true>(A, A.sq, A.counts[2], A.heads + kFetchWords, SOLHIP_KERNEL_SRV_SHADOW);
+    const uint32_t k = slot - J.base, ln = k / J.npix, p = k - ln * J.npix;
+    add_sample(A, J, slot, A.st1[slot]);
+    float pc0, pc1, pc2;
+    bool bad = false;
+    if (J.streams) {
+        // this lane of the pixel is done; the pixel's last lane (counted on
+        // lane 0's record) adds all of them up
+        if (J.lanes > 1) {
+            __threadfence();
+            if (atomicAdd(&A.fsum[J.base + p].count, 1u) != J.lanes - 1u) return false;
+            __threadfence();
+        }
+        FixSum fs = A.fsum[slot];
+        for (uint32_t l = 0; l < J.lanes; ++l)
+            if (l != ln) fix_merge(fs, A.fsum[J.base + l * J.npix + p]);
+        pc0 = fix_value(fs.c[0]);
+        pc1 = fix_value(fs.c[1]);
+        pc2 = fix_value(fs.c[2]);
+        bad = fs.bad;
+    } else {
+        const float4 ps = A.psum[slot];
+        pc0 = ps.x;
+        pc1 = ps.y;
+        pc2 = ps.z;
+    }
+    // pathtrace.rgen:88-102
+    const float inv = 1.0f / (float)J.spp;
+    const float c0 = inv * pc0, c1 = inv * pc1, c2 = inv * pc2;
+    float4 *px = J.accum + p;
+    const float4 old = *px;
+    float m0 = mixf(old.x, c0, J.alpha), m1 = mixf(old.y, c1, J.alpha), m2 = mixf(old.z, c2, J.alpha);
+    if (bad || isnan(m0) || isnan(m1) || isnan(m2) || isinf(m0) || isinf(m1) || isinf(m2)) {
+        m0 = old.x;
+        m1 = old.y;
+        m2 = old.z;
+    }
+    *px = make_float4(m0, m1, m2, 1.0f);
+    if (J.out_rgba8) {
+        const float g = 1.0f / 2.2f;
+        const uint32_t r8 = to_unorm8(powf(m0, g)), g8 = to_unorm8(powf(m1, g)), b8 = to_unorm8(powf(m2, g));
+        J.out_rgba8[p] = r8 | (g8 << 8) | (b8 << 16) | (255u << 24);
+    }
+    return true;
 }
 
-// waves per SIMD the shade kernel is compiled for (0: the compiler's choice,
-// 126 VGPRs and 4 waves; 5 fits in 96 VGPRs, but the 40-request load is
-// level with it: p50 1352-1354 vs 1356 ms)
-#ifndef SOLHIP_SRV_SHADE_WAVES
-#define SOLHIP_SRV_SHADE_WAVES 0
-#endif
-#if SOLHIP_SRV_SHADE_WAVES
-#define SOLHIP_SRV_SHADE_OCCUPANCY __attribute__((amdgpu_waves_per_eu(SOLHIP_SRV_SHADE_WAVES)))
-#else
-#define SOLHIP_SRV_SHADE_OCCUPANCY
-#endif
-
-__global__ void __launch_bounds__(kSrvShadeBlock) SOLHIP_SRV_SHADE_OCCUPANCY k_srv_shade(SrvArgs A, uint32_t cur)
+// Shades the queue, then finishes the slots whose last sample ended a step ago.
+// The slots of a block that start a new sample are gathered, so that the camera code runs in
+// full waves; the block appends to all its queues at once.  118 VGPRs, 4 waves per
+// SIMD (a budget of 5 is 3 % slower).
+__global__ void __launch_bounds__(kSrvShadeBlock) k_srv_shade(SrvArgs A, uint32_t cur)
 {
-    __shared__ uint32_t lds[kSrvShadeWaves + 1];
-    const uint32_t cnt = A.counts[cur];
+    // per wave: rays that go on, shadow rays, new samples, finished slots
+    __shared__ uint32_t lds[4][kSrvShadeWaves];
+    __shared__ uint32_t base_of[4], again_slot[kSrvShadeBlock], again_rng[kSrvShadeBlock];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    if (blockIdx.x == 0) {
+        // this step's trace is complete
+        for (uint32_t k = tid; k < kFetchParts; k += blockDim.x) fetch_reset(A.heads, k);
+    }
+    const uint32_t cnt = A.counts[cur * kCount];
     const uint32_t nthreads = gridDim.x * blockDim.x;
     for (uint32_t base = blockIdx.x * blockDim.x; base < cnt; base += nthreads) {
-        const uint32_t i = base + threadIdx.x;
+        const uint32_t i = base + tid;
         ShadeOut o;
-        bool ended = false;
-        uint32_t slot = 0;
+        bool again = false, finished = false;
+        uint32_t slot = 0, rng = 0;
         if (i < cnt) {
             const QRay r = A.q[cur][i];
             slot = r.path;
-            const JobDev &J = A.jobs[A.pmeta[slot] & 0xFFu];
+            const uint32_t meta = A.pmeta[slot];
+            const JobDev &J = A.jobs[meta & 0xFFu];
             ShadeParams P;
             P.tb = J.tb;
             P.enable_sky = J.enable_sky;
@@ -292,121 +375,93 @@ __global__ void __launch_bounds__(kSrvShadeBlock) SOLHIP_SRV_SHADE_OCCUPANCY k_s
             P.nee = J.nee && J.nlights > 0 && J.total > 0.0f;
             P.rmax = J.rmax;
             float4 s0 = A.st0[slot], s1 = A.st1[slot];
+            if (as_u(s1.w) & kEnded) {
+                add_sample(A, J, slot, s1);
+                s1 = make_float4(0.0f, 0.0f, 0.0f, as_f(kStart));
+            }
             shade_vertex(P, slot, r, A.hits[i], s0, s1, o);
-            A.st0[slot] = s0;
+            if (!o.cont) {
+                const uint32_t sample = (meta >> 8) + J.lanes;   // this slot's next sample
+                again = sample < J.spp;
+                finished = !again;
+                rng = as_u(s0.w);
+                if (again) {
+                    s1.w = as_f(kEnded);
+                    A.pmeta[slot] = (meta & 0xFFu) | (sample << 8);
+                }
+            }
+            if (o.cont) A.st0[slot] = s0;
             A.st1[slot] = s1;
-            ended = !o.cont;
         }
-        const uint32_t s_next = block_append<kSrvShadeWaves>(A.counts + (cur ^ 1u), o.cont, lds);
-        if (o.cont) A.q[cur ^ 1u][s_next] = o.nr;
-        const uint32_t s_sh = block_append<kSrvShadeWaves>(A.counts + 2, o.shadow, lds);
+        const uint64_t below = (1ull << lane) - 1ull;
+        const uint64_t m0 = __ballot(o.cont), m1 = __ballot(o.shadow), m2 = __ballot(again), m3 = __ballot(finished);
+        if (lane == 0) {
+            lds[0][wave] = (uint32_t)__popcll(m0);
+            lds[1][wave] = (uint32_t)__popcll(m1);
+            lds[2][wave] = (uint32_t)__popcll(m2);
+            lds[3][wave] = (uint32_t)__popcll(m3);
+        }
+        __syncthreads();
+        if (tid < 4) {
+            uint32_t total = 0;
+            for (uint32_t w = 0; w < kSrvShadeWaves; ++w) {
+                const uint32_t c = lds[tid][w];
+                lds[tid][w] = total;
+                total += c;
+            }
+            // new samples stand behind the rays that go on, in the same queue
+            const uint32_t news = __shfl(total, 2);
+            uint32_t *counter = A.counts + (tid == 0 ? cur ^ 1u : tid == 1 ? 2 + cur : 4 + cur) * kCount;
+            const uint32_t n = tid == 0 ? total + news : total;
+            base_of[tid] = tid == 2 || n == 0 ? total : atomicAdd(counter, n);
+        }
+        __syncthreads();
+        const uint32_t nagain = base_of[2];
+        if (o.cont) A.q[cur ^ 1u][base_of[0] + nagain + lds[0][wave] + (uint32_t)__popcll(m0 & below)] = o.nr;
         if (o.shadow) {
-            A.sq[s_sh] = o.sr;
-            A.scontrib[s_sh] = o.sc;
+            const uint32_t at = base_of[1] + lds[1][wave] + (uint32_t)__popcll(m1 & below);
+            A.sq[at] = o.sr;
+            A.scontrib[at] = o.sc;
         }
-        const uint32_t s_rt = block_append<kSrvShadeWaves>(A.counts + 3, ended, lds);
-        if (ended) A.retire[s_rt] = slot;
-    }
-}
-
-__global__ void __launch_bounds__(kSrvShadeBlock) k_srv_retire(SrvArgs A, uint32_t cur)
-{
-    __shared__ uint32_t lds[kSrvShadeWaves + 1];
-    if (blockIdx.x == 0) {
-        // this step's extend and shadow are complete
-        for (uint32_t k = threadIdx.x; k < 2 * kFetchParts; k += blockDim.x) fetch_reset(A.heads, k);
-    }
-    const uint32_t cnt = A.counts[3];
-    const uint32_t nthreads = gridDim.x * blockDim.x;
-    for (uint32_t base = blockIdx.x * blockDim.x; base < cnt; base += nthreads) {
-        const uint32_t i = base + threadIdx.x;
-        bool again = false;
-        QRay r;
-        if (i < cnt) {
-            const uint32_t slot = A.retire[i];
-            const uint32_t meta = A.pmeta[slot], job = meta & 0xFFu;
-            const JobDev &J = A.jobs[job];
-            const uint32_t sample = (meta >> 8) + J.lanes;   // this slot's next sample
-            const uint32_t k = slot - J.base, ln = k / J.npix, p = k - ln * J.npix, x = p % J.W, y = p / J.W;
-            const float4 s1 = A.st1[slot];
-            float pc0 = 0.0f, pc1 = 0.0f, pc2 = 0.0f;
-            FixSum fs;
-            fix_clear(fs);
-            bool last = true;
-            if (J.streams) {
-                fs = A.fsum[slot];
-                fix_add(fs, s1.x, s1.y, s1.z);
-            } else {
-                const float4 ps = A.psum[slot];
-                pc0 = ps.x + s1.x;
-                pc1 = ps.y + s1.y;
-                pc2 = ps.z + s1.z;
-            }
-            if (sample < J.spp) {
-                if (J.streams) {
-                    A.fsum[slot].c[0] = fs.c[0];
-                    A.fsum[slot].c[1] = fs.c[1];
-                    A.fsum[slot].c[2] = fs.c[2];
-                    A.fsum[slot].bad = fs.bad;
-                } else {
-                    A.psum[slot] = make_float4(pc0, pc1, pc2, 0.0f);
-                }
-                uint32_t rng = J.streams ? tea(p + sample * J.npix, J.frame) : as_u(A.st0[slot].w);
-                float4 s0n, s1n;
-                r = start_sample(J, slot, x, y, rng, s0n, s1n);
-                A.st0[slot] = s0n;
-                A.st1[slot] = s1n;
-                A.pmeta[slot] = job | (sample << 8);
-                again = true;
-                last = false;
-            } else if (J.streams) {
-                // this lane of the pixel is done: publish its sum; the pixel's
-                // last lane (counted on lane 0's record) adds all of them up.
-                // The count is only ever changed atomically, so the partial
-                // sum is stored field by field.
-                A.fsum[slot].c[0] = fs.c[0];
-                A.fsum[slot].c[1] = fs.c[1];
-                A.fsum[slot].c[2] = fs.c[2];
-                A.fsum[slot].bad = fs.bad;
-                if (J.lanes > 1) {
-                    __threadfence();
-                    last = atomicAdd(&A.fsum[J.base + p].count, 1u) == J.lanes - 1u;
-                    if (last) {
-                        __threadfence();
-                        for (uint32_t l = 0; l < J.lanes; ++l)
-                            if (l != ln) fix_merge(fs, A.fsum[J.base + l * J.npix + p]);
-                    }
-                }
-                pc0 = fix_value(fs.c[0]);
-                pc1 = fix_value(fs.c[1]);
-                pc2 = fix_value(fs.c[2]);
-            }
-            if (!again && last) {
-                // pathtrace.rgen:88-102
-                const float inv = 1.0f / (float)J.spp;
-                const float c0 = inv * pc0, c1 = inv * pc1, c2 = inv * pc2;
-                float4 *px = J.accum + p;
-                const float4 old = *px;
-                float m0 = mixf(old.x, c0, J.alpha), m1 = mixf(old.y, c1, J.alpha), m2 = mixf(old.z, c2, J.alpha);
-                const bool bad = (J.streams && fs.bad) || isnan(m0) || isnan(m1) || isnan(m2) || isinf(m0) ||
-                                 isinf(m1) || isinf(m2);
-                if (bad) {
-                    m0 = old.x;
-                    m1 = old.y;
-                    m2 = old.z;
-                }
-                *px = make_float4(m0, m1, m2, 1.0f);
-                if (J.out_rgba8) {
-                    const float g = 1.0f / 2.2f;
-                    const uint32_t r8 = to_unorm8(powf(m0, g)), g8 = to_unorm8(powf(m1, g)),
-                                   b8 = to_unorm8(powf(m2, g));
-                    J.out_rgba8[p] = r8 | (g8 << 8) | (b8 << 16) | (255u << 24);
-                }
-                atomicAdd(A.done + job, 1u);
-            }
+        if (again) {
+            const uint32_t at = lds[2][wave] + (uint32_t)__popcll(m2 & below);
+            again_slot[at] = slot;
+            again_rng[at] = rng;
         }
-        const uint32_t at = block_append<kSrvShadeWaves>(A.counts + (cur ^ 1u), again, lds);
-        if (again) A.q[cur ^ 1u][at] = r;
+        if (finished) {
+            const uint32_t at = base_of[3] + lds[3][wave] + (uint32_t)__popcll(m3 & below);
+            A.finished[cur ? A.max_slots - 1u - at : at] = slot;
+        }
+        __syncthreads();
+        if (tid < nagain) {
+            const uint32_t sl = again_slot[tid];
+            const uint32_t meta = A.pmeta[sl];
+            const JobDev &J = A.jobs[meta & 0xFFu];
+            const uint32_t p = (sl - J.base) % J.npix;
+            uint32_t g = J.streams ? tea(p + (meta >> 8) * J.npix, J.frame) : again_rng[tid];
+            float4 s0, s1;
+            const QRay r = start_sample(J, sl, p % J.W, p / J.W, g, s0, s1);
+            A.st0[sl] = s0;
+            A.q[cur ^ 1u][base_of[0] + tid] = r;
+        }
+        __syncthreads();   // LDS is reused by the next pass
+    }
+    const uint32_t nfin = A.counts[(4 + (cur ^ 1u)) * kCount];
+    for (uint32_t base = blockIdx.x * blockDim.x; base < nfin; base += nthreads) {
+        const uint32_t i = base + tid;
+        uint32_t job = ~0u;
+        if (i < nfin) {
+            const uint32_t slot = A.finished[cur ? i : A.max_slots - 1u - i];
+            const uint32_t j = A.pmeta[slot] & 0xFFu;
+            if (finish_slot(A, A.jobs[j], slot)) job = j;
+        }
+        // finished pixels, one atomic per job and wave
+        for (uint64_t left = __ballot(job != ~0u); left;) {
+            const int first = __ffsll((unsigned long long)left) - 1;
+            const uint64_t same = __ballot(job == (uint32_t)__shfl((int)job, first)) & left;
+            if ((int)lane == first) atomicAdd(A.done + job, (uint32_t)__popcll(same));
+            left &= ~same;
+        }
     }
 }
 
@@ -429,7 +484,7 @@ double now_ms(std::chrono::steady_clock::time_point t0)
 
 // bytes of device state per path slot: st0, st1, psum (48), order-free sum
 // (32), meta (4), two extension queues (64), hits (20), shadow queue +
-// contribution (48), retire (4)
+// contribution (48), finished list (4)
 constexpr uint64_t kSlotBytes = 48 + 32 + 4 + 64 + 20 + 48 + 4;
 // slots per pixel of a job with per-sample streams when its spec leaves it
 // open: enough lanes that a lane runs about kLaneSamples samples, within
@@ -441,6 +496,7 @@ constexpr uint32_t kLaneShare = 4;
 struct SrvScene {
     SceneView sv;
     uint64_t tlas = 0, tlas_gen = 0;   // the TLAS and its generation at registration
+    bool identity = false;             // all its instances are at the identity transform
     DevTables tb;
     DevBuf light_offsets, lights;
     uint32_t nlights = 0;
@@ -454,21 +510,23 @@ struct SrvJob {
     uint32_t base = 0, npix = 0, jidx = 0;
     uint32_t lanes_max = 1;          // slots per pixel the job may use (per-sample streams)
     uint32_t lanes = 1, slots = 0;   // slots per pixel, slots of the job (lanes * npix), set at admission
+    uint64_t first_step = 0;         // the first step that traces it
 };
 
 struct Server : Obj {
     Context *cx = nullptr;
     hipStream_t stream = nullptr;
     uint32_t max_slots = 0, max_jobs = 0, max_stack = 1;
-    DevBuf jobs, st0, st1, psum, fsum, pmeta, q0, q1, hits, sq, scontrib, retire, counts, heads, done;
-    uint32_t *done_host = nullptr;   // pinned copy of the done counters
+    DevBuf jobs, st0, st1, psum, fsum, pmeta, q0, q1, hits, sq, scontrib, finished, counts, heads, done;
+    uint32_t *done_host = nullptr;   // pinned: done counters by step parity, then those of poll()
+    hipEvent_t traced[2] = {nullptr, nullptr};   // a step's trace, which writes done_host, by its parity
     std::vector<SrvScene *> scenes;
     std::map<uint64_t, SrvJob> all;
     std::deque<uint64_t> waiting;
     std::vector<uint64_t> running_by_idx;   // job id per job index (0 = free)
     std::map<uint32_t, uint32_t> free_ranges;   // start -> length
     uint64_t next_id = 1;
-    uint32_t cur = 0;
+    uint64_t steps = 0;   // steps launched; the next one's parity is that of its queue
     std::chrono::steady_clock::time_point t0;
 
     SrvArgs args() const
@@ -486,10 +544,14 @@ struct Server : Obj {
         a.hits = (QHit *)hits.ptr;
         a.sq = (QRay *)sq.ptr;
         a.scontrib = (float4 *)scontrib.ptr;
-        a.retire = (uint32_t *)retire.ptr;
+        a.finished = (uint32_t *)finished.ptr;
         a.counts = (uint32_t *)counts.ptr;
         a.heads = (uint32_t *)heads.ptr;
         a.done = (uint32_t *)done.ptr;
+        a.done_host = done_host;
+        a.max_slots = max_slots;
+        a.max_jobs = max_jobs;
+        a.stack = max_stack + 2;   // the step traversal's two extra entries
         a.counters = cx->counters;
         return a;
     }
@@ -523,7 +585,7 @@ struct Server : Obj {
     }
     void release_all()
     {
-        for (DevBuf *b : {&jobs, &st0, &st1, &psum, &fsum, &pmeta, &q0, &q1, &hits, &sq, &scontrib, &retire, &counts, &heads,
+        for (DevBuf *b : {&jobs, &st0, &st1, &psum, &fsum, &pmeta, &q0, &q1, &hits, &sq, &scontrib, &finished, &counts, &heads,
                           &done})
             b->release();
         for (SrvScene *sc : scenes) {
@@ -534,6 +596,10 @@ struct Server : Obj {
         scenes.clear();
         if (done_host) (void)hipHostFree(done_host);
         done_host = nullptr;
+        for (hipEvent_t &e : traced) {
+            if (e) (void)hipEventDestroy(e);
+            e = nullptr;
+        }
         if (stream) (void)hipStreamDestroy(stream);
         stream = nullptr;
     }
@@ -599,7 +665,7 @@ struct Server : Obj {
             Timer *timer = cx->timer_or_null();
             if (timer) timer->begin(stream, SOLHIP_KERNEL_SRV_ADMIT);
             hipLaunchKernelGGL(k_srv_admit, dim3((nslots + kSrvBlock - 1) / kSrvBlock), dim3(kSrvBlock), 0, stream,
-                               args(), jidx, cur, nslots);
+                               args(), jidx, (uint32_t)(steps & 1u), nslots);
             if (timer) timer->end(stream, SOLHIP_KERNEL_SRV_ADMIT);
             int rc = srv_status("server admit");
             if (rc) return rc;
@@ -607,55 +673,92 @@ struct Server : Obj {
             jb.base = base;
             jb.jidx = jidx;
             jb.t_admit = now_ms(t0);
+            jb.first_step = steps;
             running_by_idx[jidx] = waiting.front();
             waiting.pop_front();
         }
         return 0;
     }
 
+    // slots of the running jobs, and a traversal form that all their scenes have:
+    // one instance at the identity transform can be traversed either way
+    void running(uint64_t &slots, uint32_t &mode)
+    {
+        bool single = true, identity = true;
+        slots = 0;
+        for (uint64_t id : running_by_idx) {
+            if (!id) continue;
+            const SrvJob &jb = all[id];
+            const SrvScene *sc = scenes[jb.desc.scene];
+            slots += jb.slots;
+            single = single && sc->sv.mode == kTravSingle;
+            identity = identity && sc->identity;
+        }
+        mode = single ? kTravSingle : identity ? kTravIdentity : kTravGeneral;
+    }
+
     int step()
     {
         const SrvArgs a = args();
-        const uint32_t persist = cx->ncu * 4 * SOLHIP_SRV_WAVES;
+        const uint32_t cur = (uint32_t)(steps & 1u);
+        uint64_t slots;
+        uint32_t mode;
+        running(slots, mode);
+        // every slot has at most one extension and one shadow ray
+        const uint32_t trace_blocks = (uint32_t)std::min<uint64_t>(cx->ncu * 4 * SOLHIP_SRV_WAVES, (2 * slots + 63) / 64);
         const uint32_t shade_blocks =
-            std::min<uint32_t>((max_slots + kSrvShadeBlock - 1) / kSrvShadeBlock, cx->ncu * 4);
-        const size_t lds = (size_t)(max_stack + 2) * sizeof(uint2) * kSrvBlock;
+            (uint32_t)std::min<uint64_t>((slots + kSrvShadeBlock - 1) / kSrvShadeBlock, cx->ncu * 32 / kSrvShadeWaves);
+        const size_t lds = (size_t)a.stack * sizeof(uint2) * kSrvBlock;
         Timer *timer = cx->timer_or_null();
         auto timed = [&](int id, auto &&launch) {
             if (timer) timer->begin(stream, id);
             launch();
             if (timer) timer->end(stream, id);
         };
-        timed(SOLHIP_KERNEL_SRV_EXTEND,
-              [&] { hipLaunchKernelGGL(k_srv_extend, dim3(persist), dim3(kSrvBlock), lds, stream, a, cur); });
+        timed(SOLHIP_KERNEL_SRV_EXTEND, [&] {
+            trav_dispatch(mode, 0, [&](auto m, auto) {
+                hipLaunchKernelGGL((k_srv_trace<m.value>), dim3(trace_blocks), dim3(kSrvBlock), lds, stream, a, cur);
+            });
+        });
+        SOLHIP_HIP_CHECK(hipEventRecord(traced[cur], stream));
         timed(SOLHIP_KERNEL_SRV_SHADE,
               [&] { hipLaunchKernelGGL(k_srv_shade, dim3(shade_blocks), dim3(kSrvShadeBlock), 0, stream, a, cur); });
-        timed(SOLHIP_KERNEL_SRV_SHADOW,
-              [&] { hipLaunchKernelGGL(k_srv_shadow, dim3(persist), dim3(kSrvBlock), lds, stream, a); });
-        timed(SOLHIP_KERNEL_SRV_RETIRE,
-              [&] { hipLaunchKernelGGL(k_srv_retire, dim3(shade_blocks), dim3(kSrvShadeBlock), 0, stream, a, cur); });
-        cur ^= 1u;
+        ++steps;
         return srv_status("server step");
     }
 
-    // reads the done counters; finished jobs give back their slots
-    int poll()
+    // the jobs whose done counters, as of the start of step `at`, are full give back their slots
+    void finish_jobs(const uint32_t *counts, uint64_t at)
     {
-        SOLHIP_HIP_CHECK(hipMemcpyAsync(done_host, done.ptr, sizeof(uint32_t) * max_jobs, hipMemcpyDeviceToHost,
-                                        stream));
-        SOLHIP_HIP_CHECK(hipStreamSynchronize(stream));
         const double t = now_ms(t0);
         for (uint32_t j = 0; j < max_jobs; ++j) {
             const uint64_t id = running_by_idx[j];
             if (!id) continue;
             SrvJob &jb = all[id];
-            if (done_host[j] >= jb.npix) {
+            if (jb.first_step <= at && counts[j] >= jb.npix) {
                 jb.state = SOLHIP_JOB_DONE;
                 jb.t_done = t;
                 free_range(jb.base, jb.slots);
                 running_by_idx[j] = 0;
             }
         }
+    }
+
+    // the counters that step `at` wrote at its start
+    int poll_step(uint64_t at)
+    {
+        SOLHIP_HIP_CHECK(hipEventSynchronize(traced[at & 1u]));
+        finish_jobs(done_host + (at & 1u) * max_jobs, at);
+        return 0;
+    }
+
+    // the counters now, once all launched steps are complete
+    int poll()
+    {
+        uint32_t *now = done_host + 2 * max_jobs;
+        SOLHIP_HIP_CHECK(hipMemcpyAsync(now, done.ptr, sizeof(uint32_t) * max_jobs, hipMemcpyDeviceToHost, stream));
+        SOLHIP_HIP_CHECK(hipStreamSynchronize(stream));
+        finish_jobs(now, steps);
         return 0;
     }
     uint32_t live() const
@@ -695,19 +798,21 @@ int32_t solhip_server_create(solhip_ctx ctx, uint64_t hbm_budget, uint32_t max_j
                 sv->pmeta.reserve(n * 4) ||
                 sv->q0.reserve(n * sizeof(QRay)) || sv->q1.reserve(n * sizeof(QRay)) ||
                 sv->hits.reserve(n * sizeof(QHit)) || sv->sq.reserve(n * sizeof(QRay)) ||
-                sv->scontrib.reserve(n * 16) || sv->retire.reserve(n * 4) || sv->counts.reserve(256) ||
-                sv->heads.reserve(2ull * kFetchWords * 4) || sv->done.reserve((uint64_t)max_jobs * 4);
+                sv->scontrib.reserve(n * 16) || sv->finished.reserve(n * 4) || sv->counts.reserve(6ull * kCount * 4) ||
+                sv->heads.reserve((uint64_t)kFetchWords * 4) || sv->done.reserve((uint64_t)max_jobs * 4);
     if (!fail) fail = hipStreamCreateWithFlags(&sv->stream, hipStreamNonBlocking) != hipSuccess ||
-                      hipHostMalloc((void **)&sv->done_host, sizeof(uint32_t) * max_jobs, hipHostMallocDefault) !=
-                          hipSuccess;
+                      hipHostMalloc((void **)&sv->done_host, 3 * sizeof(uint32_t) * max_jobs, hipHostMallocDefault) !=
+                          hipSuccess ||
+                      hipEventCreateWithFlags(&sv->traced[0], hipEventDisableTiming) != hipSuccess ||
+                      hipEventCreateWithFlags(&sv->traced[1], hipEventDisableTiming) != hipSuccess;
     if (fail) {
         sv->release_all();
         delete sv;
         set_error("render server allocation failed");
         return SOLHIP_ERROR_OUT_OF_MEMORY;
     }
-    if (launch_fill(sv->stream, (uint32_t *)sv->counts.ptr, 64, 0u) ||
-        launch_fill(sv->stream, (uint32_t *)sv->heads.ptr, 2ull * kFetchWords, 0u) ||
+    if (launch_fill(sv->stream, (uint32_t *)sv->counts.ptr, 6ull * kCount, 0u) ||
+        launch_fill(sv->stream, (uint32_t *)sv->heads.ptr, (uint64_t)kFetchWords, 0u) ||
         launch_fill(sv->stream, (uint32_t *)sv->done.ptr, max_jobs, 0u) || hipStreamSynchronize(sv->stream)) {
         sv->release_all();
         delete sv;
@@ -763,6 +868,7 @@ int32_t solhip_server_scene(solhip_ctx ctx, solhip_server h, solhip_tlas th, con
     sc->sv = view_of(t);
     sc->tlas = th;
     sc->tlas_gen = t->gen;
+    sc->identity = t->identity;
     sc->tb.instances = (const solhip_scene_instance *)tables->instances_addr;
     sc->tb.vertex_table = (const uint64_t *)tables->vertex_table_addr;
     sc->tb.index_table = (const uint64_t *)tables->index_table_addr;
@@ -846,6 +952,9 @@ int32_t solhip_server_run(solhip_ctx ctx, solhip_server h, uint32_t max_steps, u
         if (jb.state == SOLHIP_JOB_DONE) continue;
         if (const int rc = scene_fresh(sv->scenes[jb.desc.scene])) return rc;
     }
+    // The host stays a step ahead of the GPU: it looks at the done counters of the
+    // step before the one that it has just launched.
+    const uint64_t begin = sv->steps;
     for (uint32_t k = 0; k < max_steps; ++k) {
         int rc = sv->admit();
         if (rc) return rc;
@@ -854,7 +963,10 @@ int32_t solhip_server_run(solhip_ctx ctx, solhip_server h, uint32_t max_steps, u
         if (!running) break;
         rc = sv->step();
         if (rc) return rc;
-        rc = sv->poll();
+        if (sv->steps >= begin + 2 && (rc = sv->poll_step(sv->steps - 2))) return rc;
+    }
+    if (sv->steps != begin) {
+        const int rc = sv->poll();
         if (rc) return rc;
     }
     if (live) *live = sv->live();
