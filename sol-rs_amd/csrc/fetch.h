@@ -75,8 +75,12 @@ struct PartFetch {
             unsigned long long *used = reinterpret_cast<unsigned long long *>(heads + kUsedUp);
             const uint64_t bit = 1ull << part;
             if ((threadIdx.x & 63u) == 0 && base < hi) atomicOr(used, bit);   // took the last item
-            const uint64_t all = log2p ? ~0ull : 1ull;
-            exhausted = (__hip_atomic_load(used, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) | bit) == all ||
+            // one lane's value for the wave: bits are set meanwhile, and lanes that saw
+            // different words would part here, some of them without the lane that claims
+            const uint64_t word = __hip_atomic_load(used, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const uint32_t low = __builtin_amdgcn_readfirstlane((uint32_t)word);
+            const uint32_t high = __builtin_amdgcn_readfirstlane((uint32_t)(word >> 32));
+            exhausted = (((uint64_t)high << 32) | low | bit) == (log2p ? ~0ull : 1ull) ||
                         ++moved >= 1u << log2p;   // or this wave has seen every one used up
             if (log2p) {
                 part = (part + 1) % kFetchParts;
