@@ -79,7 +79,7 @@ struct SceneView {
     const uint32_t *inst_meta;  // index | mask << 24
     uint32_t stack_depth;       // LDS stack entries per lane (>= TLAS + BLAS depth)
     uint32_t single;            // 1: the TLAS holds one instance; rays enter it without the root test
-    uint32_t mode;              // kTravGeneral, kTravSingle or kTravIdentity (traverse_step.h)
+    uint32_t mode;              // kTravGeneral, kTravSingle, kTravIdentity or kTravFew (traverse_step.h)
 };
 
 struct Counters {

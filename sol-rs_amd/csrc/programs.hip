@@ -263,11 +263,21 @@ int launch_ao(hipStream_t s, const ProgArgs &a, Timer *timer)
 //                      overlapping launches share nothing.
 //
 // Both are bound by VALU issue (0.58 wave-instructions per ns and SIMD set)
-// with few lanes active: 8.4 of 64 in lockstep on 32-bounce paths, 16.8 as a
-// state machine, which costs a quarter more instructions per ray.  Cornell box, 8
-// samples, 1280x720: depth 32 12.8 -> 6.5 ms, depth 8 4.5 -> 4.0, depth 4 2.6
-// against 3.1; 500x400 (fewer pixels than resident lanes): 5.7 -> 3.9, 2.04
-// against 2.09, 1.15 against 1.42; ao.* (at most 5 rays a sample), 900x600: 0.97 against 1.13.
+// with few lanes active.  The lockstep kernel runs the step traversal, whose
+// phases a wave's lanes share whatever level of the trees they are at: with
+// trace_ray's nested loops it took 1.2 (Cornell box), 1.3 (a terrain) and 2.2 times (500
+// instances) as long.  Both repeat the triangle phase (trav_step's MORE) unless the
+// scene is one instance: 32 bounces on the Cornell box 5.67 -> 5.05 ms, ao.* 810 ->
+// 720 us, ao.* on 500 instances 7.1 -> 6.5 ms; a terrain would lose 4 and 18 %.
+//
+// Milliseconds, lockstep against state machine, 8 samples where none are given:
+//   Cornell box (kTravFew)   1280x720: depth 32 10.9 / 5.05, 8 3.5 / 3.2, 4 1.97 /
+//     2.46; 500x400: depth 16 2.8 / 2.3, 8 1.57 / 1.62; 1 sample: depth 32 0.68 / 0.77;
+//     300x200, 4 samples, depth 32 1.95 / 1.65; ao.*, 900x600: 0.72 / 0.89
+//   terrain of 131K triangles  depth 4, 1280x720 6.2 / 4.3, 500x400 2.29 / 2.13, 1
+//     sample 0.34 / 0.38, 200x150 1.51 / 1.56; ao.* 2.96 / 2.01, 1.14 / 1.04, 0.72 / 0.83
+//   500 instances  depth 4, 1280x720 19.4 / 14.9, 500x400 10.7 / 9.5, 1 sample
+//     1.41 / 1.57, 200x150 8.2 / 7.2; ao.* 8.1 / 6.3, 5.0 / 4.3, 3.6 / 3.5
 // waits of 16 to 64 lanes are within 4 %; 512 threads per block 5 % better than
 // 256, 5 waves per SIMD spill (9.9 ms)
 #ifndef SOLHIP_MEGA_SHADE
@@ -280,6 +290,8 @@ int launch_ao(hipStream_t s, const ProgArgs &a, Timer *timer)
 #define SOLHIP_MEGA_BLOCK 512
 #endif
 constexpr uint32_t kMegaBlock = SOLHIP_MEGA_BLOCK;
+// trav_step's MORE (scenes of one instance: 0)
+constexpr int kLockMore = 8, kMegaMore = 4;
 
 // a lane's ray
 struct Segment {
@@ -523,7 +535,8 @@ k_pixels(ProgArgs A)
             }
         }
         if (state == kTrace &&
-            trav_step<false, COUNT, true, MODE>(st, A.sv, 0xFFu, stack + threadIdx.x, (int)blockDim.x, tc)) {
+            trav_step<false, COUNT, true, MODE, MODE == kTravSingle ? 0 : kMegaMore>(
+                st, A.sv, 0xFFu, stack + threadIdx.x, (int)blockDim.x, tc)) {
             state = kHit;
             ++rays;
         }
@@ -545,8 +558,12 @@ __global__ void __launch_bounds__(kProgBlock) k_pixels_lockstep(ProgArgs A)
             Segment r;
             p.camera(A, r);
             do {
-                const Hit h = trace_ray<false, COUNT, MODE>(A.sv, r.o, r.d, r.tmin, r.tmax, 0xFFu, stack + threadIdx.x,
-                                                            kProgBlock, tc);
+                TravState st;
+                trav_init<MODE, COUNT>(st, A.sv, r.o, r.d, r.tmin, r.tmax, 0xFFu, tc);
+                while (!trav_step<false, COUNT, true, MODE, MODE == kTravSingle ? 0 : kLockMore>(
+                    st, A.sv, 0xFFu, stack + threadIdx.x, kProgBlock, tc)) {
+                }
+                const Hit h = trav_result(st);
                 ++rays;
                 next = p.shade(A, h, r);
             } while (next == After::kRay);
@@ -575,28 +592,40 @@ static void launch_pixels(hipStream_t s, const ProgArgs &a)
 template <class Pixel>
 static void launch_lockstep(hipStream_t s, const ProgArgs &a)
 {
+    ProgArgs p = a;
+    p.sv.stack_depth += 2;   // the step traversal's two extra entries
     trav_dispatch(a.sv.mode, a.count, [&](auto mode, auto count) {
         hipLaunchKernelGGL((k_pixels_lockstep<Pixel, count.value, mode.value>), dim3(tile_count(a.W, a.H)),
-                           dim3(kProgBlock), stack_bytes(a), s, a);
+                           dim3(kProgBlock), stack_bytes(p), s, p);
     });
+}
+
+// Whether the state machine is the faster of the two (times above).  It evens
+// out what lanes take: with a second pixel per lane (twice the resident lanes) or a
+// second sample, and only where rays or paths differ enough.  In trees of a few
+// levels rays hardly do, so paths must be long: 16 bounces, or 8 with a second pixel.
+// Elsewhere rays do, but a small image has too few lanes to fill waves that wait.
+static bool machine_pays(const ProgArgs &a, uint32_t samples, uint32_t depth)
+{
+    const uint64_t pixels = (uint64_t)a.W * a.H, resident = (uint64_t)a.ncu * 4u * SOLHIP_MEGA_WAVES * 64u;
+    const bool refills = pixels >= 2 * resident;
+    if (a.sv.mode == kTravFew) return depth >= 16 ? refills || samples >= 2 : depth >= 8 && refills;
+    // long paths as before
+    return refills || (samples >= 2 && (2 * pixels >= resident || depth >= 16));
 }
 
 int launch_ao_glsl(hipStream_t s, const ProgArgs &a, Timer *timer)
 {
     if (timer) timer->begin(s, SOLHIP_KERNEL_AO_GLSL);
-    launch_lockstep<AoPixel>(s, a);
+    if (machine_pays(a, 4, 5)) launch_pixels<AoPixel>(s, a);   // ao.rgen's samples and rays
+    else launch_lockstep<AoPixel>(s, a);
     if (timer) timer->end(s, SOLHIP_KERNEL_AO_GLSL);
     return launch_status("AO-glsl");
 }
 
 int launch_pathtrace_glsl(hipStream_t s, const ProgArgs &a, Timer *timer)
 {
-    // long paths differ enough in length for the state machine to pay off, with
-    // 8 bounces only where lanes also get a second pixel (twice the resident
-    // lanes), and from 16 where a lane has a second sample or a second pixel;
-    // see the times above
-    const bool refills = (uint64_t)a.W * a.H >= 2ull * a.ncu * 4u * SOLHIP_MEGA_WAVES * 64u;
-    const bool machine = a.max_depth >= 16 ? refills || a.spp >= 2 : a.max_depth >= 8 && refills;
+    const bool machine = machine_pays(a, a.spp, a.max_depth);
     if (timer) timer->begin(s, SOLHIP_KERNEL_PATHTRACE_GLSL);
     if (machine) launch_pixels<PtPixel>(s, a);
     else launch_lockstep<PtPixel>(s, a);

@@ -28,6 +28,7 @@ inline void trav_dispatch(uint32_t mode, bool count, Launch launch)
     };
     if (mode == kTravSingle) with_mode(std::integral_constant<int, kTravSingle>{});
     else if (mode == kTravIdentity) with_mode(std::integral_constant<int, kTravIdentity>{});
+    else if (mode == kTravFew) with_mode(std::integral_constant<int, kTravFew>{});
     else with_mode(std::integral_constant<int, kTravGeneral>{});
 }
 

@@ -250,8 +250,9 @@ SOLHIP_HD void intersect_node(const uint4 w0, const uint4 w1, const uint4 w2, co
 }
 
 // forms of a scene (SceneView::mode): any; one instance; every instance at the
-// identity transform
-constexpr int kTravGeneral = 0, kTravSingle = 1, kTravIdentity = 2;
+// identity transform; the same in trees of a few levels
+constexpr int kTravGeneral = 0, kTravSingle = 1, kTravIdentity = 2, kTravFew = 3;
+constexpr uint32_t kFewLevels = 4;   // TLAS and BLAS levels together, as SceneView::stack_depth counts them
 
 // the inverse that inverse3x4 gives the identity (its translation is -0)
 constexpr float kIdentityInverse[12] = {1.0f, 0.0f, 0.0f, -0.0f, 0.0f, 1.0f, 0.0f, -0.0f, 0.0f, 0.0f, 1.0f, -0.0f};
@@ -272,10 +273,8 @@ SOLHIP_HD ObjectRay object_ray(const float *m, V3 wo, V3 wd)
 // number of lanes sharing the array, sv.stack_depth entries per lane.  Stack
 // entries are 8-byte node groups (child_base, remaining hits in visit order |
 // imask << 8).  A BLAS is traversed by a nested loop that uses the stack
-// above the TLAS entries.  MODE: the scene's form (SceneView::mode); a single
-// instance is traced without a TLAS loop, and identity instances share one
-// object ray, its divisions made once (traverse_step.h has the same forms).
-template <bool ANY, bool COUNT, int MODE = kTravGeneral>
+// above the TLAS entries.
+template <bool ANY, bool COUNT>
 SOLHIP_HD Hit trace_ray(const SceneView sv, V3 wo, V3 wd, float tmin, float tmax, uint32_t cull, uint2 *lds,
                         int stride, TravCounts &cnt)
 {
@@ -360,29 +359,12 @@ SOLHIP_HD Hit trace_ray(const SceneView sv, V3 wo, V3 wd, float tmin, float tmax
             }
         };
 
-        if (MODE == kTravSingle) {
-            const uint32_t meta = SOLHIP_G1(sv.inst_meta)[0];
-            if (((meta >> 24) & cull) != 0u) {
-                const uint4 *ip = reinterpret_cast<const uint4 *>(sv.insts);
-                const uint4 i0 = SOLHIP_G4(ip)[0], i1 = SOLHIP_G4(ip)[1], i2 = SOLHIP_G4(ip)[2],
-                            i3 = SOLHIP_G4(ip)[3];
-                if (COUNT) cnt.insts++;
-                const uint64_t bn = ((uint64_t)i3.y << 32) | i3.x, tr = ((uint64_t)i3.w << 32) | i3.z;
-                const float m[12] = {as_f(i0.x), as_f(i0.y), as_f(i0.z), as_f(i0.w), as_f(i1.x), as_f(i1.y),
-                                     as_f(i1.z), as_f(i1.w), as_f(i2.x), as_f(i2.y), as_f(i2.z), as_f(i2.w)};
-                if (bn != 0)
-                    trace_blas(reinterpret_cast<const WideNode *>(bn), reinterpret_cast<const TriRec *>(tr),
-                               object_ray(m, wo, wd), meta & 0xFFFFFFu);
-            }
-        }
-        ObjectRay shared_ray;
-        if (MODE == kTravIdentity) shared_ray = object_ray(kIdentityInverse, wo, wd);
-        const V3 winv = MODE == kTravIdentity ? shared_ray.inv : safe_inv(wd);
+        const V3 winv = safe_inv(wd);
         const uint32_t woct = octant(wd);
         // the TLAS root, or, with one instance, its leaf (record 0) at once
         uint32_t ng_base = 0, ng_hits = sv.single ? 0u : 1u << woct, ng_imask = 1u;
         uint32_t tg_base = 0, tg_mask = sv.single ? 1u : 0u, tg_valid = 1u;
-        while (MODE != kTravSingle) {
+        while (true) {
             if (tg_mask) {
                 // instance leaf: transform the ray and trace its BLAS
                 const uint32_t k = __builtin_ctz(tg_mask);
@@ -395,13 +377,10 @@ SOLHIP_HD Hit trace_ray(const SceneView sv, V3 wo, V3 wd, float tmin, float tmax
                 if (COUNT) cnt.insts++;
                 const uint64_t bn = ((uint64_t)i3.y << 32) | i3.x, tr = ((uint64_t)i3.w << 32) | i3.z;
                 if (bn == 0) continue;
-                ObjectRay ray = shared_ray;
-                if (MODE != kTravIdentity) {
-                    const uint4 i0 = SOLHIP_G4(ip)[0], i1 = SOLHIP_G4(ip)[1], i2 = SOLHIP_G4(ip)[2];
-                    const float m[12] = {as_f(i0.x), as_f(i0.y), as_f(i0.z), as_f(i0.w), as_f(i1.x), as_f(i1.y),
-                                         as_f(i1.z), as_f(i1.w), as_f(i2.x), as_f(i2.y), as_f(i2.z), as_f(i2.w)};
-                    ray = object_ray(m, wo, wd);
-                }
+                const uint4 i0 = SOLHIP_G4(ip)[0], i1 = SOLHIP_G4(ip)[1], i2 = SOLHIP_G4(ip)[2];
+                const float m[12] = {as_f(i0.x), as_f(i0.y), as_f(i0.z), as_f(i0.w), as_f(i1.x), as_f(i1.y),
+                                     as_f(i1.z), as_f(i1.w), as_f(i2.x), as_f(i2.y), as_f(i2.z), as_f(i2.w)};
+                const ObjectRay ray = object_ray(m, wo, wd);
                 if (trace_blas(reinterpret_cast<const WideNode *>(bn), reinterpret_cast<const TriRec *>(tr), ray,
                                meta & 0xFFFFFFu))
                     break;

@@ -12,7 +12,7 @@
 // instance-leaf group, tagged in bit 31), so closest and first hits equal
 // trace_ray's bit for bit.
 //
-// Three forms of it, by what the TLAS holds (SceneView::mode, decided when the
+// Four forms of it, by what the TLAS holds (SceneView::mode, decided when the
 // TLAS is built):
 //   kTravGeneral   any scene.
 //   kTravSingle    one instance: the ray enters it when it starts, in object space
@@ -22,12 +22,14 @@
 //                  transforms are baked into its vertices): the object ray is the same
 //                  in every instance, so it and its divisions are made once per
 //                  ray and an instance entry only switches node arrays.
+//   kTravFew       kTravIdentity in trees of at most kFewLevels levels (a room of a few
+//                  boxes), whose nodes lead to many triangles each: trav_step's MORE.
 // An instance entry is 6 divisions and a 3x4 transform for the few lanes of a
 // wave that are at one, in almost every step, and the world ray 9 registers
 // (k_trace_rays 89 -> 70 VGPRs).  One instance of 2.1M triangles: AO frame 3.25
 // -> 2.76 ms; 1.5M scattered rays 404 -> 354 us; the Cornell box's six: 16-spp
 // path-traced frame 5.5 -> 5.2 ms.
-// All three give the same hits and fetch counts.
+// All give the same hits and fetch counts.
 #pragma once
 
 #include "traverse.h"
@@ -54,7 +56,23 @@ struct TravState {
 // trav_step's ANY: closest hit, first hit, or as the ray says (TravState::any)
 constexpr int kClosest = 0, kAny = 1, kAnyOfRay = 2;
 
+constexpr int kMoreByScene = -1;   // trav_step's MORE
+
+// the form whose phases a form has
+constexpr int form_of(int form) { return form == kTravFew ? kTravIdentity : form; }
+
 constexpr uint32_t kLeafGroupTag = 0x80000000u;
+
+// at least n of the wave's active lanes say yes (the host has one lane)
+SOLHIP_HD bool lanes_vote(bool yes, int n)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    return __popcll(__ballot(yes)) >= n;
+#else
+    (void)n;
+    return yes;
+#endif
+}
 
 // transforms the world ray into an instance and readies its triangle test
 SOLHIP_HD void trav_object_ray(TravState &s, const float *m, V3 wo, V3 wd)
@@ -66,10 +84,11 @@ SOLHIP_HD void trav_object_ray(TravState &s, const float *m, V3 wo, V3 wd)
     s.wt = r.wt;
 }
 
-template <int MODE, bool COUNT>
+template <int FORM, bool COUNT>
 SOLHIP_HD void trav_init(TravState &s, const SceneView &sv, V3 wo, V3 wd, float tmin, float tmax, uint32_t cull,
                          TravCounts &cnt)
 {
+    constexpr int MODE = form_of(FORM);
     s.wo = wo;
     s.wd = wd;
     s.tmin = tmin;
@@ -157,30 +176,47 @@ SOLHIP_HD Hit trav_result(const TravState &s)
 // with it; the path tracer's extension kernel, whose rays leave a BLAS 3.9
 // times on average, 6 % faster once its register budget holds the three
 // registers (at 5 waves per SIMD they spilled and it ran 1 % slower).
-template <int ANY, bool COUNT, bool WINV = true, int MODE = kTravGeneral>
+//
+// MORE: the triangle phase is repeated while at least MORE lanes have another
+// triangle (0: never), since lanes with triangles left sit out the step's node test.  It
+// pays where a ray meets many triangles per node (trees of a node or two) or where
+// the wave waits for its slowest ray anyway; elsewhere the extra tests run for few lanes.
+// kMoreByScene: 8 in the form kTravFew, never in the others.  Cornell box: 2M
+// rays 132 -> 107 us, 1080p AO 640 -> 548, path-traced frame 3.38 -> 3.18 ms (8, 12 and 16 are
+// within 3 %).  A terrain in 16 BLASes of 32K triangles loses 2 to 4 % by the vote alone.
+template <int ANY, bool COUNT, bool WINV = true, int FORM = kTravGeneral, int MORE = kMoreByScene>
 SOLHIP_HD bool trav_step(TravState &s, const SceneView &sv, uint32_t cull, uint2 *lds, int stride, TravCounts &cnt)
 {
+    constexpr int MODE = form_of(FORM);
+    constexpr int more = MORE != kMoreByScene ? MORE : FORM == kTravFew ? 8 : 0;
     const int depth = (int)sv.stack_depth;
     // 1. one triangle
-    if ((MODE == kTravSingle || s.level) && s.tg_mask) {
-        const uint32_t k = __builtin_ctz(s.tg_mask);
-        s.tg_mask &= s.tg_mask - 1u;
-        const uint4 *tp = reinterpret_cast<const uint4 *>(s.tris + leaf_record(s.tg_base, s.tg_valid, k));
-        const uint4 a = SOLHIP_G4(tp)[0], b = SOLHIP_G4(tp)[1];
-        const uint2 c = SOLHIP_G2(tp + 2)[0];
-        const float vv[9] = {as_f(a.x), as_f(a.y), as_f(a.z), as_f(a.w), as_f(b.x),
-                             as_f(b.y), as_f(b.z), as_f(b.w), as_f(c.x)};
-        if (COUNT) cnt.tris++;
-        float t, u, v;
-        if (wt_hit(s.wt, s.tmin, s.best.t, vv, t, u, v) && better(t, s.inst, c.y, s.best)) {
-            s.best.t = t;
-            s.best.u = u;
-            s.best.v = v;
-            s.best.inst = s.inst;
-            s.best.prim = c.y;
-            if (ANY == kAny || (ANY == kAnyOfRay && s.any)) return true;
+    bool found = false;
+    while (true) {
+        const bool tri = (MODE == kTravSingle || s.level) && s.tg_mask && !found;
+        if (tri) {
+            const uint32_t k = __builtin_ctz(s.tg_mask);
+            s.tg_mask &= s.tg_mask - 1u;
+            const uint4 *tp = reinterpret_cast<const uint4 *>(s.tris + leaf_record(s.tg_base, s.tg_valid, k));
+            const uint4 a = SOLHIP_G4(tp)[0], b = SOLHIP_G4(tp)[1];
+            const uint2 c = SOLHIP_G2(tp + 2)[0];
+            const float vv[9] = {as_f(a.x), as_f(a.y), as_f(a.z), as_f(a.w), as_f(b.x),
+                                 as_f(b.y), as_f(b.z), as_f(b.w), as_f(c.x)};
+            if (COUNT) cnt.tris++;
+            float t, u, v;
+            if (wt_hit(s.wt, s.tmin, s.best.t, vv, t, u, v) && better(t, s.inst, c.y, s.best)) {
+                s.best.t = t;
+                s.best.u = u;
+                s.best.v = v;
+                s.best.inst = s.inst;
+                s.best.prim = c.y;
+                found = ANY == kAny || (ANY == kAnyOfRay && s.any);
+            }
         }
+        // the lanes' vote: uniform, so they leave the loop together
+        if (more == 0 || !lanes_vote(tri && s.tg_mask && !found, more)) break;
     }
+    if (ANY != kClosest && found) return true;
     // 2. nothing left of the last node: the next stack entry (pushed groups are
     // never empty, so one pop leads to work).  An empty stack ends the ray at
     // once, also inside a BLAS: nothing of the TLAS is pending (its work is

@@ -36,6 +36,8 @@ extern "C" void hc_trace_mode(void *h, const float *rays, uint32_t n, uint32_t a
         Hit hit;
         if (mode == kTravSingle)
             any ? run_mode<true, kTravSingle>(s, sv, r, lds, tc, hit) : run_mode<false, kTravSingle>(s, sv, r, lds, tc, hit);
+        else if (mode == kTravFew)
+            any ? run_mode<true, kTravFew>(s, sv, r, lds, tc, hit) : run_mode<false, kTravFew>(s, sv, r, lds, tc, hit);
         else if (mode == kTravIdentity)
             any ? run_mode<true, kTravIdentity>(s, sv, r, lds, tc, hit) : run_mode<false, kTravIdentity>(s, sv, r, lds, tc, hit);
         else
