@@ -267,17 +267,18 @@ int launch_ao(hipStream_t s, const ProgArgs &a, Timer *timer)
 // phases a wave's lanes share whatever level of the trees they are at: with
 // trace_ray's nested loops it took 1.2 (Cornell box), 1.3 (a terrain) and 2.2 times (500
 // instances) as long.  Both repeat the triangle phase (trav_step's MORE) unless the
-// scene is one instance: 32 bounces on the Cornell box 5.67 -> 5.05 ms, ao.* 810 ->
-// 720 us, ao.* on 500 instances 7.1 -> 6.5 ms; a terrain would lose 4 and 18 %.
+// scene is one instance: 32 bounces on the Cornell box 5.67 -> 4.9 ms, ao.* 810 ->
+// 716 us; a terrain would lose 4 and 18 %.
 //
 // Milliseconds, lockstep against state machine, 8 samples where none are given:
-//   Cornell box (kTravFew)   1280x720: depth 32 10.9 / 5.05, 8 3.5 / 3.2, 4 1.97 /
-//     2.46; 500x400: depth 16 2.8 / 2.3, 8 1.57 / 1.62; 1 sample: depth 32 0.68 / 0.77;
-//     300x200, 4 samples, depth 32 1.95 / 1.65; ao.*, 900x600: 0.72 / 0.89
+//   Cornell box (kTravFew)   1280x720: depth 32 10.9 / 4.9, 8 3.5 / 3.1, 4 1.95 /
+//     2.46; 500x400: depth 16 2.8 / 2.2, 8 1.52 / 1.62; 1 sample: depth 32 0.63 / 0.77;
+//     300x200, 4 samples, depth 32 1.95 / 1.5; ao.*, 900x600: 0.72 / 0.89
 //   terrain of 131K triangles  depth 4, 1280x720 6.2 / 4.3, 500x400 2.29 / 2.13, 1
 //     sample 0.34 / 0.38, 200x150 1.51 / 1.56; ao.* 2.96 / 2.01, 1.14 / 1.04, 0.72 / 0.83
 //   500 instances  depth 4, 1280x720 19.4 / 14.9, 500x400 10.7 / 9.5, 1 sample
-//     1.41 / 1.57, 200x150 8.2 / 7.2; ao.* 8.1 / 6.3, 5.0 / 4.3, 3.6 / 3.5
+//     1.41 / 1.57, 200x150 8.2 / 7.2; ao.* 8.1 / 6.3, 5.0 / 4.3, 3.6 / 3.5 (before the
+//     instance entry's vote; with it the state machine 13.1, 8.4, lockstep 1.2, 6.8)
 // waits of 16 to 64 lanes are within 4 %; 512 threads per block 5 % better than
 // 256, 5 waves per SIMD spill (9.9 ms)
 #ifndef SOLHIP_MEGA_SHADE
@@ -291,7 +292,7 @@ int launch_ao(hipStream_t s, const ProgArgs &a, Timer *timer)
 #endif
 constexpr uint32_t kMegaBlock = SOLHIP_MEGA_BLOCK;
 // trav_step's MORE (scenes of one instance: 0)
-constexpr int kLockMore = 8, kMegaMore = 4;
+constexpr int kMore = 4;
 
 // a lane's ray
 struct Segment {
@@ -535,7 +536,7 @@ k_pixels(ProgArgs A)
             }
         }
         if (state == kTrace &&
-            trav_step<false, COUNT, true, MODE, MODE == kTravSingle ? 0 : kMegaMore>(
+            trav_step<false, COUNT, true, MODE, MODE == kTravSingle ? 0 : kMore>(
                 st, A.sv, 0xFFu, stack + threadIdx.x, (int)blockDim.x, tc)) {
             state = kHit;
             ++rays;
@@ -560,7 +561,7 @@ __global__ void __launch_bounds__(kProgBlock) k_pixels_lockstep(ProgArgs A)
             do {
                 TravState st;
                 trav_init<MODE, COUNT>(st, A.sv, r.o, r.d, r.tmin, r.tmax, 0xFFu, tc);
-                while (!trav_step<false, COUNT, true, MODE, MODE == kTravSingle ? 0 : kLockMore>(
+                while (!trav_step<false, COUNT, true, MODE, MODE == kTravSingle ? 0 : kMore>(
                     st, A.sv, 0xFFu, stack + threadIdx.x, kProgBlock, tc)) {
                 }
                 const Hit h = trav_result(st);

@@ -248,7 +248,7 @@ __global__ void __launch_bounds__(kSrvBlock) SOLHIP_SRV_OCCUPANCY k_srv_trace(Sr
         }
         if (__ballot(has) == 0 && pf.exhausted) break;
         if (has &&
-            trav_step<kAnyOfRay, false, true, MODE, 0>(st, sv, 0xFFu, stack + threadIdx.x, kSrvBlock, tc)) {
+            trav_step<kAnyOfRay, false, true, MODE, 4>(st, sv, 0xFFu, stack + threadIdx.x, kSrvBlock, tc)) {
             const Hit h = trav_result(st);
             if (!st.any) {
                 QHit out;

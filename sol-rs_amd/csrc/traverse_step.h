@@ -63,13 +63,14 @@ constexpr int form_of(int form) { return form == kTravFew ? kTravIdentity : form
 
 constexpr uint32_t kLeafGroupTag = 0x80000000u;
 
-// at least n of the wave's active lanes say yes (the host has one lane)
-SOLHIP_HD bool lanes_vote(bool yes, int n)
+// at least one in `of` of the wave's active lanes says yes, and one at all (the host has one lane)
+SOLHIP_HD bool lanes_vote(bool yes, int of)
 {
 #ifdef __HIP_DEVICE_COMPILE__
-    return __popcll(__ballot(yes)) >= n;
+    const uint64_t y = __ballot(yes);
+    return y != 0 && __popcll(y) * of >= __popcll(__ballot(true));
 #else
-    (void)n;
+    (void)of;
     return yes;
 #endif
 }
@@ -177,18 +178,24 @@ SOLHIP_HD Hit trav_result(const TravState &s)
 // times on average, 6 % faster once its register budget holds the three
 // registers (at 5 waves per SIMD they spilled and it ran 1 % slower).
 //
-// MORE: the triangle phase is repeated while at least MORE lanes have another
-// triangle (0: never), since lanes with triangles left sit out the step's node test.  It
-// pays where a ray meets many triangles per node (trees of a node or two) or where
-// the wave waits for its slowest ray anyway; elsewhere the extra tests run for few lanes.
-// kMoreByScene: 8 in the form kTravFew, never in the others.  Cornell box: 2M
-// rays 132 -> 107 us, 1080p AO 640 -> 548, path-traced frame 3.38 -> 3.18 ms (8, 12 and 16 are
-// within 3 %).  A terrain in 16 BLASes of 32K triangles loses 2 to 4 % by the vote alone.
+// A phase costs the wave its instructions however few lanes need it, so lanes vote:
+// - An instance entry (general form: the transform, its six divisions) is taken by a few
+//   lanes in almost every step: it waits until a quarter of the active lanes want
+//   one (10,000 instances, 1080p 53.4 -> 48.1 ms; 2M rays on 500 instances 1073 -> 973 us;
+//   a half or a third or a sixth are 1 to 6 % slower; 8 lanes, not a share, hold up the last rays
+//   of a launch: 0.2M rays 355 -> 415 us).
+// - Lanes with triangles left sit out the node test, so the triangle phase is repeated
+//   while one in MORE active lanes has another triangle (0: never).  kMoreByScene: 6 in trees
+//   of a few levels (Cornell box: 2M rays 132 -> 104 us, 1080p AO 640 -> 555, path-traced
+//   frame 3.38 -> 3.1 ms; 3 to 16 within 4 %), 3 in the general form (500 instances: 0.2M rays
+//   353 -> 298 us, 2M 970 -> 911; 10,000: level), else never (terrain: 1 to 4 % slower, in one
+//   instance or in 16 of 32K triangles).
+// Which lane works when changes nothing for its ray: same visits, hits and counts.
 template <int ANY, bool COUNT, bool WINV = true, int FORM = kTravGeneral, int MORE = kMoreByScene>
 SOLHIP_HD bool trav_step(TravState &s, const SceneView &sv, uint32_t cull, uint2 *lds, int stride, TravCounts &cnt)
 {
     constexpr int MODE = form_of(FORM);
-    constexpr int more = MORE != kMoreByScene ? MORE : FORM == kTravFew ? 8 : 0;
+    constexpr int more = MORE != kMoreByScene ? MORE : FORM == kTravFew ? 6 : FORM == kTravGeneral ? 3 : 0;
     const int depth = (int)sv.stack_depth;
     // 1. one triangle
     bool found = false;
@@ -245,7 +252,8 @@ SOLHIP_HD bool trav_step(TravState &s, const SceneView &sv, uint32_t cull, uint2
         }
     }
     // 3. an instance leaf: enter its BLAS
-    if (MODE != kTravSingle && !s.level && s.tg_mask) {
+    const bool enter = MODE != kTravSingle && !s.level && s.tg_mask;
+    if ((MODE != kTravGeneral || lanes_vote(enter, 4)) && enter) {
         const uint32_t k = __builtin_ctz(s.tg_mask);
         s.tg_mask &= s.tg_mask - 1u;
         const uint32_t li = leaf_record(s.tg_base, s.tg_valid, k);
