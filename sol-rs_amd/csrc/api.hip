@@ -418,7 +418,7 @@ int trace_wavefront(Context *c, hipStream_t s, Program *p, Tlas *t, const ProgAr
     // small queues are finished path by path; not with the radiance cache
     // (queries and records hang on the bounces) nor while launches are timed
     if (!p->spec.nrc && !c->timer_or_null()) {
-        w.finish_blocks = c->ncu * wf_finish_lanes_per_cu() / 64u;
+        w.finish_blocks = c->ncu * wf_finish_lanes_per_cu(w.sv.mode) / 64u;
         w.finish_at = w.finish_blocks * 64u * (w.sv.mode == kTravGeneral ? kFinishGeneral : kFinishOther);
     }
     w.counters = c->counters;

@@ -200,7 +200,7 @@ int launch_pathtrace_finalize(hipStream_t s, const WfArgs &a, Timer *timer);
 // threads per CU that the traversal kernels' register budget keeps resident
 uint32_t wf_threads_per_cu();
 // resident lanes of the kernel that finishes small queues, per CU
-uint32_t wf_finish_lanes_per_cu();
+uint32_t wf_finish_lanes_per_cu(uint32_t mode);
 // words of WfArgs::heads per logical fetch head (its partitions' heads)
 uint32_t wf_head_words();
 // writes the frame constants through a kernel argument (no host buffer to keep alive)

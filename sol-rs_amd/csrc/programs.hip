@@ -23,17 +23,14 @@
 
 namespace solhip {
 
-// minimum waves per SIMD requested for the AO ray kernel: it is VALU-issue
-// bound, so the register budget is traded against latency hiding
-#ifndef SOLHIP_AO_WAVES
-#define SOLHIP_AO_WAVES 5
-#endif
-#define SOLHIP_AO_RAYS_OCCUPANCY __attribute__((amdgpu_waves_per_eu(SOLHIP_AO_WAVES)))
-// persistent AO rays: a wave takes new rays for its idle lanes once at least
-// this many are idle
-#ifndef SOLHIP_AO_REFILL
-#define SOLHIP_AO_REFILL 16
-#endif
+// Waves per SIMD of the AO ray kernel: it is VALU-issue bound, so registers
+// are traded against latency hiding until they spill (79 VGPRs at 6 waves; the general
+// form would spill 18).  1080p, 8 rays per pixel on 2.1M triangles: 2606, 2387, 2298, 2593 us
+// with 4 to 7 waves.
+constexpr uint32_t ao_waves(uint32_t mode) { return mode == (uint32_t)kTravGeneral ? 5u : 6u; }
+// A wave takes new rays for its idle lanes once at least this many are idle: a new ray is
+// 315 instructions, an idle lane a share of every step (2298, 2272, 2297 us at 16, 20, 24).
+constexpr uint32_t kAoRefill = 20;
 
 // ---------------------------------------------------------------------------
 // plain ray-traced AO (wavefront)
@@ -131,7 +128,7 @@ __global__ void __launch_bounds__(kPrimaryBlock) k_ao_primary(ProgArgs A)
 // leave most of a wave waiting for its slowest lane.  Ray r = (queue entry
 // r / n_ao, AO ray r % n_ao).
 template <bool ANY, bool COUNT, int MODE>
-__global__ void __launch_bounds__(kProgBlock) SOLHIP_AO_RAYS_OCCUPANCY k_ao_rays_persist(ProgArgs A)
+__global__ void __launch_bounds__(kProgBlock) __attribute__((amdgpu_waves_per_eu(ao_waves(MODE)))) k_ao_rays_persist(ProgArgs A)
 {
     extern __shared__ uint2 stack[];
     const uint32_t count = *A.qcount;
@@ -147,7 +144,7 @@ __global__ void __launch_bounds__(kProgBlock) SOLHIP_AO_RAYS_OCCUPANCY k_ao_rays
     while (true) {
         const uint64_t idle = __ballot(!has);
         const uint32_t nidle = (uint32_t)__popcll(idle);
-        if (!pf.exhausted && nidle >= (uint32_t)SOLHIP_AO_REFILL) {
+        if (!pf.exhausted && nidle >= kAoRefill) {
             uint32_t end;
             const uint32_t base = pf.claim(nidle, end);
             if (!has) {
@@ -222,8 +219,8 @@ int launch_ao(hipStream_t s, const ProgArgs &a, Timer *timer)
     ProgArgs p = a;
     p.sv.stack_depth = a.sv.stack_depth + 2;
     const size_t lds = (size_t)p.sv.stack_depth * sizeof(uint2) * kProgBlock;
-    // persistent grid: as many waves as fit (SOLHIP_AO_WAVES per SIMD, 4 SIMDs per CU)
-    const uint32_t blocks = a.ncu * 4 * SOLHIP_AO_WAVES;
+    // persistent grid: as many waves as fit on the 4 SIMDs of each CU
+    const uint32_t blocks = a.ncu * 4 * ao_waves(a.sv.mode);
     // the fetch heads start at zero (a fill kernel: no memset node in a captured graph)
     int rc = launch_fill(s, a.aoheads, (uint64_t)kFetchWords, 0u);
     if (rc) return rc;

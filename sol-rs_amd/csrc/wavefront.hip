@@ -155,17 +155,12 @@ __global__ void k_pt_fold(WfArgs A, uint32_t pass)
     A.fsum[pix] = fs;
 }
 
-// Register budget of the traversal kernels (waves per SIMD they must fit).
-// BLAS exits restore the world ray's inverse direction from the ray state
-// (trav_step's WINV), and the traversal kernels ask for 4 waves per SIMD so
-// that those registers fit: on 10,000 instances (3.9 BLAS exits per ray)
-// 1279 -> 1356 Mrays/s; the inverse at 5 waves spilled (1275), 4 waves
-// without it gave 1295
-#ifndef SOLHIP_WF_WINV
-#define SOLHIP_WF_WINV true
-#endif
+// Register budget of the traversal kernels: waves per SIMD they must fit (93
+// VGPRs, the world ray's inverse direction for BLAS exits included).  Milliseconds with
+// 4, 5, 6 waves: Cornell box 16 spp 3.18, 3.13, 3.17, 2,000 instances 9.49, 9.28,
+// 10.2, a terrain 3.56, 3.48, 3.68, 10,000 instances 48.2, 48.2, 59.4.
 #ifndef SOLHIP_WF_WAVES
-#define SOLHIP_WF_WAVES 4
+#define SOLHIP_WF_WAVES 5
 #endif
 #define SOLHIP_WF_OCCUPANCY __attribute__((amdgpu_waves_per_eu(SOLHIP_WF_WAVES)))
 
@@ -242,7 +237,7 @@ __device__ __forceinline__ void trace_queue(const WfArgs &A, const QRay *q, uint
             }
         }
         if (__ballot(has) == 0 && pf.exhausted) break;
-        if (has && trav_step<ANY, COUNT, SOLHIP_WF_WINV, MODE>(st, A.sv, 0xFFu, stack + threadIdx.x, A.block, tc)) {
+        if (has && trav_step<ANY, COUNT, true, MODE>(st, A.sv, 0xFFu, stack + threadIdx.x, A.block, tc)) {
             queue_result<ANY>(A, idx, path, trav_result(st));
             has = false;
         }
@@ -300,11 +295,13 @@ __device__ __forceinline__ ShadeParams shade_params(const WfArgs &A)
 #ifndef SOLHIP_FINISH_SHADE
 #define SOLHIP_FINISH_SHADE 16
 #endif
-#ifndef SOLHIP_FINISH_WAVES
-#define SOLHIP_FINISH_WAVES 3
-#endif
+// waves per SIMD: long rays through many instances want more of them (10,000 instances,
+// 1 sample 5.5 -> 4.65 ms with 4 instead of 3), short ones their registers (Cornell box,
+// 1 sample 0.76 -> 0.98)
+constexpr uint32_t finish_waves(uint32_t mode) { return mode == (uint32_t)kTravGeneral ? 4u : 3u; }
+
 template <bool COUNT, int MODE>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(SOLHIP_FINISH_WAVES)))
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(finish_waves(MODE))))
 k_pt_finish(WfArgs A, uint32_t b)
 {
     extern __shared__ uint2 stack[];
@@ -808,7 +805,7 @@ uint32_t wf_threads_per_cu() { return 4u * SOLHIP_WF_WAVES * 64u; }
 
 uint32_t wf_head_words() { return kFetchWords; }
 
-uint32_t wf_finish_lanes_per_cu() { return 4u * SOLHIP_FINISH_WAVES * 64u; }
+uint32_t wf_finish_lanes_per_cu(uint32_t mode) { return 4u * finish_waves(mode) * 64u; }
 
 int launch_lights_count(hipStream_t s, const DevTables &tb, const uint32_t *inst_tris, uint32_t n_inst,
                         uint32_t *offsets, Timer *timer)
