@@ -42,7 +42,7 @@ struct HostBins {
     float hi(int a, int b, int k) const { return h[a][b][k]; }
 };
 
-// binned SAH binary tree, level by level as the GPU build (k_sah_level)
+// binned SAH binary tree, level by level as the GPU build (bvh_sah.hip)
 void sah_tree(const float *pbox, uint32_t n, std::vector<uint32_t> &vals, std::vector<uint32_t> &left,
               std::vector<uint32_t> &right, std::vector<uint32_t> &rfirst, std::vector<uint32_t> &ncount)
 {
