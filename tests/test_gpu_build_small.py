@@ -1,4 +1,5 @@
-"""Morton builds around the size up to which one workgroup makes the binary tree:
+"""Morton builds around the sizes up to which one workgroup makes the binary tree,
+walks the refit's frontier and scans the radix sort's counts:
 the same node count, depth, hits and fetches as the host replay, for triangles
 and for instances."""
 import numpy as np
@@ -48,3 +49,16 @@ def test_instances(ctx, n):
     st = ctx.stats(reset=True)
     assert g.tobytes() == h.tobytes()
     assert (st.node_fetches, st.tri_fetches, st.inst_fetches, st.overflow) == tuple(int(c) for c in counts)
+
+
+@pytest.mark.parametrize("kind", ["even", "duplicates"])
+@pytest.mark.parametrize("n", [8192, 8193, 32768, 32769, 131072, 131073])
+def test_frontier_and_scan(ctx, n, kind):
+    sd = _soup(n, kind)
+    print("build", n, kind, flush=True)
+    gs = solhip.GpuScene(ctx, sd)
+    (h, counts), rays = _same(ctx, sd, 0, ctx.blas_info(gs.blas[0]), 1.5)
+    ctx.stats(reset=True)
+    g = ctx.trace_rays(gs.tlas, rays[:64], solhip.TRACE_COUNT)
+    assert ctx.stats(reset=True).overflow == 0
+    assert g.tobytes() == h[:64].tobytes()
