@@ -355,19 +355,20 @@ int trace_nrc(Context *c, hipStream_t s, Program *p, Tlas *t, WfArgs &w, Timer *
 
 // image slices of a frame when the spec leaves it open: with a stream per
 // sample and enough paths for both to fill the GPU, two slices overlap one
-// another's slowest rays; more only add launches (1, 2, 3, 4, 6 slices: 10,000
-// instances, 33M paths 58.1, 55.8, 59.7, 58.3, 63.2 ms; Cornell box, 4.2M 3.87,
-// 3.76, 4.05, 4.38, 5.5; 51K 0.50, 0.65, 0.73, 0.82, 1.20).  With one stream
-// per pixel, passes are one sample each
+// another's slowest rays; more only add launches (1, 2, 3, 4 slices: 10,000
+// instances, 33M paths 49.2, 48.2, 50.3, 49.9 ms; Cornell box, 4.2M 3.25, 3.16,
+// 3.19, 3.25; 51K 0.33, 0.47, 0.54, 0.62).  With one stream per pixel, passes are
+// one sample each
 constexpr uint32_t kDefaultSlicesStreams = 2;
 constexpr uint64_t kSlicePaths = 1ull << 20;   // paths per default slice, at least
 // a queue is finished path by path below this many rays per lane of the
 // finishing kernel: many transformed instances make long and uneven rays, whose
-// tails are worth more than the wider kernels' occupancy.  Milliseconds at 0 (never), 2, 4, 8:
-// 10,000 instances, 1080p, 16 streams 62.2, 60.1, 58.8, 58.5; 1 sample 10.5,
-// 7.8, 7.8, 6.4; 2,000 instances, 720p, 4 samples in sequence 19.4, 13.8, 12.6, 11.5; the
-// Cornell box 4.33, 4.35, 4.93, 5.14, 16 samples in sequence 13.3, 9.0, 9.0, 9.0;
-// a terrain 4.06, 4.10, 4.25, 4.29
+// tails are worth more than the wider kernels' occupancy.  Milliseconds at 0 (never), 2, 4, 8, 16:
+// 10,000 instances, 1080p, 16 streams 49.3, 48.2, 47.7, 48.0, 47.2; 1 sample 8.9, 6.5,
+// 5.9, 4.7, 4.65; 2,000 instances, 720p, 16 streams 9.1, 9.0, 9.0, 9.0, 9.6, 4 samples in
+// sequence 15.4, 11.3, 9.5, 9.5, 9.4.  At 0, 1, 2, 3, 4: the Cornell box 3.03, 3.16, 3.16,
+// 3.16, 3.16, 16 samples in sequence 6.9, 6.6, 6.0, 6.0, 6.0, 51K paths 0.47, 0.33, 0.33,
+// 0.33, 0.33; a terrain 3.54, 3.51, 3.46, 3.51, 3.50
 constexpr uint32_t kFinishGeneral = 8, kFinishOther = 2;
 // paths in flight per pass that the default samples-per-pass aims for
 constexpr uint64_t kPathsInFlight = 64ull << 20;

@@ -157,10 +157,11 @@ int launch_trace_rays(hipStream_t s, const SceneView &sv, const solhip_ray *rays
     const uint32_t resident = (simds * SOLHIP_TRACE_WAVES + 7u) & ~7u;
     // Refill pays once there are more rays than lanes, except in trees of a few
     // levels, whose rays end together anyway.  Microseconds, one ray per lane
-    // against refill: 2M rays on 131K triangles 321 / 202, on 500 instances 1692 / 1086,
-    // in the Cornell box (6 instances of 2 to 12 triangles, depth 4) 135 / 164;
-    // 0.4M rays on the triangles 98.7 / 97.5.  (2M with a counter atomic per wave,
-    // as before: 463, 2055 and 400.)
+    // against refill when the rule was set: 2M rays on 131K triangles 321 / 202, on 500
+    // instances 1692 / 1086 (195 and 911 since the phases are voted on), in the Cornell
+    // box (6 instances of 2 to 12 triangles, depth 4) 135 / 164 (105 / - now); 0.4M rays
+    // on the triangles 98.7 / 97.5.  (2M with a counter atomic per wave, as before:
+    // 463, 2055 and 400.)
     if (n > resident * 64u && sv.stack_depth > 4) {
         trav_dispatch(sv.mode, count, [&](auto mode, auto cnt) {
             if (any)
