@@ -19,9 +19,8 @@
 // activations pass from layer to layer in registers.  Products and their order
 // in k are those of X W.
 //
-// Kernels: forward (weights in registers); training (k_mlp_train: forward, loss
-// gradient, ReLU masks and weight gradients of a tile of 64 samples in one kernel,
-// per-workgroup partials); reduce + Adam.  Loss: relative L2,
+// Kernels: forward (weights in registers); training (k_mlp_backprop: forward, loss
+// gradient and back, k_mlp_wgrad: weight gradients by chunks of 1024 rows); reduce + Adam.  Loss: relative L2,
 // sum_c (p_c - t_c)^2 / (sg(p_c)^2 + 0.01) / N (Mueller et al. 2021).
 #include <hip/hip_runtime.h>
 
@@ -32,6 +31,7 @@
 #include <vector>
 
 #include "objects.h"
+#include "wave.h"
 
 namespace solhip {
 
@@ -185,80 +185,89 @@ __global__ void __launch_bounds__(kMlpBlock) k_mlp_fwd(FwdArgs A)
 }
 
 struct TrainArgs {
-    const bf16 *x;              // N x 64
-    const float4 *target;       // N targets (x, y, z, -)
-    uint32_t n;
+    const bf16 *x;              // the slab's rows, 64 wide
+    const float4 *target;       // their targets (x, y, z, -)
+    uint32_t n;                 // rows of the slab
+    float invn;                 // 1 / rows of the whole batch
     const bf16 *wt, *wb;        // forward / backward layout
-    float *partials;            // [gridDim.x][kP]: weight gradients of the workgroup's rows
-    float *loss;                // [gridDim.x]: their loss
+    bf16 *frags;                // operands of the weight gradients (below)
+    float *loss;                // [gridDim.x]: the workgroups' loss
 };
 
-// One workgroup (4 waves) per tile of 64 samples, a wave per band of 16.  The
-// weights stand in LDS in both layouts; a layer's inputs and output gradients are
-// written to LDS feature-major, where the weight gradient X^T dZ (k = samples) reads
-// its operands; its accumulators stay in registers over all of the workgroup's tiles (wave
-// w owns input features 16w .. 16w+15 of every layer).  Rows are padded to 36
-// dwords, which spreads both the 2-byte writes and the 16-byte reads over all banks.
-// Nothing but the inputs and one set of partial sums per workgroup goes
-// through memory (activations and gradients of five layers, feature-major, before).
-// 65,536 rows: a step 172 -> 51 us (this kernel 37, Adam 6); bound by the
-// latency of a tile's chain of layers with one wave per SIMD (144 KB of LDS); loading the next tile ahead costs registers
-// and 4 us.
-constexpr uint32_t kTile = 64;                 // samples
-constexpr uint32_t kRow = kTile + 8;           // row stride of every LDS matrix, in elements
+// Training in two kernels: k_mlp_backprop runs every row forward and back and
+// stores the operands of the weight gradients X^T dZ; k_mlp_wgrad sums them
+// over chunks of kChunk rows, in row order in one accumulator, and k_mlp_adam adds the
+// chunks one after the other.  FP32 sums depend on their order and training
+// carries the difference into every later weight, so the order is fixed by the rows
+// alone, not by how many workgroups there are.
+//
+// Operands, per block of 32 rows: 5 x 4 tiles of layer inputs, then 4 x 4 + 1 tiles of
+// output gradients, each 16 features x 32 rows as one wave's MFMA operand (lane
+// (r, q): feature r, rows 8q .. 8q+7, 16 B): k_mlp_wgrad reads 1 KB a
+// load, nothing twice but by the waves that share an operand.
+constexpr uint32_t kChunk = 1024;              // rows per partial sum
+constexpr uint32_t kFrag = 512;                // elements of an operand
+constexpr uint32_t kFragsX = 5 * 4, kFrags = kFragsX + 4 * 4 + 1;   // per 32 rows
+// rows whose operands are in memory at a time: 151 MB, within the last-level cache
+// (300,001 rows 160 us a step; 180 and 303 with slabs of 64 and 32 chunks, whose launches do not
+// fill the GPU)
+constexpr uint32_t kSlab = 128 * kChunk;
+constexpr uint32_t kRow = 64 + 8;              // row stride of the weights in LDS, in elements
+constexpr int kBackBlock = 1024, kBackWaves = kBackBlock / 64;
 
 struct TrainLds {
     bf16 wt[(4 * 64 + 16) * kRow];             // forward layout: row = output, 64 inputs
     bf16 wb[4 * 64 * kRow];                    // backward layout: row = input, 64 outputs
     bf16 wb4[64 * 24];                         // output layer: row = input, 16 outputs (padded to 24)
-    bf16 act[5][64 * kRow];                    // layer inputs: row = feature
-    bf16 dz[2][64 * kRow];                     // output gradients of the layer at hand: row = feature
-    float loss[4];
+    bf16 turn[kBackWaves][64 * 24];            // a wave's values of its 16 rows: row = feature
+    float loss[kBackWaves];
 };
 
-__global__ void __launch_bounds__(kMlpBlock) k_mlp_train(TrainArgs A)
+// A wave per band of 16 rows, 16 waves per workgroup (4 per SIMD: a band is a chain of
+// nine dependent layers), weights in LDS in both layouts, rows padded to 36
+// dwords.  A layer's values pass to the next in registers and, turned to
+// feature-major through the wave's own LDS, to memory: no barrier after the
+// weights are loaded.  65,536 rows 19 us, of 78 MB written.  A step of training (microseconds
+// at 1024, 65,536, 300,001 rows): 26, 41, 160; with activations and gradients written row by
+// row in three kernels, in the same order of sums, 60, 161, 490.  One kernel that kept
+// the weight gradients in registers took 18, 43, 125, but summed tiles of 64 rows by
+// workgroup: the weights after 5 steps differed by 2e-4 of their outputs.
+__global__ void __launch_bounds__(kBackBlock) k_mlp_backprop(TrainArgs A)
 {
     extern __shared__ uint4 lds_raw[];
     TrainLds &S = *reinterpret_cast<TrainLds *>(lds_raw);
     const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, q = lane >> 4, wv = tid >> 6;
     // weights: rows of 64 (8 x 16 B), padded
-    for (uint32_t i = tid; i < (4 * 64 + 16) * 8; i += kMlpBlock)
+    for (uint32_t i = tid; i < (4 * 64 + 16) * 8; i += kBackBlock)
         *reinterpret_cast<bf16x8 *>(S.wt + (i >> 3) * kRow + (i & 7u) * 8) = reinterpret_cast<const bf16x8 *>(A.wt)[i];
-    for (uint32_t i = tid; i < 4 * 64 * 8; i += kMlpBlock)
+    for (uint32_t i = tid; i < 4 * 64 * 8; i += kBackBlock)
         *reinterpret_cast<bf16x8 *>(S.wb + (i >> 3) * kRow + (i & 7u) * 8) = reinterpret_cast<const bf16x8 *>(A.wb)[i];
-    for (uint32_t i = tid; i < 64 * 2; i += kMlpBlock)
+    for (uint32_t i = tid; i < 64 * 2; i += kBackBlock)
         *reinterpret_cast<bf16x8 *>(S.wb4 + (i >> 1) * 24 + (i & 1u) * 8) =
             reinterpret_cast<const bf16x8 *>(A.wb + 4 * 4096)[i];
-    // the output layer's gradient has 16 rows, 3 of them ever written
-    for (uint32_t i = tid; i < 16 * kRow / 8; i += kMlpBlock) reinterpret_cast<bf16x8 *>(S.dz[0])[i] = zero8();
-    f32x4 gw[kHidden][4], gw4 = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int l = 0; l < kHidden; ++l)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) gw[l][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const float invn = 1.0f / (float)A.n;
     float lsum = 0.0f;
-    const uint32_t tiles = (A.n + kTile - 1) / kTile, s = wv * 16 + r;   // this lane's sample within a tile
-    // a tile's D-layout values (features 16 nt + 4q + i of sample s) into a feature-major matrix
-    auto put = [&](bf16 *m, int nt, bf16x4 v) {
+    bf16 *T = S.turn[wv];
+    // D-layout values (features 16 nt + 4q + i of row r of the band) into feature-major rows
+    auto put = [&](int nt, bf16x4 v) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) m[(nt * 16 + 4 * q + i) * kRow + s] = v[i];
+        for (int i = 0; i < 4; ++i) T[(nt * 16 + 4 * q + i) * 24 + r] = v[i];
     };
-    // weight gradient tiles of M-tile wv: X^T (rows = inputs) times dZ (rows = outputs), k = the tile's samples
-    auto accumulate = [&](const bf16 *x, const bf16 *d, f32x4 *acc, int ntiles) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const bf16x8 a = *reinterpret_cast<const bf16x8 *>(x + (wv * 16 + r) * kRow + 32 * h + 8 * q);
-#pragma unroll
-            for (int t = 0; t < ntiles; ++t) {
-                const bf16x8 b = *reinterpret_cast<const bf16x8 *>(d + (t * 16 + r) * kRow + 32 * h + 8 * q);
-                acc[t] = mfma(a, b, acc[t]);
-            }
-        }
-    };
+    // features 32 p + lane % 32: 8 rows a lane, 2 x 512 B a wave, as the band's half of two operands
+    const uint32_t feat = ((lane >> 5) << 4) + r, half = (lane >> 4) & 1u;
     __syncthreads();
-    for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        const uint32_t row = tile * kTile + s;
+    const uint32_t bands = (A.n + 31) / 32 * 2;   // whole blocks of 32 rows: rows from n on are zeros
+    for (uint32_t band = blockIdx.x * kBackWaves + wv; band < bands; band += gridDim.x * kBackWaves) {
+        bf16 *out = A.frags + (uint64_t)(band >> 1) * (kFrags * kFrag) + (2 * (band & 1u) + half) * 128 + r * 8;
+        // the turned values of `tiles` feature tiles as operands at `at`
+        auto store = [&](uint32_t at, int tiles) {
+            wave_lds_sync();
+            for (int p = 0; p < tiles; p += 2)
+                if (p + (int)(lane >> 5) < tiles)
+                    *reinterpret_cast<bf16x8 *>(out + (at + p + (lane >> 5)) * kFrag) =
+                        *reinterpret_cast<const bf16x8 *>(T + (16 * p + feat) * 24 + 8 * half);
+            wave_lds_sync();
+        };
+        const uint32_t row = band * 16 + r;
         const bool in = row < A.n;
         const bf16 *xp = A.x + (uint64_t)(in ? row : 0u) * 64 + 8 * q;
         bf16x8 x0 = in ? *reinterpret_cast<const bf16x8 *>(xp) : zero8();
@@ -266,9 +275,10 @@ __global__ void __launch_bounds__(kMlpBlock) k_mlp_train(TrainArgs A)
         const float4 tg = in && q == 0 ? A.target[row] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            S.act[0][(8 * q + j) * kRow + s] = x0[j];
-            S.act[0][(32 + 8 * q + j) * kRow + s] = x1[j];
+            T[(8 * q + j) * 24 + r] = x0[j];
+            T[(32 + 8 * q + j) * 24 + r] = x1[j];
         }
+        store(0, 4);
         // forward; bit 4 nt + i of mask[l]: the lane's value of layer l's output is positive
         uint32_t mask[kHidden];
 #pragma unroll
@@ -284,9 +294,10 @@ __global__ void __launch_bounds__(kMlpBlock) k_mlp_train(TrainArgs A)
                 t[nt] = relu4(acc);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) mk |= (float)t[nt][i] > 0.0f ? 1u << (4 * nt + i) : 0u;
-                put(S.act[l + 1], nt, t[nt]);
+                put(nt, t[nt]);
             }
             mask[l] = mk;
+            store(4 * (l + 1), 4);
             x0 = next_operand(t[0], t[1]);
             x1 = next_operand(t[2], t[3]);
         }
@@ -303,18 +314,15 @@ __global__ void __launch_bounds__(kMlpBlock) k_mlp_train(TrainArgs A)
 #pragma unroll
             for (int c = 0; c < kOut; ++c) {
                 const float den = y[c] * y[c] + 0.01f, d = y[c] - tc[c];
-                lsum += d * d / den * invn;
-                g0[c] = (bf16)(2.0f * d / den * invn);
+                lsum += d * d / den * A.invn;
+                g0[c] = (bf16)(2.0f * d / den * A.invn);
             }
         }
-        if (q == 0)
-            for (int c = 0; c < kOut; ++c) S.dz[0][c * kRow + s] = g0[c];
-        __syncthreads();   // all bands' layer inputs and output gradients
-        accumulate(S.act[4], S.dz[0], &gw4, 1);
+        put(0, bf16x4{g0[0], g0[1], g0[2], g0[3]});   // zeros but for outputs 0..2
+        store(kFragsX + 16, 1);
         // back through layer 4 (k = 16 outputs, padded to 32), then 3..1
 #pragma unroll
         for (int l = kHidden; l >= 1; --l) {
-            bf16 *dz = S.dz[(kHidden - l + 1) & 1];
             bf16x4 t[4];
 #pragma unroll
             for (int nt = 0; nt < 4; ++nt) {
@@ -329,38 +337,86 @@ __global__ void __launch_bounds__(kMlpBlock) k_mlp_train(TrainArgs A)
                 }
 #pragma unroll
                 for (int i = 0; i < 4; ++i) t[nt][i] = (mask[l - 1] >> (4 * nt + i)) & 1u ? (bf16)acc[i] : (bf16)0.0f;
-                put(dz, nt, t[nt]);
+                put(nt, t[nt]);
             }
+            store(kFragsX + 4 * (l - 1), 4);
             g0 = next_operand(t[0], t[1]);
             g1 = next_operand(t[2], t[3]);
-            __syncthreads();   // this layer's gradients; the other buffer is free again
-            accumulate(S.act[l - 1], dz, gw[l - 1], 4);
         }
-        __syncthreads();       // act and dz are rewritten by the next tile
-        // dz[0] held layer 0's gradients: rows 3..15 are zero again for the output's
-        for (uint32_t i = tid; i < 16 * kRow / 8; i += kMlpBlock) reinterpret_cast<bf16x8 *>(S.dz[0])[i] = zero8();
-        __syncthreads();
-    }
-    float *P = A.partials + (uint64_t)blockIdx.x * kP;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t k_in = wv * 16 + 4 * q + i;
-#pragma unroll
-        for (int l = 0; l < kHidden; ++l)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) P[l * 4096 + k_in * 64 + t * 16 + r] = gw[l][t][i];
-        P[16384 + k_in * 16 + r] = gw4[i];
     }
     for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off);
     if (lane == 0) S.loss[wv] = lsum;
     __syncthreads();
-    if (tid == 0) A.loss[blockIdx.x] = S.loss[0] + S.loss[1] + S.loss[2] + S.loss[3];
+    if (tid == 0) {
+        float l = 0.0f;
+        for (int w = 0; w < kBackWaves; ++w) l += S.loss[w];
+        A.loss[blockIdx.x] = l;
+    }
+}
+
+// Weight gradients of one chunk and layer: X^T (rows = inputs) times dZ (rows =
+// outputs), k = the chunk's rows in order.  Wave w: input features 16w .. 16w+15.
+// Bound by the latency of its 32 dependent blocks of 32 rows, 8 of them in flight
+// (65,536 rows 13.4 us, 15.2 with the loads where the compiler puts them).
+constexpr int kStages = 8;
+
+template <int TILES>
+__device__ __forceinline__ void wgrad(const bf16 *x, const bf16 *d, uint32_t steps, f32x4 acc[TILES])
+{
+    constexpr uint32_t stride = kFrags * kFrag;
+    uint32_t s = 0;
+    for (; s + kStages <= steps; s += kStages) {
+        bf16x8 a[kStages], b[kStages][TILES];
+#pragma unroll
+        for (int j = 0; j < kStages; ++j) {
+            a[j] = *reinterpret_cast<const bf16x8 *>(x + (uint64_t)(s + j) * stride);
+#pragma unroll
+            for (int t = 0; t < TILES; ++t)
+                b[j][t] = *reinterpret_cast<const bf16x8 *>(d + (uint64_t)(s + j) * stride + t * kFrag);
+        }
+        __builtin_amdgcn_sched_barrier(0);   // all loads first: the compiler would spread them to save registers
+#pragma unroll
+        for (int j = 0; j < kStages; ++j)
+#pragma unroll
+            for (int t = 0; t < TILES; ++t) acc[t] = mfma(a[j], b[j][t], acc[t]);
+    }
+    for (; s < steps; ++s) {
+        const bf16x8 a = *reinterpret_cast<const bf16x8 *>(x + (uint64_t)s * stride);
+#pragma unroll
+        for (int t = 0; t < TILES; ++t)
+            acc[t] = mfma(a, *reinterpret_cast<const bf16x8 *>(d + (uint64_t)s * stride + t * kFrag), acc[t]);
+    }
+}
+
+// grid (chunks of the slab, 5 layers); partials: [chunks of the slab][kP]
+__global__ void __launch_bounds__(kMlpBlock) k_mlp_wgrad(const bf16 *frags, uint32_t blocks32, float *partials)
+{
+    const uint32_t lane = threadIdx.x & 63u, r = lane & 15u, q = lane >> 4, wv = threadIdx.x >> 6;
+    const uint32_t layer = blockIdx.y, first = blockIdx.x * (kChunk / 32), steps = min(kChunk / 32, blocks32 - first);
+    const bf16 *base = frags + (uint64_t)first * (kFrags * kFrag) + lane * 8;
+    const bf16 *x = base + (4 * layer + wv) * kFrag, *d = base + (kFragsX + 4 * layer) * kFrag;
+    float *P = partials + (uint64_t)blockIdx.x * kP + layer * 4096;
+    f32x4 acc[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (layer < (uint32_t)kHidden) {
+        wgrad<4>(x, d, steps, acc);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) P[(wv * 16 + 4 * q + i) * 64 + t * 16 + r] = acc[t][i];
+    } else {
+        wgrad<1>(x, d, steps, acc);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) P[(wv * 16 + 4 * q + i) * 16 + r] = acc[0][i];
+    }
 }
 
 struct AdamArgs {
     const float *partials;
-    uint32_t nparts;
+    uint32_t nchunks;
     const float *loss_parts;
+    uint32_t nloss;
     float *loss;
     float *w, *m, *v;
     bf16 *wt, *wb;
@@ -384,23 +440,35 @@ __device__ __forceinline__ void write_bf16(bf16 *wt, bf16 *wb, uint32_t p, float
     }
 }
 
-// sums the workgroups' partial gradients (64 parameters per block, 4 threads
-// each, in fixed order) and applies Adam; block 0 also sums the loss
+// Adds the chunks' partial gradients one after the other (64 parameters per
+// block; 4 threads each fetch kAdamChunks chunks at a time into LDS, one adds) and
+// applies Adam; block 0 also sums the loss.
+constexpr uint32_t kAdamChunks = 64;
+
 __global__ void __launch_bounds__(256) k_mlp_adam(AdamArgs A)
 {
-    __shared__ float s_sum[4][64], s_loss[256];
+    __shared__ float s_part[kAdamChunks][64], s_loss[256];
     const uint32_t j = threadIdx.x & 63u, g = threadIdx.x >> 6, p = blockIdx.x * 64 + j;
-    float g0 = 0.0f;
+    float gr = 0.0f;
+    for (uint32_t c0 = 0; c0 < A.nchunks; c0 += kAdamChunks) {
+        const uint32_t m = min(kAdamChunks, A.nchunks - c0);
+#pragma unroll
+        for (uint32_t k = 0; k < kAdamChunks / 4; ++k) {
+            const uint32_t c = 4 * k + g;
+            if (c < m) s_part[c][j] = A.partials[(uint64_t)(c0 + c) * kP + p];
+        }
+        __syncthreads();
+        if (g == 0) {
 #pragma unroll 8
-    for (uint32_t c = g; c < A.nparts; c += 4) g0 += A.partials[(uint64_t)c * kP + p];
-    s_sum[g][j] = g0;
-    if (blockIdx.x == 0) {
-        float l = 0.0f;
-        for (uint32_t c = threadIdx.x; c < A.nparts; c += 256) l += A.loss_parts[c];
-        s_loss[threadIdx.x] = l;
+            for (uint32_t c = 0; c < m; ++c) gr += s_part[c][j];
+        }
+        __syncthreads();
     }
-    __syncthreads();
     if (blockIdx.x == 0) {   // block-uniform
+        float l = 0.0f;
+        for (uint32_t c = threadIdx.x; c < A.nloss; c += 256) l += A.loss_parts[c];
+        s_loss[threadIdx.x] = l;
+        __syncthreads();
         for (uint32_t h = 128; h > 0; h >>= 1) {
             if (threadIdx.x < h) s_loss[threadIdx.x] += s_loss[threadIdx.x + h];
             __syncthreads();
@@ -408,7 +476,6 @@ __global__ void __launch_bounds__(256) k_mlp_adam(AdamArgs A)
         if (threadIdx.x == 0) *A.loss = s_loss[0];
     }
     if (g != 0) return;
-    float gr = (s_sum[0][j] + s_sum[1][j]) + (s_sum[2][j] + s_sum[3][j]);
     if (padded(p)) gr = 0.0f;
     if (A.grad_out) A.grad_out[p] = gr;
     if (!A.update) return;
@@ -442,12 +509,12 @@ int mlp_status(const char *what)
 }  // namespace
 
 struct Mlp : Obj {
-    DevBuf w, m, v, wt, wb, partials, loss, loss_parts, grad;
+    DevBuf w, m, v, wt, wb, frags, partials, loss, loss_parts, grad;
     float lr = 1e-2f, b1 = 0.9f, b2 = 0.99f, eps = 1e-8f;
     uint32_t step = 0, ncu = 256;
     void release_all()
     {
-        for (DevBuf *b : {&w, &m, &v, &wt, &wb, &partials, &loss, &loss_parts, &grad}) b->release();
+        for (DevBuf *b : {&w, &m, &v, &wt, &wb, &frags, &partials, &loss, &loss_parts, &grad}) b->release();
     }
     // blocks of 4 waves that cover the bands of n rows, two per CU at most
     uint32_t forward_blocks(uint32_t n) const
@@ -469,23 +536,36 @@ struct Mlp : Obj {
     // loss and its gradient on (x, target), applied by Adam when update
     int fit(hipStream_t s, const bf16 *x, const float4 *target, uint32_t n, bool update, float *grad_host)
     {
-        // one workgroup per CU, each over several tiles
-        const uint32_t tiles = (n + kTile - 1) / kTile, blocks = std::min(tiles, ncu);
-        if (partials.reserve((uint64_t)blocks * kP * 4) || loss_parts.reserve((uint64_t)blocks * 4))
+        const uint32_t chunks = (n + kChunk - 1) / kChunk, slabs = (n + kSlab - 1) / kSlab;
+        const uint64_t block_bytes = kFrags * kFrag * sizeof(bf16), rows = std::min(n, kSlab);
+        if (partials.reserve((uint64_t)chunks * kP * 4) || frags.reserve((rows + 31) / 32 * block_bytes) ||
+            loss_parts.reserve((uint64_t)slabs * ncu * 4))
             return SOLHIP_ERROR_OUT_OF_MEMORY;
-        TrainArgs b;
-        b.x = x;
-        b.target = target;
-        b.n = n;
-        b.wt = (const bf16 *)wt.ptr;
-        b.wb = (const bf16 *)wb.ptr;
-        b.partials = (float *)partials.ptr;
-        b.loss = (float *)loss_parts.ptr;
-        hipLaunchKernelGGL(k_mlp_train, dim3(blocks), dim3(kMlpBlock), sizeof(TrainLds), s, b);
+        uint32_t nloss = 0;
+        for (uint32_t k = 0; k < slabs; ++k) {
+            const uint64_t row0 = (uint64_t)k * kSlab;
+            TrainArgs b;
+            b.x = x + row0 * 64;
+            b.target = target + row0;
+            b.n = (uint32_t)std::min<uint64_t>(kSlab, n - row0);
+            b.invn = 1.0f / (float)n;
+            b.wt = (const bf16 *)wt.ptr;
+            b.wb = (const bf16 *)wb.ptr;
+            b.frags = (bf16 *)frags.ptr;
+            b.loss = (float *)loss_parts.ptr + nloss;
+            const uint32_t blocks32 = (b.n + 31) / 32;
+            const uint32_t grid = std::min((2 * blocks32 + kBackWaves - 1) / kBackWaves, ncu);
+            hipLaunchKernelGGL(k_mlp_backprop, dim3(grid), dim3(kBackBlock), sizeof(TrainLds), s, b);
+            hipLaunchKernelGGL(k_mlp_wgrad, dim3((b.n + kChunk - 1) / kChunk, kHidden + 1), dim3(kMlpBlock), 0, s,
+                               (const bf16 *)frags.ptr, blocks32,
+                               (float *)partials.ptr + (uint64_t)k * (kSlab / kChunk) * kP);
+            nloss += grid;
+        }
         AdamArgs d;
         d.partials = (const float *)partials.ptr;
-        d.nparts = blocks;
+        d.nchunks = chunks;
         d.loss_parts = (const float *)loss_parts.ptr;
+        d.nloss = nloss;
         d.loss = (float *)loss.ptr;
         d.w = (float *)w.ptr;
         d.m = (float *)m.ptr;
@@ -582,10 +662,10 @@ Mlp *mlp_new(Context *c, uint32_t seed, float lr)
         return nullptr;
     }
     // more LDS than the 64 KiB a launch may ask for by default
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(k_mlp_train), hipFuncAttributeMaxDynamicSharedMemorySize,
+    if (hipFuncSetAttribute(reinterpret_cast<const void *>(k_mlp_backprop), hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)sizeof(TrainLds)) != hipSuccess) {
         mlp_delete(m);
-        set_error("the device does not give k_mlp_train its LDS");
+        set_error("the device does not give k_mlp_backprop its LDS");
         return nullptr;
     }
     std::vector<float> w;
