@@ -116,7 +116,7 @@ uint32_t stack_depth_of(const Tlas *t)
 
 SceneView view_of(const Tlas *t)
 {
-    SceneView v;
+    SceneView v{};
     v.stack_depth = std::min<uint32_t>(stack_depth_of(t), (uint32_t)kMaxStack);
     v.single = t->bvh.prim_count == 1 ? 1u : 0u;
     v.mode = v.single ? kTravSingle : !t->identity ? kTravGeneral : v.stack_depth <= kFewLevels ? kTravFew : kTravIdentity;

@@ -72,7 +72,8 @@ struct alignas(16) InstRec {
 };
 static_assert(sizeof(InstRec) == 64, "InstRec must be 64 bytes");
 
-// device view of a two-level scene
+// device view of a two-level scene (compared byte by byte as part of a captured
+// frame's key: no bytes outside its members)
 struct SceneView {
     const WideNode *tnodes;     // TLAS nodes (nullptr: empty TLAS)
     const InstRec *insts;       // TLAS leaf records
@@ -80,7 +81,9 @@ struct SceneView {
     uint32_t stack_depth;       // LDS stack entries per lane (>= TLAS + BLAS depth)
     uint32_t single;            // 1: the TLAS holds one instance; rays enter it without the root test
     uint32_t mode;              // kTravGeneral, kTravSingle, kTravIdentity or kTravFew (traverse_step.h)
+    uint32_t pad;               // 0
 };
+static_assert(sizeof(SceneView) == 40, "SceneView: pointers, then an even number of words");
 
 struct Counters {
     unsigned long long rays, nodes, tris, insts, overflow;
