@@ -661,7 +661,7 @@ Mlp *mlp_new(Context *c, uint32_t seed, float lr)
         set_error("mlp allocation failed");
         return nullptr;
     }
-    // more LDS than the 64 KiB a launch may ask for by default
+    // 128 KB of the 160 that a workgroup may have
     if (hipFuncSetAttribute(reinterpret_cast<const void *>(k_mlp_backprop), hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)sizeof(TrainLds)) != hipSuccess) {
         mlp_delete(m);

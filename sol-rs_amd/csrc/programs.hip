@@ -85,7 +85,7 @@ __device__ __forceinline__ void ao_camera(const ProgArgs &A, uint32_t x, uint32_
 // Primary rays: one lane per pixel, a wave per 8x8 tile, kPrimaryWaves tiles per
 // block, whose hits are appended to the AO queue with one atomic (1080p, 1, 2, 4
 // and 8 tiles: AO frame 2.42, 2.39, 2.40, 2.42 ms; with a ray-counter atomic
-// per wave beside it 2.53).
+// per wave beside it 2.53).  The stacks of a block are 66 KiB at kMaxStack levels.
 #ifndef SOLHIP_AO_PRIMARY_WAVES
 #define SOLHIP_AO_PRIMARY_WAVES 2
 #endif
@@ -576,7 +576,8 @@ static void launch_pixels(hipStream_t s, const ProgArgs &a)
 {
     ProgArgs p = a;
     p.sv.stack_depth = a.sv.stack_depth + 2;   // the step traversal's two extra entries
-    // blocks of kMegaBlock lanes, or fewer where their stacks would pass 64 KiB of LDS
+    // blocks of kMegaBlock lanes, or fewer where their stacks would pass 64 KiB, so that
+    // two of 512 lanes still share a CU's 160 KiB of LDS (which one workgroup may have)
     uint32_t block = kMegaBlock;
     while (block > 64 && (size_t)p.sv.stack_depth * sizeof(uint2) * block > 65536) block /= 2;
     const size_t lds = (size_t)p.sv.stack_depth * sizeof(uint2) * block;
