@@ -313,7 +313,7 @@ k_pt_finish(WfArgs A, uint32_t b)
     const QRay *q = A.q[b & 1];
     enum : uint32_t { kIdle, kTrace, kDone };
     uint32_t state = kIdle, path = 0, rays = 0, shadows = 0;
-    TravCounts tc{0, 0, 0, false};
+    TravCounts tc{0, 0, 0, false}, before = tc, shadow_tc = tc;   // (COUNT) before the ray in hand; shadow rays'
     TravState st;
     st.any = false;
     float4 s0, s1;
@@ -332,6 +332,13 @@ k_pt_finish(WfArgs A, uint32_t b)
             float tmax = A.rmax;
             if (state == kDone) {
                 const Hit h = trav_result(st);
+                if (COUNT && st.any) {
+                    shadow_tc.nodes += tc.nodes - before.nodes;
+                    shadow_tc.tris += tc.tris - before.tris;
+                    shadow_tc.insts += tc.insts - before.insts;
+                    before.overflow = tc.overflow;
+                    tc = before;
+                }
                 if (st.any) {
                     // the shadow ray's answer, then the next ray from the same point
                     if (h.inst == SOLHIP_MISS) {
@@ -399,6 +406,7 @@ k_pt_finish(WfArgs A, uint32_t b)
             if (go) {
                 if (st.any) ++shadows;
                 else ++rays;
+                if (COUNT) before = tc;
                 trav_init<MODE, COUNT>(st, A.sv, o, d, tmin, tmax, 0xFFu, tc);
                 state = kTrace;
             }
@@ -408,6 +416,7 @@ k_pt_finish(WfArgs A, uint32_t b)
     }
     for (int off = 32; off > 0; off >>= 1) shadows += __shfl_xor(shadows, off);
     if (lane == 0 && shadows) atomicAdd(&A.counters[SOLHIP_KERNEL_PT_SHADOW].rays, (unsigned long long)shadows);
+    if (COUNT) count_fetches<true>(A.counters + SOLHIP_KERNEL_PT_SHADOW, shadow_tc);
     count_rays<COUNT>(A.counters + SOLHIP_KERNEL_PT_EXTEND, rays, tc);
 }
 
