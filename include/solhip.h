@@ -410,7 +410,10 @@ int32_t solhip_server_scene(solhip_ctx ctx, solhip_server srv, solhip_tlas t, co
 int32_t solhip_server_submit(solhip_ctx ctx, solhip_server srv, const solhip_job_desc *job, uint64_t *job_id);
 /* runs up to max_steps wavefront steps (admitting and retiring jobs between
  * steps); returns early when nothing is queued or running; *live = jobs
- * queued or running afterwards */
+ * queued or running afterwards.  A step carries every path of the running jobs one
+ * segment further, and no step is in flight when the call returns.  The host works
+ * ahead of the GPU: within a call, a job that waits for another's slots starts
+ * three steps after those were left. */
 int32_t solhip_server_run(solhip_ctx ctx, solhip_server srv, uint32_t max_steps, uint32_t *live);
 int32_t solhip_server_job(solhip_ctx ctx, solhip_server srv, uint64_t job_id, solhip_job_status *out);
 

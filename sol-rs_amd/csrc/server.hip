@@ -199,12 +199,14 @@ __global__ void k_srv_admit(SrvArgs A, uint32_t j, uint32_t cur, uint32_t nslots
 // last step's shading queued.  A lane takes a new ray once at least 16 lanes
 // of its wave are idle.  Both kinds in one launch: a launch of either lasts as
 // long as its slowest ray, and the shadow rays fill that time.  MODE: the traversal
-// form that every running job's scene has, or the general one.
+// form that every running job's scene has, or the general one.  extend = 0: the shadow rays alone.
 template <int MODE>
-__global__ void __launch_bounds__(kSrvBlock) SOLHIP_SRV_OCCUPANCY k_srv_trace(SrvArgs A, uint32_t cur)
+__global__ void __launch_bounds__(kSrvBlock) SOLHIP_SRV_OCCUPANCY k_srv_trace(SrvArgs A, uint32_t cur,
+                                                                                    uint32_t extend)
 {
     extern __shared__ uint2 stack[];
-    const uint32_t cnt = A.counts[cur * kCount], shadows = A.counts[(2 + (cur ^ 1u)) * kCount], lane = threadIdx.x;
+    const uint32_t cnt = extend ? A.counts[cur * kCount] : 0u, lane = threadIdx.x;
+    const uint32_t shadows = A.counts[(2 + (cur ^ 1u)) * kCount];
     if (blockIdx.x == 0) {
         for (uint32_t j = lane; j < A.max_jobs; j += kSrvBlock) A.done_host[cur * A.max_jobs + j] = A.done[j];
         if (lane == 0) {
@@ -338,11 +340,11 @@ __device__ __forceinline__ bool finish_slot(const SrvArgs &A, const JobDev &J, u
     return true;
 }
 
-// Shades the queue, then finishes the slots whose last sample ended a step ago.
-// The slots of a block that start a new sample are gathered, so that the camera code runs in
+// Shades the queue (extend = 0: leaves it alone), then finishes the slots whose last
+// sample ended a step ago.  The slots of a block that start a new sample are gathered, so that the camera code runs in
 // full waves; the block appends to all its queues at once.  118 VGPRs, 4 waves per
 // SIMD (a budget of 5 is 3 % slower).
-__global__ void __launch_bounds__(kSrvShadeBlock) k_srv_shade(SrvArgs A, uint32_t cur)
+__global__ void __launch_bounds__(kSrvShadeBlock) k_srv_shade(SrvArgs A, uint32_t cur, uint32_t extend)
 {
     // per wave: rays that go on, shadow rays, new samples, finished slots
     __shared__ uint32_t lds[4][kSrvShadeWaves];
@@ -352,7 +354,7 @@ __global__ void __launch_bounds__(kSrvShadeBlock) k_srv_shade(SrvArgs A, uint32_
         // this step's trace is complete
         for (uint32_t k = tid; k < kFetchParts; k += blockDim.x) fetch_reset(A.heads, k);
     }
-    const uint32_t cnt = A.counts[cur * kCount];
+    const uint32_t cnt = extend ? A.counts[cur * kCount] : 0u;
     const uint32_t nthreads = gridDim.x * blockDim.x;
     for (uint32_t base = blockIdx.x * blockDim.x; base < cnt; base += nthreads) {
         const uint32_t i = base + tid;
@@ -697,10 +699,10 @@ struct Server : Obj {
         mode = single ? kTravSingle : identity ? kTravIdentity : kTravGeneral;
     }
 
-    int step()
+    // a step's two kernels on the queue of parity cur
+    int launch(uint32_t cur, uint32_t extend)
     {
         const SrvArgs a = args();
-        const uint32_t cur = (uint32_t)(steps & 1u);
         uint64_t slots;
         uint32_t mode;
         running(slots, mode);
@@ -717,14 +719,35 @@ struct Server : Obj {
         };
         timed(SOLHIP_KERNEL_SRV_EXTEND, [&] {
             trav_dispatch(mode, 0, [&](auto m, auto) {
-                hipLaunchKernelGGL((k_srv_trace<m.value>), dim3(trace_blocks), dim3(kSrvBlock), lds, stream, a, cur);
+                hipLaunchKernelGGL((k_srv_trace<m.value>), dim3(trace_blocks), dim3(kSrvBlock), lds, stream, a, cur,
+                                   extend);
             });
         });
-        SOLHIP_HIP_CHECK(hipEventRecord(traced[cur], stream));
-        timed(SOLHIP_KERNEL_SRV_SHADE,
-              [&] { hipLaunchKernelGGL(k_srv_shade, dim3(shade_blocks), dim3(kSrvShadeBlock), 0, stream, a, cur); });
-        ++steps;
+        if (extend) SOLHIP_HIP_CHECK(hipEventRecord(traced[cur], stream));
+        timed(SOLHIP_KERNEL_SRV_SHADE, [&] {
+            hipLaunchKernelGGL(k_srv_shade, dim3(shade_blocks), dim3(kSrvShadeBlock), 0, stream, a, cur, extend);
+        });
         return srv_status("server step");
+    }
+
+    int step()
+    {
+        const int rc = launch((uint32_t)(steps & 1u), 1u);
+        ++steps;
+        return rc;
+    }
+
+    // what the last step left for the next one besides its queue: its shadow rays
+    // are answered and the slots that ended in it finished, so that a job is done after
+    // as many steps as its longest pixel has segments
+    int settle()
+    {
+        const uint32_t next = (uint32_t)(steps & 1u), last = next ^ 1u;
+        if (std::all_of(running_by_idx.begin(), running_by_idx.end(), [](uint64_t id) { return id == 0; })) return 0;
+        int rc = launch(next, 0u);
+        if (!rc) rc = launch_fill(stream, (uint32_t *)counts.ptr + (2 + last) * kCount, 1, 0u);
+        if (!rc) rc = launch_fill(stream, (uint32_t *)counts.ptr + (4 + last) * kCount, 1, 0u);
+        return rc;
     }
 
     // the jobs whose done counters, as of the start of step `at`, are full give back their slots
@@ -955,20 +978,24 @@ int32_t solhip_server_run(solhip_ctx ctx, solhip_server h, uint32_t max_steps, u
     // The host stays a step ahead of the GPU: it looks at the done counters of the
     // step before the one that it has just launched.
     const uint64_t begin = sv->steps;
-    for (uint32_t k = 0; k < max_steps; ++k) {
-        int rc = sv->admit();
-        if (rc) return rc;
-        bool running = false;
+    bool running = false;
+    int rc = 0;
+    for (uint32_t k = 0; k < max_steps && !rc; ++k) {
+        rc = sv->admit();
+        if (rc) break;
+        running = false;
         for (uint64_t id : sv->running_by_idx) running = running || id != 0;
         if (!running) break;
         rc = sv->step();
-        if (rc) return rc;
-        if (sv->steps >= begin + 2 && (rc = sv->poll_step(sv->steps - 2))) return rc;
+        if (!rc && sv->steps >= begin + 2) rc = sv->poll_step(sv->steps - 2);
     }
+    // no step is in flight on return, with an error neither
     if (sv->steps != begin) {
-        const int rc = sv->poll();
-        if (rc) return rc;
+        if (!rc && running) rc = sv->settle();
+        const int polled = sv->poll();
+        if (!rc) rc = polled;
     }
+    if (rc) return rc;
     if (live) *live = sv->live();
     return SOLHIP_OK;
 }
