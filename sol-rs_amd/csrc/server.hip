@@ -718,10 +718,13 @@ struct Server : Obj {
             if (timer) timer->end(stream, id);
         };
         timed(SOLHIP_KERNEL_SRV_EXTEND, [&] {
-            trav_dispatch(mode, 0, [&](auto m, auto) {
+            auto go = [&](auto m) {
                 hipLaunchKernelGGL((k_srv_trace<m.value>), dim3(trace_blocks), dim3(kSrvBlock), lds, stream, a, cur,
                                    extend);
-            });
+            };
+            if (mode == kTravSingle) go(std::integral_constant<int, kTravSingle>{});
+            else if (mode == kTravIdentity) go(std::integral_constant<int, kTravIdentity>{});
+            else go(std::integral_constant<int, kTravGeneral>{});
         });
         if (extend) SOLHIP_HIP_CHECK(hipEventRecord(traced[cur], stream));
         timed(SOLHIP_KERNEL_SRV_SHADE, [&] {

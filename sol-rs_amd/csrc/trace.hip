@@ -162,14 +162,16 @@ int launch_trace_rays(hipStream_t s, const SceneView &sv, const solhip_ray *rays
     // box (6 instances of 2 to 12 triangles, depth 4) 135 / 164 (105 / - now); 0.4M rays
     // on the triangles 98.7 / 97.5.  (2M with a counter atomic per wave, as before:
     // 463, 2055 and 400.)
-    if (n > resident * 64u && sv.stack_depth > 4) {
+    if (n > resident * 64u && sv.stack_depth > kFewLevels) {
         trav_dispatch(sv.mode, count, [&](auto mode, auto cnt) {
-            if (any)
-                hipLaunchKernelGGL((k_trace_rays_persist<true, cnt.value, mode.value>), dim3(resident), block, lds, s, v,
-                                   rays, hits, n, counters);
-            else
-                hipLaunchKernelGGL((k_trace_rays_persist<false, cnt.value, mode.value>), dim3(resident), block, lds, s,
-                                   v, rays, hits, n, counters);
+            if constexpr (mode.value != kTravFew) {   // (a scene of that form has no more than kFewLevels)
+                if (any)
+                    hipLaunchKernelGGL((k_trace_rays_persist<true, cnt.value, mode.value>), dim3(resident), block, lds, s,
+                                       v, rays, hits, n, counters);
+                else
+                    hipLaunchKernelGGL((k_trace_rays_persist<false, cnt.value, mode.value>), dim3(resident), block, lds, s,
+                                       v, rays, hits, n, counters);
+            }
         });
     } else {
         // lanes per wave: as many as leave a wave for every SIMD (64 rays on
