@@ -338,7 +338,12 @@ enum {
     SOLHIP_KERNEL_SRV_RETIRE = 16,  /* none: finished samples are part of SRV_SHADE */
     SOLHIP_KERNEL_COUNT = 17
 };
-#define SOLHIP_PROFILE_TIME   0x1u  /* hipEvents around every launch, on the launch stream */
+/* SOLHIP_PROFILE_TIME: hipEvents around every launch, on the launch stream.  A frame of
+ * SOLHIP_PROG_PATHTRACE then runs bounce by bounce to its end on one stream (one image slice),
+ * each kernel under its own id; untimed, queues of a few rays per lane are finished path by
+ * path in a launch that has no id, so the last bounces' times are not those of an untimed frame.
+ * Images, ray and fetch counts are the same. */
+#define SOLHIP_PROFILE_TIME   0x1u
 #define SOLHIP_PROFILE_COUNT  0x2u  /* fetch-counting kernel variants */
 int32_t solhip_profile(solhip_ctx ctx, uint32_t flags);
 typedef struct {

@@ -363,12 +363,13 @@ constexpr uint32_t kDefaultSlicesStreams = 2;
 constexpr uint64_t kSlicePaths = 1ull << 20;   // paths per default slice, at least
 // a queue is finished path by path below this many rays per lane of the
 // finishing kernel: many transformed instances make long and uneven rays, whose
-// tails are worth more than the wider kernels' occupancy.  Milliseconds at 0 (never), 2, 4, 8, 16:
-// 10,000 instances, 1080p, 16 streams 49.3, 48.2, 47.7, 48.0, 47.2; 1 sample 8.9, 6.5,
+// tails are worth more than the wider kernels' occupancy.  Milliseconds at 0 (never), 2, 4, 8, 16,
+// frames without a rebuild of the scene: 10,000 instances, 1080p, 16 streams 49.3, 48.2, 47.7, 48.0, 47.2; 1 sample 8.9, 6.5,
 // 5.9, 4.7, 4.65; 2,000 instances, 720p, 16 streams 9.1, 9.0, 9.0, 9.0, 9.6, 4 samples in
 // sequence 15.4, 11.3, 9.5, 9.5, 9.4.  At 0, 1, 2, 3, 4: the Cornell box 3.03, 3.16, 3.16,
 // 3.16, 3.16, 16 samples in sequence 6.9, 6.6, 6.0, 6.0, 6.0, 51K paths 0.47, 0.33, 0.33,
-// 0.33, 0.33; a terrain 3.54, 3.51, 3.46, 3.51, 3.50
+// 0.33, 0.33; a terrain 3.54, 3.51, 3.46, 3.51, 3.50.  The Cornell box's 4 % with 16 streams (the
+// only loss) is the price of 13 to 30 % where queues are small from the first bounce on
 constexpr uint32_t kFinishGeneral = 8, kFinishOther = 2;
 // paths in flight per pass that the default samples-per-pass aims for
 constexpr uint64_t kPathsInFlight = 64ull << 20;

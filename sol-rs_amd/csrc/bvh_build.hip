@@ -7,14 +7,16 @@
 // Pipeline (all on the stream the caller passes):
 //   1. primitive boxes + centroid bounds   (triangles: 3 vertex fetches at the
 //      caller's stride; instances: 8 transformed corners of the BLAS root box)
+//      (2 to 5 of up to kSmallTree primitives: one workgroup, k_small_tree; with
+//      SOLHIP_BUILD_PREFER_FAST_TRACE bvh_sah.hip instead)
 //   2. 30-bit Morton codes of the centroids (10 bits per axis)
 //   3. stable LSD radix sort of (code, index), 8-bit digits: per-tile LDS
 //      histograms, one exclusive scan, per-tile stable scatter whose local
 //      ranks come from wave64 ballots (match on the 8 digit bits)
 //   4. Karras 2012 binary radix tree (index tie-break for equal codes)
 //   5. bottom-up box refit in two phases: inside each 256-leaf block with
-//      LDS flags, then across blocks from the frontier nodes with one
-//      agent-scope acq_rel flag per node
+//      LDS flags, then across blocks from the frontier nodes with one acq_rel
+//      flag per node: of one workgroup up to kCrossOne leaves, agent-scope above
 //   6. top-down collapse, one launch per level, to 8-wide nodes: a node
 //      repeatedly opens its largest-area internal child until it has 8
 //      children; children of <= leaf_max primitives become leaves, the others

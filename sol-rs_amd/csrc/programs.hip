@@ -4,7 +4,7 @@
 //                             k_ao_primary  generate + extend + shade of the
 //                                           primary rays; hits are compacted
 //                                           into the AO queue with one atomic
-//                                           per wave (ballot + mbcnt)
+//                                           per block (block_append)
 //                             k_ao_rays_persist  n_ao rays per queue entry, an
 //                                           occlusion byte each
 //                             k_ao_resolve  the bytes of a pixel into its value
@@ -25,11 +25,11 @@ namespace solhip {
 
 // Waves per SIMD of the AO ray kernel: it is VALU-issue bound, so registers
 // are traded against latency hiding until they spill (79 VGPRs at 6 waves; the general
-// form would spill 18).  1080p, 8 rays per pixel on 2.1M triangles: 2606, 2387, 2298, 2593 us
-// with 4 to 7 waves.
+// form would spill 18).  A 1080p frame, 8 rays per pixel on 2.1M triangles, frames one after
+// another (2.38 ms one by one): 2582, 2370, 2280, 2559 us with 4 to 7 waves.
 constexpr uint32_t ao_waves(uint32_t mode) { return mode == (uint32_t)kTravGeneral ? 5u : 6u; }
 // A wave takes new rays for its idle lanes once at least this many are idle: a new ray is
-// 315 instructions, an idle lane a share of every step (2298, 2272, 2297 us at 16, 20, 24).
+// 315 instructions, an idle lane a share of every step (2297, 2280, 2304 us at 16, 20, 24).
 constexpr uint32_t kAoRefill = 20;
 
 // ---------------------------------------------------------------------------

@@ -19,7 +19,8 @@
 // wavefront, in the same order: a job's image is bit-identical to a
 // solhip_trace of the same program.  Admission is first-come first-served
 // into free slot ranges; the trace kernel writes the per-job done counters to pinned memory,
-// where the host reads a step's while the next one runs.
+// where the host reads a step's while the next one runs.  A run whose steps are used up
+// ends by answering the last step's shadow rays and finishing its ended slots.
 //
 // A step of four kernels (extend, shade, shadow, retire) and a copy of the counters
 // that the host waited for took 90 steps of a burst of 8 jobs 21.2 ms: 130 us of
@@ -161,7 +162,6 @@ __global__ void k_srv_set_job(JobDev *jobs, uint32_t *done, uint32_t j, JobDev v
     }
 }
 
-// first sample of every pixel of job j, appended to queue cur (8x8 tiles)
 // the first sample of every slot of job j (lane-major, 8x8 tiles within a
 // lane), appended to queue cur; nslots = lanes * tile slots
 __global__ void k_srv_admit(SrvArgs A, uint32_t j, uint32_t cur, uint32_t nslots)

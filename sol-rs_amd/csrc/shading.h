@@ -112,7 +112,8 @@ __device__ __forceinline__ void store_hit(solhip_hit *dst, const Hit &h)
 // one after the other, about 15 ns each (70 per us): one per wave on the ray
 // counter bounded the AO primary kernel and added 60 us to the end of
 // every persistent launch.  A kernel whose ray count is known adds it once
-// (count_known); one that must count adds once per block of its waves' sums.
+// (count_known).  One that must count, the GLSL programs' and k_pt_finish, adds once
+// per wave: their waves run for milliseconds, or end one by one.
 template <bool COUNT>
 __device__ __forceinline__ void count_fetches(Counters *c, const TravCounts &tc)
 {

@@ -181,7 +181,8 @@ SOLHIP_HD Hit trav_result(const TravState &s)
 // A phase costs the wave its instructions however few lanes need it, so lanes vote:
 // - An instance entry (general form: the transform, its six divisions) is taken by a few
 //   lanes in almost every step: it waits until a quarter of the active lanes want
-//   one (10,000 instances, 1080p 53.4 -> 48.1 ms; 2M rays on 500 instances 1073 -> 973 us;
+//   one (10,000 instances, a 1080p frame without its rebuild 53.4 -> 48.1 ms; 2M rays on 500
+//   instances 1073 -> 973 us;
 //   a half or a third or a sixth are 1 to 6 % slower; 8 lanes, not a share, hold up the last rays
 //   of a launch: 0.2M rays 355 -> 415 us).
 // - Lanes with triangles left sit out the node test, so the triangle phase is repeated

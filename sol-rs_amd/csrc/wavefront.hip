@@ -4,12 +4,13 @@
 //   generate  camera rays of all pixels into extension queue 0 (8x8 pixel
 //             tiles, one per 64 slots); folds the previous sample's radiance
 //             into the per-pixel sum
-//   extend    closest hit of every queued ray (persistent grid, waves fetch
-//             64 slots at a time from an atomic head)
+//   finish    a queue of a few rays per lane: its paths to their ends in one
+//             launch (k_pt_finish); the three kernels below then find nothing to do
+//   extend    closest hit of every queued ray (persistent grid, waves refill their
+//             idle lanes from the partitioned fetch heads of fetch.h)
 //   shade     pathtrace.rchit's material model; emission / sky into the
 //             path's radiance, the next ray and the next-event shadow ray
-//             appended to their queues with one atomic per wave (ballot +
-//             popcount + mbcnt)
+//             appended to their queues with one atomic per block (block_append)
 //   shadow    any-hit test of the shadow queue; unoccluded contributions are
 //             added to the path's radiance
 //   finalize  sample mean, accumulation (pathtrace.rgen:88-99), RGBA8 (:102)
